@@ -6,18 +6,26 @@
 
 namespace emu {
 
-// Device scratch of one call: the box list (keys, permutation, counts, starts,
-// cursors), the gather's combined fields and the scan's temporary storage.
-struct BoxScratchSize {
-    size_t ints = 0, comb = 0, scan = 0, total = 0;
-};
-BoxScratchSize box_scratch_size(int64_t np, int64_t nk, int nf, bool gather);
+// The three calls: the deposit, the deposit from the fixed scratch (no room
+// for records: it lists particles by index), and the gather.
+enum class BoxCall { deposit, deposit_static, gather };
 
-// List the particles by box, then deposit them into the fab (deposit = true;
-// the caller zeroes the deposited components first and folds the ghosts after)
-// or gather the RHS of each from it.  `scratch` holds box_scratch_size(...)
-// bytes.  Asynchronous on the context stream.
-int box_list_and_run(emu_ctx* ctx, const PView& P, const Fab& fab, bool deposit, void* scratch, size_t scratch_bytes);
+// Device scratch of one call on np particles and nk fab cells: the box list,
+// the records, the gather's results and combined fields, the scan's storage.
+struct BoxScratchSize {
+    size_t ints = 0, rec = 0, out = 0, comb = 0, scan = 0, total = 0;
+};
+BoxScratchSize box_scratch_size(int64_t np, int64_t nk, int nf, BoxCall call);
+
+// List the particles by box, then deposit them into the fab (the caller zeroes
+// the deposited components first and folds the ghosts after) or gather the RHS
+// of each from it into dst (which may be P itself).  `scratch` holds
+// box_scratch_size(...) bytes.  Asynchronous on the context stream.
+int box_list_and_run(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& fab, BoxCall call, void* scratch,
+                     size_t scratch_bytes);
+
+// The same with the context's scratch, in batches of particles that it holds.
+int box_run_batched(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& fab, BoxCall call);
 
 // The context's scratch, grown to `need` bytes (hipMalloc) on first use.
 int box_scratch(emu_ctx* ctx, size_t need, void** out);

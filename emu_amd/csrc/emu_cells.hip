@@ -20,6 +20,14 @@
 //    (N + s Nbar + matter delta_c0) and (F_d + s Fbar_d), s = -1 for real and
 //    +1 for imaginary parts (generate_code.py:317-323).
 //
+// The particles arrive in any order, and a run's own order is scattered too:
+// directions drift apart, so that after a few cells' travel no two neighbours
+// of the arrays share a box.  Reading attribute arrays through the list then
+// fetches a cache line per value.  So what crosses between array order and box
+// order does it as records, one contiguous piece per particle: the gather's
+// input (position, velocity) and result (NH potentials) always, the deposit's
+// input where the arrays are scattered (k_box_place).
+//
 // The per-particle formulas are the reference's; the order of the sums
 // differs (the deposit's also between runs, as with the reference's GPU
 // atomics), which moves results by rounding only.  A particle whose box
@@ -58,21 +66,21 @@ __device__ __forceinline__ bool particle_box(const PView& P, int64_t ip, const F
     return in;
 }
 
-// Per-wave aggregation of per-lane keys: for each distinct key among the
-// active lanes, f(key, lanes holding it, leader lane).
-template <typename F> __device__ __forceinline__ void for_each_key(bool act, int key, F&& f)
-{
-    unsigned long long left = __ballot(act);
-    while (left) {
-        const int lead = __ffsll((long long)left) - 1;
-        const int k = __shfl(key, lead);
-        const unsigned long long m = __ballot(act && key == k);
-        f(k, m, lead);
-        left &= ~m;
-    }
-}
+// Each particle's rank within its box, and the boxes' counts (box nk: the
+// particles whose box leaves the fab).  One atomic pass: the lanes of a wave
+// that share a box are grouped (up to kGroups boxes, enough for particles in
+// cell order, which hold one or two; lanes past that go singly), and then every
+// group's first lane adds its count at once, so the wave waits on one round
+// trip.  Grouping every box with an atomic inside the loop, and again in a
+// second pass for the permutation, took up to 64 round trips per wave on
+// scattered particles (0.17 + 0.36 ms per list of 3.0 M; this pass 0.11 ms, bound
+// by the atomics themselves).  Sampled blocks add their waves' boxes (the groups
+// and the single lanes) to counts[nk + 2], the measure of how scattered the
+// arrays are.
+constexpr int kGroups = 8;
 
-__global__ void k_box_keys(PView P, Fab fab, Geom g, int nk, int* __restrict__ key, int* __restrict__ counts)
+__global__ __launch_bounds__(kB) void k_box_rank(PView P, Fab fab, Geom g, int nk, int sample_every, int* __restrict__ rank,
+                                                 int* __restrict__ counts)
 {
     const int64_t ip = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const bool act = ip < P.np;
@@ -82,28 +90,26 @@ __global__ void k_box_keys(PView P, Fab fab, Geom g, int nk, int* __restrict__ k
         int o[3];
         double w[3][3];
         if (particle_box(P, ip, fab, g, o, w)) k = (o[2] * fab.nf[1] + o[1]) * fab.nf[0] + o[0];
-        key[ip] = k;
     }
-    for_each_key(act, k, [&](int kk, unsigned long long m, int lead) {
-        if (lane == lead) atomicAdd(&counts[kk], __popcll(m));
-    });
-}
-
-// perm lists the particles box by box; within a box, lane order within a
-// wave and waves in the order their atomics land.
-__global__ void k_box_perm(int64_t np, const int* __restrict__ key, const int* __restrict__ start, int* cursor,
-                           int* __restrict__ perm)
-{
-    const int64_t ip = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    const bool act = ip < np;
-    const int lane = threadIdx.x & 63;
-    const int k = act ? key[ip] : 0;
-    for_each_key(act, k, [&](int kk, unsigned long long m, int lead) {
-        int base = 0;
-        if (lane == lead) base = atomicAdd(&cursor[kk], __popcll(m));
-        base = __shfl(base, lead);
-        if ((m >> lane) & 1ull) perm[start[kk] + base + __popcll(m & ((1ull << lane) - 1ull))] = (int)ip;
-    });
+    unsigned long long left = __ballot(act);
+    int lead = lane, below = 0, size = 1, groups = 0;
+    while (left && groups < kGroups) {
+        const int l = __ffsll((long long)left) - 1;
+        const int kk = __shfl(k, l);
+        const unsigned long long m = __ballot(act && k == kk);
+        if ((m >> lane) & 1ull) {
+            lead = l;
+            below = __popcll(m & ((1ull << lane) - 1ull));
+            size = __popcll(m);
+        }
+        left &= ~m;
+        groups++;
+    }
+    int base = 0;
+    if (act && lead == lane) base = atomicAdd(&counts[k], size);
+    base = __shfl(base, lead);
+    if (act) rank[ip] = base + below;
+    if (blockIdx.x % sample_every == 0 && lane == 0) atomicAdd(&counts[nk + 2], groups + (int)__popcll(left));
 }
 
 __global__ void k_fill_i32(int* p, int64_t n, int v)
@@ -112,10 +118,121 @@ __global__ void k_fill_i32(int* p, int64_t n, int v)
         p[t] = v;
 }
 
-__global__ void k_count_skipped(const int* start, int nk, unsigned long long* oob)
+// The deposit's record of a particle, in doubles: position, velocity p/p_t,
+// then the products N f_c and Nbar fbar_c; an even count, moved as double2.
+template <int NF> struct DepRec {
+    static constexpr int V = 3, Q = 6, size = 6 + 2 * NH<NF>;
+};
+// The gather's: position and velocity; its result: the NH gathered potentials,
+// padded to an even count.
+struct GatRec {
+    static constexpr int V = 3, size = 6;
+};
+template <int NF> constexpr int gat_out_size() { return (NH<NF> + 1) / 2 * 2; }
+
+// Whether the arrays are scattered enough for the deposit to read records
+// (uniform over the grid; rec_min < 0: there is no room for records).
+__device__ __forceinline__ bool use_records(const int* counts, int nk, int rec_min)
 {
-    const int n = start[nk + 1] - start[nk];
-    if (threadIdx.x == 0 && n > 0) atomicAdd(oob, (unsigned long long)n);
+    return rec_min >= 0 && __builtin_amdgcn_readfirstlane(counts[nk + 2]) >= rec_min;
+}
+
+__device__ __forceinline__ void count_skipped(const int* start, int nk, unsigned long long* oob)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const int n = start[nk + 1] - start[nk];
+        if (n > 0) atomicAdd(oob, (unsigned long long)n);
+    }
+}
+
+// A particle's slot in box order: its box's start plus its rank.
+__device__ __forceinline__ int particle_slot(const PView& P, int64_t ip, const Fab& fab, const Geom& g, int nk,
+                                             const int* start, int rank)
+{
+    int o[3];
+    double w[3][3];
+    const int k = particle_box(P, ip, fab, g, o, w) ? (o[2] * fab.nf[1] + o[1]) * fab.nf[0] + o[0] : nk;
+    return start[k] + rank;
+}
+
+// The deposit's list: perm (perm[slot] = particle) for arrays nearly in box
+// order, or the records themselves.  A wave reads its 64 particles' attributes
+// coalesced, forms their records in LDS and writes them out 16 bytes a lane, a
+// record at a time; the odd row stride keeps the rows off one bank.
+template <int NF>
+__global__ __launch_bounds__(kB) void k_dep_place(PView P, Fab fab, Geom g, int nk, const int* __restrict__ counts,
+                                                  const int* __restrict__ start, const int* __restrict__ rank,
+                                                  int rec_min, int* __restrict__ perm, double2* __restrict__ rec,
+                                                  unsigned long long* oob)
+{
+    using I = PIdx<NF>;
+    using R = DepRec<NF>;
+    constexpr int nh = NH<NF>, LS = R::size + 1, H = R::size / 2;
+    __shared__ double lds[kB * LS];
+    count_skipped(start, nk, oob);
+    const int64_t ip = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const bool act = ip < P.np;
+    const int64_t ipl = act ? ip : P.np - 1;
+    const int slot = act ? particle_slot(P, ipl, fab, g, nk, start, rank[ipl]) : -1;
+    if (!use_records(counts, nk, rec_min)) {
+        if (act) perm[slot] = (int)ip;
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    double* wl = lds + (threadIdx.x - lane) * LS;
+    double* row = wl + lane * LS;
+    const double ipt = 1.0 / P.r[I::pupt][ipl];
+    const double N = P.r[I::N][ipl], Nb = P.r[I::Nbar][ipl];
+#pragma unroll
+    for (int d = 0; d < 3; d++) row[d] = P.pos[d][ipl];
+#pragma unroll
+    for (int d = 0; d < 3; d++) row[R::V + d] = P.r[I::pupx + d][ipl] * ipt;
+#pragma unroll
+    for (int c = 0; c < nh; c++) row[R::Q + c] = N * P.r[I::f + c][ipl];
+#pragma unroll
+    for (int c = 0; c < nh; c++) row[R::Q + nh + c] = Nb * P.r[I::fbar + c][ipl];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int j = 0; j < H; j++) {
+        const int e = j * 64 + lane, r = e / H, part = e - r * H;
+        const int dst = __shfl(slot, r);
+        if (dst >= 0) rec[(int64_t)dst * H + part] = make_double2(wl[r * LS + 2 * part], wl[r * LS + 2 * part + 1]);
+    }
+}
+
+// The gather's list: perm, or each particle's record at its slot and slot[ip]
+// (over its rank).  With dst other than P (nattr > 0) it also copies what the
+// gather does not write there: the positions, and every attribute of a skipped
+// particle.
+template <int NF>
+__global__ __launch_bounds__(kB) void k_gat_place(PView P, PView dst, int nattr, Fab fab, Geom g, int nk,
+                                                  const int* __restrict__ counts, const int* __restrict__ start,
+                                                  int* __restrict__ slot, int rec_min, int* __restrict__ perm,
+                                                  double2* __restrict__ rec, unsigned long long* oob)
+{
+    using I = PIdx<NF>;
+    count_skipped(start, nk, oob);
+    const int64_t ip = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (ip >= P.np) return;
+    const int s = particle_slot(P, ip, fab, g, nk, start, slot[ip]);
+    if (nattr > 0) {
+        for (int d = 0; d < 3; d++) dst.pos[d][ip] = P.pos[d][ip];
+        if (s >= start[nk])
+            for (int k = 0; k < nattr; k++) dst.r[k][ip] = P.r[k][ip];
+    }
+    if (!use_records(counts, nk, rec_min)) {
+        perm[s] = (int)ip;
+        return;
+    }
+    slot[ip] = s;
+    const double pt = P.r[I::pupt][ip];
+    const double v[3] = {P.r[I::pupx][ip] / pt, P.r[I::pupy][ip] / pt, P.r[I::pupz][ip] / pt};
+    double2* out = rec + (int64_t)s * (GatRec::size / 2);
+    out[0] = make_double2(P.pos[0][ip], P.pos[1][ip]);
+    out[1] = make_double2(P.pos[2][ip], v[0]);
+    out[2] = make_double2(v[1], v[2]);
 }
 
 // The gather's combined fields of every fab cell, cell-major [cell][4][NH]:
@@ -156,13 +273,63 @@ __device__ __forceinline__ int64_t box_block(int blocks_per_xcd)
 constexpr int kGatherRun = 8;
 constexpr int kWavesGather = kGatherRun / 2;
 
-template <int NF, int WX, int WY, int WZ>
+// What the right-hand side does with a particle's gathered potential: the
+// vacuum term (generate_code.py:239-255), the two commutators and the
+// reference's outputs (Evolve.cpp:160-172), from src into dst (which may be the
+// same arrays: the particle's values are read before they are written).
+template <int NF>
+__device__ __forceinline__ void rhs_outputs(const PView& src, const PView& dst, int64_t ip, const Geom& g,
+                                            const double* __restrict__ M2, const double* in)
+{
+    using I = PIdx<NF>;
+    constexpr int nh = NH<NF>;
+    const double pup[3] = {src.r[I::pupx][ip], src.r[I::pupy][ip], src.r[I::pupz][ip]}, pupt = src.r[I::pupt][ip];
+    const double coef = M_SQRT2 * phys::GF * g.inv_cell_volume;
+    double V[nh], Vb[nh];
+#pragma unroll
+    for (int c = 0; c < nh; c++) {
+        const double vac = M2[c] * phys::c4 / (2. * pupt), term = coef * in[c];
+        V[c] = vac + term;
+        Vb[c] = is_im_comp<NF>(c) ? -vac + term : vac - term;
+    }
+    double f[nh], d[nh];
+#pragma unroll
+    for (int c = 0; c < nh; c++) f[c] = src.r[I::f + c][ip];
+    commutator_rhs<NF, double>(V, f, d, 1.0 / phys::hbar);
+#pragma unroll
+    for (int c = 0; c < nh; c++) dst.r[I::f + c][ip] = d[c];
+#pragma unroll
+    for (int c = 0; c < nh; c++) f[c] = src.r[I::fbar + c][ip];
+    commutator_rhs<NF, double>(Vb, f, d, 1.0 / phys::hbar);
+#pragma unroll
+    for (int c = 0; c < nh; c++) dst.r[I::fbar + c][ip] = d[c];
+    dst.r[I::x][ip] = pup[0] / pupt * phys::c;
+    dst.r[I::y][ip] = pup[1] / pupt * phys::c;
+    dst.r[I::z][ip] = pup[2] / pupt * phys::c;
+    dst.r[I::time][ip] = 1.0;
+    dst.r[I::pupx][ip] = 0;
+    dst.r[I::pupy][ip] = 0;
+    dst.r[I::pupz][ip] = 0;
+    dst.r[I::pupt][ip] = 0;
+    dst.r[I::N][ip] = 0;
+    dst.r[I::Nbar][ip] = 0;
+    dst.r[I::L][ip] = 0;
+    dst.r[I::Lbar][ip] = 0;
+}
+
+// REC: the particles of a box are consecutive records, and so are the results
+// (k_rhs_finish takes them on in array order).  Otherwise the particles are
+// read through perm and finished here.
+template <int NF, int WX, int WY, int WZ, bool REC>
 __global__ __launch_bounds__(64 * kWavesGather) __attribute__((amdgpu_waves_per_eu(5))) void k_gather_boxes(
-    PView P, Fab fab, Geom g, const double* __restrict__ comb, const double* __restrict__ M2,
-    const int* __restrict__ start, const int* __restrict__ perm, int nrun_x, int64_t nruns, int blocks_per_xcd)
+    PView P, PView dst, Fab fab, Geom g, const double* __restrict__ comb, const double* __restrict__ M2, int nk,
+    const int* __restrict__ counts, const int* __restrict__ start, const int* __restrict__ perm,
+    const double2* __restrict__ rec, double2* __restrict__ out, int rec_min, int nrun_x, int64_t nruns,
+    int blocks_per_xcd)
 {
     using I = PIdx<NF>;
     constexpr int nh = NH<NF>, QG = 4 * nh, NT = WX * WY * WZ, UX = kGatherRun + WX - 1;
+    if (use_records(counts, nk, rec_min) != REC) return; // the launch of the other kind runs
     // the run's fields, the same for every lane of a box: a lane's read of a
     // cell's values is an LDS broadcast (two addresses per wave, one per box)
     __shared__ double2 run_lds[WZ * WY * UX * QG / 2];
@@ -198,26 +365,39 @@ __global__ __launch_bounds__(64 * kWavesGather) __attribute__((amdgpu_waves_per_
     const int mid = __builtin_amdgcn_readfirstlane(start[kb + 1]);
     const int end = __builtin_amdgcn_readfirstlane(start[kb + nb]);
     if (beg >= end) return;
-    const double coef = M_SQRT2 * phys::GF * g.inv_cell_volume;
     const double* runf = reinterpret_cast<const double*>(run_lds);
     for (int base = beg; base < end; base += 64) {
         const bool act = base + lane < end;
-        const int64_t ip = perm[act ? base + lane : beg];
+        const int64_t at = act ? base + lane : beg;
         // this lane's box: the wave's first or second
         const double* boxf = runf + (2 * wave + (base + lane >= mid ? 1 : 0)) * QG;
-        const double pupx = P.r[I::pupx][ip], pupy = P.r[I::pupy][ip], pupz = P.r[I::pupz][ip],
-                     pupt = P.r[I::pupt][ip];
-        int o[3];
-        double w[3][3];
-        particle_box(P, ip, fab, g, o, w);
-        const double vx = pupx / pupt, vy = pupy / pupt, vz = pupz / pupt;
-        double in[nh];
+        int64_t ip = at;
+        double x[3], vx, vy, vz;
+        if constexpr (REC) {
+            const double2* r = rec + at * (GatRec::size / 2);
+            const double2 r0 = r[0], r1 = r[1], r2 = r[2];
+            x[0] = r0.x, x[1] = r0.y, x[2] = r1.x;
+            vx = r1.y, vy = r2.x, vz = r2.y;
+        } else {
+            ip = perm[at];
+            const double pt = P.r[I::pupt][ip];
 #pragma unroll
-        for (int c = 0; c < nh; c++) in[c] = 0.0;
+            for (int d = 0; d < 3; d++) x[d] = P.pos[d][ip];
+            vx = P.r[I::pupx][ip] / pt, vy = P.r[I::pupy][ip] / pt, vz = P.r[I::pupz][ip] / pt;
+        }
+        double w[3][3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            int idx;
+            shape3((x[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, w[d]);
+        }
+        double in[nh + 1];
+#pragma unroll
+        for (int c = 0; c <= nh; c++) in[c] = 0.0;
         // one box cell per iteration: per field v the lane's coefficient
         // w_t s_v, s = (1, -v_x, -v_y, -v_z), times the NH uniform values of
         // that field
-        auto pick = [](const double* x, int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); };
+        auto pick = [](const double* y, int i) { return i == 0 ? y[0] : (i == 1 ? y[1] : y[2]); };
 #pragma unroll 1
         for (int t = 0; t < NT; t++) {
             const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
@@ -230,51 +410,39 @@ __global__ __launch_bounds__(64 * kWavesGather) __attribute__((amdgpu_waves_per_
                 for (int c = 0; c < nh; c++) in[c] += a[v] * G[v * nh + c];
         }
         if (!act) continue;
-        // vacuum (generate_code.py:239-255), then the gathered potential
-        double V[nh], Vb[nh];
+        if constexpr (REC) {
+            constexpr int H = gat_out_size<NF>() / 2;
 #pragma unroll
-        for (int i = 0; i < NF; i++)
-#pragma unroll
-            for (int j = i; j < NF; j++) {
-                const int cr = herm_re<NF>(i, j);
-                V[cr] = Vb[cr] = M2[cr] * phys::c4 / (2. * pupt);
-                if (j > i) {
-                    const int ci = herm_im<NF>(i, j);
-                    V[ci] = M2[ci] * phys::c4 / (2. * pupt);
-                    Vb[ci] = -V[ci];
-                }
-            }
-#pragma unroll
-        for (int c = 0; c < nh; c++) {
-            const double term = coef * in[c];
-            V[c] += term;
-            Vb[c] += is_im_comp<NF>(c) ? term : -term;
+            for (int j = 0; j < H; j++) out[at * H + j] = make_double2(in[2 * j], in[2 * j + 1]);
+        } else {
+            rhs_outputs<NF>(P, dst, ip, g, M2, in);
         }
-        // Evolve.cpp:160-172
-        P.r[I::x][ip] = pupx / pupt * phys::c;
-        P.r[I::y][ip] = pupy / pupt * phys::c;
-        P.r[I::z][ip] = pupz / pupt * phys::c;
-        P.r[I::time][ip] = 1.0;
-        P.r[I::pupx][ip] = 0;
-        P.r[I::pupy][ip] = 0;
-        P.r[I::pupz][ip] = 0;
-        P.r[I::pupt][ip] = 0;
-        P.r[I::N][ip] = 0;
-        P.r[I::Nbar][ip] = 0;
-        P.r[I::L][ip] = 0;
-        P.r[I::Lbar][ip] = 0;
-        double f[nh], d[nh];
-#pragma unroll
-        for (int c = 0; c < nh; c++) f[c] = P.r[I::f + c][ip];
-        commutator_rhs<NF, double>(V, f, d, 1.0 / phys::hbar);
-#pragma unroll
-        for (int c = 0; c < nh; c++) P.r[I::f + c][ip] = d[c];
-#pragma unroll
-        for (int c = 0; c < nh; c++) f[c] = P.r[I::fbar + c][ip];
-        commutator_rhs<NF, double>(Vb, f, d, 1.0 / phys::hbar);
-#pragma unroll
-        for (int c = 0; c < nh; c++) P.r[I::fbar + c][ip] = d[c];
     }
+}
+
+// The rest of the right-hand side of the record form, in array order.  Bound by
+// HBM: 22 values read and 30 written per particle, all coalesced, and the
+// record of the potential, fetched whole.
+template <int NF>
+__global__ __launch_bounds__(kB) void k_rhs_finish(PView src, PView dst, Geom g, const double* __restrict__ M2, int nk,
+                                                   const int* __restrict__ counts, const int* __restrict__ start,
+                                                   const int* __restrict__ slot, const double2* __restrict__ pot,
+                                                   int rec_min)
+{
+    constexpr int H = gat_out_size<NF>() / 2;
+    if (!use_records(counts, nk, rec_min)) return;
+    const int64_t ip = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (ip >= src.np) return;
+    const int s = slot[ip];
+    if (s >= start[nk]) return; // skipped
+    double in[2 * H];
+#pragma unroll
+    for (int j = 0; j < H; j++) {
+        const double2 v = pot[(int64_t)s * H + j];
+        in[2 * j] = v.x;
+        in[2 * j + 1] = v.y;
+    }
+    rhs_outputs<NF>(src, dst, ip, g, M2, in);
 }
 
 // The deposit takes boxes a patch at a time: PX x PY x PZ boxes (2 x 2 x 1 for
@@ -316,8 +484,9 @@ constexpr int dep_lds_doubles()
 
 template <int NF, int WX, int WY, int WZ>
 __global__ __launch_bounds__((64 * DepPatch<WX, WY, WZ>::WAVES)) __attribute__((amdgpu_waves_per_eu(3))) void k_deposit_boxes(
-    PView P, Fab fab, Geom g, const int* __restrict__ start, const int* __restrict__ perm, int npx, int npy,
-    int64_t npatch, int blocks_per_xcd)
+    PView P, Fab fab, Geom g, int nk, const int* __restrict__ counts, const int* __restrict__ start,
+    const int* __restrict__ perm, const double2* __restrict__ rec, int rec_min, int npx, int npy, int64_t npatch,
+    int blocks_per_xcd)
 {
     using I = PIdx<NF>;
     using PT = DepPatch<WX, WY, WZ>;
@@ -380,54 +549,89 @@ __global__ __launch_bounds__((64 * DepPatch<WX, WY, WZ>::WAVES)) __attribute__((
     // those rows are never flushed)
     const double* wl = Wf + (lane >> 4) * R::W + (lane & 15);
     const double* sl = Src + (lane >> 4) * R::S;
+    const bool records = use_records(counts, nk, rec_min);
+    auto pick = [](const double* x, int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); };
+    // an inactive row gets zero weights: its sources then add nothing
+    auto put_weights = [&](const double w[3][3], bool act) {
+#pragma unroll
+        for (int kk = 0; kk < WZ; kk++)
+#pragma unroll
+            for (int jj = 0; jj < WY; jj++) {
+                const double yz = pick(w[1], WY == 3 ? jj : 1) * pick(w[2], WZ == 3 ? kk : 1);
+#pragma unroll
+                for (int ii = 0; ii < WX; ii++) {
+                    const double x = pick(w[0], WX == 3 ? ii : 1);
+                    wr[(kk * WY + jj) * WX + ii] = (act ? x : 0.0) * yz;
+                }
+            }
+    };
     // each chunk's permutation entry is loaded one chunk ahead, so that the
     // particle loads wait on one round trip instead of two
-    int ip_next = beg < end ? perm[beg + cl < end ? beg + cl : beg] : 0;
+    int ip_next = beg < end && !records ? perm[beg + cl < end ? beg + cl : beg] : 0;
     for (int base = beg; base < end; base += kDepChunk) {
         const bool act = base + cl < end;
-        const int64_t ip = ip_next;
-        const int nb = base + kDepChunk;
-        if (nb < end) ip_next = perm[nb + cl < end ? nb + cl : beg];
-        int o[3];
-        double w[3][3];
-        particle_box(P, ip, fab, g, o, w);
-        // every lane loads (inactive ones a valid particle), so that the loads
-        // issue together, nu's batch then nubar's.  An inactive row gets zero
-        // weights: its sources then add nothing.
-        {
-            const double pupt = P.r[I::pupt][ip], pv[3] = {P.r[I::pupx][ip], P.r[I::pupy][ip], P.r[I::pupz][ip]};
-            const double N = P.r[I::N][ip];
-            double fv[nh];
+        if (records) {
+            // the box's particles are consecutive records: lanes 0-31 read the
+            // first halves of the chunk's records, lanes 32-63 the second
+            using DR = DepRec<NF>;
+            constexpr int H = DR::size / 4, H0 = DR::size / 2 - H; // double2 per half: H0 in the first, H in the second
+            const double2* r = rec + (int64_t)(act ? base + cl : beg) * (DR::size / 2) + (row ? 0 : H0);
+            double v[2 * H0];
 #pragma unroll
-            for (int c = 0; c < nh; c++) fv[c] = P.r[I::f + c][ip];
-            if (row) {
-                auto pick = [](const double* x, int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); };
-#pragma unroll
-                for (int kk = 0; kk < WZ; kk++)
-#pragma unroll
-                    for (int jj = 0; jj < WY; jj++) {
-                        const double yz = pick(w[1], WY == 3 ? jj : 1) * pick(w[2], WZ == 3 ? kk : 1);
-#pragma unroll
-                        for (int ii = 0; ii < WX; ii++) {
-                            const double x = pick(w[0], WX == 3 ? ii : 1);
-                            wr[(kk * WY + jj) * WX + ii] = (act ? x : 0.0) * yz;
-                        }
-                    }
-#pragma unroll
-                for (int c = 0; c < nh; c++) sr[c] = N * fv[c];
-                const double ipt = 1.0 / pupt;
-#pragma unroll
-                for (int d = 0; d < 3; d++) sr[R::ONE + 1 + d] = pv[d] * ipt;
+            for (int j = 0; j < H0; j++) {
+                const double2 x = j < H || row ? r[j] : make_double2(0.0, 0.0);
+                v[2 * j] = x.x;
+                v[2 * j + 1] = x.y;
             }
-        }
-        {
-            const double Nb = P.r[I::Nbar][ip];
-            double fv[nh];
-#pragma unroll
-            for (int c = 0; c < nh; c++) fv[c] = P.r[I::fbar + c][ip];
             if (row) {
+                double w[3][3];
 #pragma unroll
-                for (int c = 0; c < nh; c++) sr[nh + c] = Nb * fv[c];
+                for (int d = 0; d < 3; d++) {
+                    int idx;
+                    shape3((v[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, w[d]);
+                }
+                put_weights(w, act);
+#pragma unroll
+                for (int d = 0; d < 3; d++) sr[R::ONE + 1 + d] = v[DR::V + d];
+#pragma unroll
+                for (int c = DR::Q; c < 2 * H0; c++) sr[c - DR::Q] = v[c];
+            } else {
+#pragma unroll
+                for (int c = 0; c < 2 * H; c++) sr[2 * H0 - DR::Q + c] = v[c];
+            }
+        } else {
+            const int64_t ip = ip_next;
+            const int nb = base + kDepChunk;
+            if (nb < end) ip_next = perm[nb + cl < end ? nb + cl : beg];
+            int o[3];
+            double w[3][3];
+            particle_box(P, ip, fab, g, o, w);
+            // every lane loads (inactive ones a valid particle), so that the loads
+            // issue together, nu's batch then nubar's
+            {
+                const double pupt = P.r[I::pupt][ip], pv[3] = {P.r[I::pupx][ip], P.r[I::pupy][ip], P.r[I::pupz][ip]};
+                const double N = P.r[I::N][ip];
+                double fv[nh];
+#pragma unroll
+                for (int c = 0; c < nh; c++) fv[c] = P.r[I::f + c][ip];
+                if (row) {
+                    put_weights(w, act);
+#pragma unroll
+                    for (int c = 0; c < nh; c++) sr[c] = N * fv[c];
+                    const double ipt = 1.0 / pupt;
+#pragma unroll
+                    for (int d = 0; d < 3; d++) sr[R::ONE + 1 + d] = pv[d] * ipt;
+                }
+            }
+            {
+                const double Nb = P.r[I::Nbar][ip];
+                double fv[nh];
+#pragma unroll
+                for (int c = 0; c < nh; c++) fv[c] = P.r[I::fbar + c][ip];
+                if (row) {
+#pragma unroll
+                    for (int c = 0; c < nh; c++) sr[nh + c] = Nb * fv[c];
+                }
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -515,41 +719,62 @@ __global__ __launch_bounds__((64 * DepPatch<WX, WY, WZ>::WAVES)) __attribute__((
     }
 }
 
-template <int NF, int WX, int WY, int WZ>
-void launch_boxes(bool deposit, hipStream_t s, const PView& P, const Fab& fab, const Geom& g, const double* comb,
-                  const double* M2, const int* start, const int* perm, int nk)
+// One call's arrays in its scratch.
+struct BoxArrays {
+    int *rank, *perm, *counts, *start; // rank becomes the gather's slots in its record form
+    double2 *rec, *out;                // records, and the gather's result records
+    double* comb;
+    void* scan;
+};
+
+struct Launch {
+    hipStream_t s;
+    const Geom& g;
+    const Fab& fab;
+    const PView &P, &dst;
+    const BoxArrays& b;
+    const double* M2;
+    int nk, rec_min;
+};
+
+template <int NF, int WX, int WY, int WZ> void launch_boxes(bool deposit, const Launch& L)
 {
+    const Fab& fab = L.fab;
     if (deposit) {
         using PT = DepPatch<WX, WY, WZ>;
         const int npx = (fab.nf[0] + PT::PX - 1) / PT::PX, npy = (fab.nf[1] + PT::PY - 1) / PT::PY;
         const int npz = (fab.nf[2] + PT::PZ - 1) / PT::PZ;
         const int64_t npatch = (int64_t)npx * npy * npz;
         const int bpx = (int)((npatch + 7) / 8);
-        hipLaunchKernelGGL((k_deposit_boxes<NF, WX, WY, WZ>), dim3(8 * bpx), dim3(64 * PT::WAVES), 0, s, P, fab, g,
-                           start, perm, npx, npy, npatch, bpx);
+        hipLaunchKernelGGL((k_deposit_boxes<NF, WX, WY, WZ>), dim3(8 * bpx), dim3(64 * PT::WAVES), 0, L.s, L.P, fab,
+                           L.g, L.nk, L.b.counts, L.b.start, L.b.perm, L.b.rec, L.rec_min, npx, npy, npatch, bpx);
     } else {
         const int nrun_x = (fab.nf[0] + kGatherRun - 1) / kGatherRun;
         const int64_t nruns = (int64_t)nrun_x * fab.nf[1] * fab.nf[2];
         const int bpx = (int)((nruns + 7) / 8);
-        hipLaunchKernelGGL((k_gather_boxes<NF, WX, WY, WZ>), dim3(8 * bpx), dim3(64 * kWavesGather), 0, s, P, fab, g,
-                           comb, M2, start, perm, nrun_x, nruns, bpx);
+        // both forms, of which the one that the arrays' order asks for runs
+        hipLaunchKernelGGL((k_gather_boxes<NF, WX, WY, WZ, true>), dim3(8 * bpx), dim3(64 * kWavesGather), 0, L.s, L.P,
+                           L.dst, fab, L.g, L.b.comb, L.M2, L.nk, L.b.counts, L.b.start, L.b.perm, L.b.rec, L.b.out,
+                           L.rec_min, nrun_x, nruns, bpx);
+        hipLaunchKernelGGL((k_gather_boxes<NF, WX, WY, WZ, false>), dim3(8 * bpx), dim3(64 * kWavesGather), 0, L.s, L.P,
+                           L.dst, fab, L.g, L.b.comb, L.M2, L.nk, L.b.counts, L.b.start, L.b.perm, L.b.rec, L.b.out,
+                           L.rec_min, nrun_x, nruns, bpx);
     }
 }
 
-template <int NF>
-void launch_boxes_nf(bool deposit, const Geom& g, hipStream_t s, const PView& P, const Fab& fab, const double* comb,
-                     const double* M2, const int* start, const int* perm, int nk)
+template <int NF> void launch_boxes_nf(bool deposit, const Launch& L)
 {
-    const int w = (g.order[0] > 0 ? 1 : 0) | (g.order[1] > 0 ? 2 : 0) | (g.order[2] > 0 ? 4 : 0);
+    const int* o = L.g.order;
+    const int w = (o[0] > 0 ? 1 : 0) | (o[1] > 0 ? 2 : 0) | (o[2] > 0 ? 4 : 0);
     switch (w) {
-    case 0: launch_boxes<NF, 1, 1, 1>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    case 1: launch_boxes<NF, 3, 1, 1>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    case 2: launch_boxes<NF, 1, 3, 1>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    case 3: launch_boxes<NF, 3, 3, 1>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    case 4: launch_boxes<NF, 1, 1, 3>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    case 5: launch_boxes<NF, 3, 1, 3>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    case 6: launch_boxes<NF, 1, 3, 3>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
-    default: launch_boxes<NF, 3, 3, 3>(deposit, s, P, fab, g, comb, M2, start, perm, nk); break;
+    case 0: launch_boxes<NF, 1, 1, 1>(deposit, L); break;
+    case 1: launch_boxes<NF, 3, 1, 1>(deposit, L); break;
+    case 2: launch_boxes<NF, 1, 3, 1>(deposit, L); break;
+    case 3: launch_boxes<NF, 3, 3, 1>(deposit, L); break;
+    case 4: launch_boxes<NF, 1, 1, 3>(deposit, L); break;
+    case 5: launch_boxes<NF, 3, 1, 3>(deposit, L); break;
+    case 6: launch_boxes<NF, 1, 3, 3>(deposit, L); break;
+    default: launch_boxes<NF, 3, 3, 3>(deposit, L); break;
     }
 }
 
@@ -562,53 +787,128 @@ size_t scan_bytes(int64_t n)
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// Records are used where the sampled waves of 64 particles hold on average at
+// least this many boxes.  In box order a wave of 92 particles per cell holds
+// 1.7 (its cell or two); after a drift of d cells the lattice of every direction
+// is shifted and a wave holds about 8 at d = 0.6, 14 at 0.8, 20 at 1 and nearly
+// 64 from 3 on.  Measured at 64^3 x 92, NF = 3, ms per call, list included:
+//   d                          0      0.6    0.8    1.0    1.5    3.0
+//   gather through perm        3.8    7.2    9.6    12.7   14.4   24.1
+//   gather by records          5.2    5.3    5.7    5.8    5.9    6.4
+//   deposit through perm       4.5    5.1    6.3    7.3    7.7    14.2
+//   deposit by records         -      6.1    6.5    6.6    6.6    7.1
+constexpr int kScatteredDeposit = 24, kScatteredGather = 7;
+
 } // namespace
 
-BoxScratchSize box_scratch_size(int64_t np, int64_t nk, int nf, bool gather)
+BoxScratchSize box_scratch_size(int64_t np, int64_t nk, int nf, BoxCall call)
 {
+    const size_t n = (size_t)np;
+    const int nh = nf * nf;
     BoxScratchSize s;
-    s.ints = align256(sizeof(int) * (size_t)(2 * np + 3 * (nk + 2)));
-    s.comb = gather ? align256(sizeof(double) * (size_t)nk * 4 * nf * nf) : 0;
+    s.ints = align256(sizeof(int) * (2 * n + 2 * (size_t)nk + 5));
+    if (call == BoxCall::deposit) s.rec = align256(sizeof(double) * n * (6 + 2 * nh));
+    if (call == BoxCall::gather) {
+        s.rec = align256(sizeof(double) * n * GatRec::size);
+        s.out = align256(sizeof(double) * n * ((nh + 1) / 2 * 2));
+        s.comb = align256(sizeof(double) * (size_t)nk * 4 * nh);
+    }
     s.scan = align256(scan_bytes(nk + 2));
-    s.total = s.ints + s.comb + s.scan;
+    s.total = s.ints + s.rec + s.out + s.comb + s.scan;
     return s;
 }
 
-int box_list_and_run(emu_ctx* ctx, const PView& P, const Fab& fab, bool deposit, void* scratch, size_t scratch_bytes)
+int box_list_and_run(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& fab, BoxCall call, void* scratch,
+                     size_t scratch_bytes)
 {
     hipStream_t s = ctx->stream;
     const int64_t nk64 = fab.cstride;
-    if (nk64 + 2 > (int64_t)INT32_MAX || P.np > (int64_t)INT32_MAX)
+    if (nk64 + 3 > (int64_t)INT32_MAX || P.np > (int64_t)INT32_MAX)
         return set_error(ctx, EMU_ERR_UNSUPPORTED, "more than 2^31 particles or fab cells");
     const int nk = (int)nk64;
     const int nf = ctx->p.nf;
-    const BoxScratchSize sz = box_scratch_size(P.np, nk, nf, !deposit);
+    const bool deposit = call != BoxCall::gather;
+    const BoxScratchSize sz = box_scratch_size(P.np, nk, nf, call);
     if (scratch_bytes < sz.total) return set_error(ctx, EMU_ERR_ARG, "box list scratch too small");
-    char* b = (char*)scratch;
-    int* key = (int*)b;
-    int* perm = key + P.np;
-    int* counts = perm + P.np;
-    int* start = counts + (nk + 2);
-    int* cursor = start + (nk + 2);
-    double* comb = (double*)(b + sz.ints);
-    void* tmp = b + sz.ints + sz.comb;
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(2 * (nk + 2))), dim3(kB), 0, s, counts, 2 * (int64_t)(nk + 2), 0);
-    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(nk + 2)), dim3(kB), 0, s, cursor, (int64_t)(nk + 2), 0);
-    if (P.np > 0)
-        hipLaunchKernelGGL(k_box_keys, dim3(nblk(P.np)), dim3(kB), 0, s, P, fab, ctx->g, nk, key, counts);
+    if (P.np == 0) return EMU_OK;
+    BoxArrays b;
+    char* at = (char*)scratch;
+    b.rank = (int*)at;
+    b.perm = b.rank + P.np;
+    b.counts = b.perm + P.np;
+    b.start = b.counts + (nk + 3);
+    b.rec = (double2*)(at += sz.ints);
+    b.out = (double2*)(at += sz.rec);
+    b.comb = (double*)(at += sz.out);
+    b.scan = at + sz.comb;
+    // blocks sampled for the order of the arrays: at most 256 of them
+    const unsigned nb = nblk(P.np);
+    const int every = (int)((nb + 255) / 256);
+    const int waves = (int)((nb + every - 1) / every) * (kB / 64);
+    const int rec_min = call == BoxCall::deposit_static ? -1 : (deposit ? kScatteredDeposit : kScatteredGather) * waves;
+    hipLaunchKernelGGL(k_fill_i32, dim3(nblk(nk + 3)), dim3(kB), 0, s, b.counts, (int64_t)nk + 3, 0);
+    hipLaunchKernelGGL(k_box_rank, dim3(nb), dim3(kB), 0, s, P, fab, ctx->g, nk, every, b.rank, b.counts);
     size_t tb = sz.scan;
-    EMU_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(tmp, tb, counts, start, nk + 2, s));
-    if (P.np > 0) hipLaunchKernelGGL(k_box_perm, dim3(nblk(P.np)), dim3(kB), 0, s, P.np, key, start, cursor, perm);
-    hipLaunchKernelGGL(k_count_skipped, dim3(1), dim3(64), 0, s, start, nk, ctx->d_red + 7);
-    if (!deposit) {
-        if (nf == 2) hipLaunchKernelGGL(k_combine<2>, dim3(nblk(nk)), dim3(kB), 0, s, fab, ctx->g, comb);
-        else hipLaunchKernelGGL(k_combine<3>, dim3(nblk(nk)), dim3(kB), 0, s, fab, ctx->g, comb);
+    EMU_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(b.scan, tb, b.counts, b.start, nk + 2, s));
+    const PView& D = dst ? *dst : P;
+    const Launch L{s, ctx->g, fab, P, D, b, ctx->d_M2, nk, rec_min};
+#define BOX_NF(kernel, ...)                                                                        \
+    do {                                                                                           \
+        if (nf == 2) hipLaunchKernelGGL(kernel<2>, dim3(nb), dim3(kB), 0, s, __VA_ARGS__);         \
+        else hipLaunchKernelGGL(kernel<3>, dim3(nb), dim3(kB), 0, s, __VA_ARGS__);                 \
+    } while (0)
+    if (deposit) {
+        BOX_NF(k_dep_place, P, fab, ctx->g, nk, b.counts, b.start, b.rank, rec_min, b.perm, b.rec, ctx->d_red + 7);
+    } else {
+        const int nattr = D.r[0] != P.r[0] ? 12 + 2 * nf * nf : 0;
+        BOX_NF(k_gat_place, P, D, nattr, fab, ctx->g, nk, b.counts, b.start, b.rank, rec_min, b.perm, b.rec,
+               ctx->d_red + 7);
+        if (nf == 2) hipLaunchKernelGGL(k_combine<2>, dim3(nblk(nk)), dim3(kB), 0, s, fab, ctx->g, b.comb);
+        else hipLaunchKernelGGL(k_combine<3>, dim3(nblk(nk)), dim3(kB), 0, s, fab, ctx->g, b.comb);
     }
-    if (P.np > 0) {
-        if (nf == 2) launch_boxes_nf<2>(deposit, ctx->g, s, P, fab, comb, ctx->d_M2, start, perm, nk);
-        else launch_boxes_nf<3>(deposit, ctx->g, s, P, fab, comb, ctx->d_M2, start, perm, nk);
-    }
+    if (nf == 2) launch_boxes_nf<2>(deposit, L);
+    else launch_boxes_nf<3>(deposit, L);
+    if (!deposit) BOX_NF(k_rhs_finish, P, D, ctx->g, ctx->d_M2, nk, b.counts, b.start, b.rank, b.out, rec_min);
+#undef BOX_NF
     EMU_LAUNCH_CHECK(ctx, deposit ? "deposit_to_mesh" : "interpolate_rhs_from_mesh");
+    return EMU_OK;
+}
+
+// Runs the call in batches of particles (the deposit adds up, the gather is
+// per particle), so that the scratch stays bounded: kBoxBatch particles, or
+// fewer where that does not fit beside what the caller holds.
+constexpr int64_t kBoxBatch = int64_t(1) << 25, kBoxBatchMin = int64_t(1) << 16;
+
+int box_run_batched(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& fab, BoxCall call)
+{
+    if (ctx->box_batch == 0) ctx->box_batch = kBoxBatch;
+    void* scratch = nullptr;
+    size_t need = 0;
+    for (;;) {
+        need = box_scratch_size(std::min(P.np, ctx->box_batch), fab.cstride, ctx->p.nf, call).total;
+        const int e = box_scratch(ctx, need, &scratch);
+        if (e == EMU_OK) break;
+        const int64_t half = std::min(P.np, ctx->box_batch) / 2;
+        if (half < kBoxBatchMin) return e;
+        ctx->box_batch = half;
+    }
+    auto part = [](const PView& V, int64_t at, int64_t n) {
+        PView p = V;
+        p.np = n;
+        for (int d = 0; d < 3; d++)
+            if (p.pos[d]) p.pos[d] += at;
+        for (int k = 0; k < EMU_MAX_ATTRIBS; k++)
+            if (p.r[k]) p.r[k] += at;
+        return p;
+    };
+    int64_t at = 0;
+    do {
+        const int64_t n = std::min(P.np - at, ctx->box_batch);
+        const PView Pp = part(P, at, n), Dp = dst ? part(*dst, at, n) : PView{};
+        const int e = box_list_and_run(ctx, Pp, dst ? &Dp : nullptr, fab, call, scratch, need);
+        if (e != EMU_OK) return e;
+        at += n;
+    } while (at < P.np);
     return EMU_OK;
 }
 
@@ -650,7 +950,7 @@ int static_scratch(emu_ctx* ctx, int64_t np, int64_t ncells, void** out, size_t*
                          "emu_deposit_to_mesh_static holds at most " + std::to_string(kStaticMaxParticles) +
                              " particles and " + std::to_string(kStaticMaxCells) + " fab cells (got " +
                              std::to_string(np) + " and " + std::to_string(ncells) + ")");
-    const BoxScratchSize sz = box_scratch_size(np, ncells, ctx->p.nf, false);
+    const BoxScratchSize sz = box_scratch_size(np, ncells, ctx->p.nf, BoxCall::deposit_static);
     if (sz.total > kStaticScratchBytes || sz.scan > kStaticScanBytes)
         return set_error(ctx, EMU_ERR_UNSUPPORTED, "static scratch too small for this grid");
     int dev = -1;
@@ -668,6 +968,7 @@ int box_scratch(emu_ctx* ctx, size_t need, void** out)
         ctx->box_scratch = nullptr;
         ctx->box_scratch_bytes = 0;
         if (hipMalloc(&ctx->box_scratch, need) != hipSuccess) {
+            (void)hipGetLastError(); // not the next launch check's
             ctx->box_scratch = nullptr;
             return set_error(ctx, EMU_ERR_NOMEM, "box list scratch");
         }

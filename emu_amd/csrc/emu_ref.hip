@@ -364,14 +364,16 @@ extern "C" int emu_destroy(emu_ctx* ctx);
 
 namespace emu {
 namespace {
-// deposit_to_mesh (Evolve.cpp:91-126) into `fab` with the given box-list
-// scratch: zero the deposited components (valid and ghost cells), deposit,
-// then SumBoundary.  Launches kernels only.
+// deposit_to_mesh (Evolve.cpp:91-126) into `fab`: zero the deposited
+// components (valid and ghost cells), deposit, then SumBoundary.  With
+// `scratch` (the fixed one) it launches kernels only; otherwise the context's
+// scratch is used, and grown where it is too small.
 int deposit_into(emu_ctx* ctx, const PView& P, const Fab& fab, void* scratch, size_t bytes)
 {
     const int nc = 3 + 8 * ctx->p.nf * ctx->p.nf;
     hipLaunchKernelGGL(k_zero_comps, dim3(1024), dim3(kBlock), 0, ctx->stream, fab, 3, nc);
-    const int e = box_list_and_run(ctx, P, fab, true, scratch, bytes);
+    const int e = scratch ? box_list_and_run(ctx, P, nullptr, fab, BoxCall::deposit_static, scratch, bytes)
+                          : box_run_batched(ctx, P, nullptr, fab, BoxCall::deposit);
     if (e != EMU_OK) return e;
     const int64_t ncell = (int64_t)ctx->g.n[0] * ctx->g.n[1] * ctx->g.n[2];
     hipLaunchKernelGGL(k_sum_boundary, dim3(nblocks(ncell), comp_blocks(nc - 3)), dim3(kBlock), 0, ctx->stream, fab,
@@ -478,11 +480,7 @@ extern "C" int emu_deposit_to_mesh(emu_ctx* ctx, const emu_particles* parts, emu
     Fab fab;
     PView P;
     if (!make_fab(ctx, state, fab) || !make_pview(ctx, parts, P)) return set_error(ctx, EMU_ERR_ARG, "bad grid or particles");
-    const size_t need = box_scratch_size(P.np, fab.cstride, ctx->p.nf, false).total;
-    void* scratch = nullptr;
-    const int e = box_scratch(ctx, need, &scratch);
-    if (e != EMU_OK) return e;
-    return deposit_into(ctx, P, fab, scratch, need);
+    return deposit_into(ctx, P, fab, nullptr, 0);
 }
 
 extern "C" int emu_deposit_to_mesh_static(emu_ctx* ctx, const emu_particles* parts, emu_grid* state)
@@ -516,11 +514,7 @@ extern "C" int emu_interpolate_rhs_from_mesh(emu_ctx* ctx, emu_particles* rhs, c
     PView P;
     if (!make_fab(ctx, state, fab) || !make_pview(ctx, rhs, P)) return set_error(ctx, EMU_ERR_ARG, "bad grid or particles");
     if (P.np == 0) return EMU_OK;
-    const size_t need = box_scratch_size(P.np, fab.cstride, ctx->p.nf, true).total;
-    void* scratch = nullptr;
-    const int e = box_scratch(ctx, need, &scratch);
-    if (e != EMU_OK) return e;
-    return box_list_and_run(ctx, P, fab, false, scratch, need);
+    return box_run_batched(ctx, P, &P, fab, BoxCall::gather);
 }
 
 extern "C" int emu_compute_dt(emu_ctx* ctx, const emu_grid* state, double Vvac_max, double* dt_out)
