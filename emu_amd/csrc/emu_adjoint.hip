@@ -380,8 +380,7 @@ __global__ void k_positions(int64_t np, double* pos, const double* pup, double d
             x[d] = pos[(int64_t)d * np + p];
             v[d] = pup[(int64_t)d * np + p] / pup[3 * np + p] * phys::c;
         }
-        int nc;
-        end_position(x, v, dt, g, nx, nc);
+        end_position(x, v, dt, g, nx);
         for (int d = 0; d < 3; d++) pos[(int64_t)d * np + p] = nx[d];
     }
 }
@@ -922,8 +921,7 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_fwd_stage(AdjInT<T> in, Geo
 #pragma unroll
                 for (int d = 0; d < 3; d++)
                     vv[d] = double(in.pup[(int64_t)d * np + p]) / double(in.pup[3 * np + p]) * phys::c;
-                int nc;
-                end_position(x, vv, dt, g, nx, nc);
+                end_position(x, vv, dt, g, nx);
 #pragma unroll
                 for (int d = 0; d < 3; d++) pos_out[(int64_t)d * np + p] = nx[d];
             }

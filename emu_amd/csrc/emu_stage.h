@@ -59,20 +59,86 @@ template <typename T> struct PArrays {
     T* f;      // [2 NH][np]: nu components then nubar
 };
 
+// What the next step's dt follows from, besides the grid's maxima.
+struct DtParams {
+    double dt_translation, flavor_cfl, max_adaptive_speedup, Vvac_max, fixed_dt;
+    int use_flavor;
+    double vst_scale; // 2 NF sqrt2 GF / dV of the scaled weights
+};
+
+// compute_dt's maxima, as the bit patterns of non-negative doubles: word 0 the
+// adaptive speed, then the conservative one in kSlots words, a cache line
+// apart, that the maximum is the largest of.  Stage 4's waves spread over the
+// slots: all on one word they queued for it (16^3 cells, NF = 2: 40 us a
+// launch against 21).
+struct DtRed {
+    static constexpr int kSlots = 64, kStride = 16, words = (1 + kSlots) * kStride;
+    static EMU_HD int slot(int i) { return (1 + i % kSlots) * kStride; }
+};
+
+// main.cpp:193-198 and Evolve.cpp:57-88: the next dt from the maxima, which are
+// left at zero for the next step's.  All 64 lanes of one wave call it.
+__device__ __forceinline__ double next_dt(unsigned long long* red, const DtParams& p, unsigned long long* err)
+{
+    const int lane = threadIdx.x & 63;
+    double vst_max = __longlong_as_double((long long)red[DtRed::slot(lane)]);
+    for (int off = 32; off > 0; off >>= 1) vst_max = fmax(vst_max, __shfl_xor(vst_max, off));
+    const double vad_max = __longlong_as_double((long long)red[0]);
+    double dt_flavor = 0.0;
+    if (p.use_flavor) {
+        const double vad = vad_max + p.Vvac_max;
+        const double vst = vst_max + p.Vvac_max;
+        const double dfa = phys::hbar / vad * p.flavor_cfl;
+        const double dfs = phys::hbar / vst * p.flavor_cfl;
+        dt_flavor = dfs;
+        if (p.max_adaptive_speedup > 1) dt_flavor = fmin(dfs * p.max_adaptive_speedup, dfa);
+    }
+    red[DtRed::slot(lane)] = 0;
+    if (lane == 0) red[0] = 0;
+    if (p.fixed_dt > 0) return p.fixed_dt;
+    if (p.dt_translation != 0.0 && dt_flavor != 0.0) return fmin(p.dt_translation, dt_flavor);
+    if (p.dt_translation != 0.0) return p.dt_translation;
+    if (dt_flavor == 0.0 && lane == 0) atomicMin(err, status_word_noindex(EMU_ERR_DT));
+    return dt_flavor;
+}
+
+// The particles' time after a step of length h: the four weighted stages.
+__device__ __forceinline__ double advance_time(double t, double h)
+{
+#pragma clang fp contract(off)
+    t = h * (1. / 6.) * 1.0 + t;
+    t = h * (1. / 3.) * 1.0 + t;
+    t = h * (1. / 3.) * 1.0 + t;
+    t = h * (1. / 6.) * 1.0 + t;
+    return t;
+}
+
 template <typename T> struct StageArgs {
     PArrays<T> cur; // current copy, sorted by cell_start
     PArrays<T> dst; // stage 4 writes the step's result here, sorted by the new cells
     T* Y;           // stage state
     T* acc;         // RK accumulator
-    int* newcell;   // stage 1 writes each particle's end-of-step cell
+    // the sort plan: stage 1 writes each particle's move (of 27) and its rank
+    // among the particles of its cell with that move, and the cells' counts per
+    // move; stage 4 reads rank, move and the moves' destinations
+    int* rank;
+    unsigned char* mv;
+    int* mcount;
     const int* mbase;
-    const int* rank;
-    const unsigned char* mv;
     const int* cell_start; // first slot of each cell (a multiple of the slot alignment)
     const int* cell_cnt;   // particles of each cell
     const double* gin;  // grid read by the gather
     double* gout;       // grid deposited by this launch
     double* aux;        // compute_dt auxiliaries
+    double* gclear;     // grid this launch sets to its base for a later deposit (null: none)
+    int clear_aux;      // and the auxiliaries
+    double m00;         // the base: the matter term on component 0, zero elsewhere
+    int want_dt;        // stage 4: the conservative flavour bound of the grid it gathers, into red
+    unsigned long long* red; // compute_dt's maxima (DtRed)
+    int step_end;       // stage 0: also finish the step (StepEnd)
+    DtParams dtp;
+    double* scal;       // [0] time [1] dt
+    int64_t* steps;
     const double* dt;
     unsigned long long* err;
     int64_t np; // slots per array: the stride of the component-major arrays
@@ -85,6 +151,12 @@ template <typename T> struct StageArgs {
     double coef;   // sqrt2 GF / dV / hbar
     double maxError;
 };
+
+// Component of the i-th diagonal entry, i at run time.
+template <int NF> __device__ __forceinline__ int herm_re_rt(int i)
+{
+    return i == 0 ? 0 : (i == 1 ? herm_re<NF>(1, 1) : herm_re<NF>(NF - 1, NF - 1));
+}
 
 template <int NF> __device__ __forceinline__ constexpr bool is_im_comp(int c)
 {
@@ -157,16 +229,30 @@ __device__ __forceinline__ int renorm_fp64(double* f, double L, double maxError)
 
 // End-of-step position: the four stage saxpys, then the periodic shift.
 __device__ __forceinline__ void end_position(const double pos[3], const double v[3], double dt, const Geom& g,
-                                             double npos[3], int& newcell)
+                                             double npos[3])
 {
     const double ai[4] = {dt * (1. / 6.), dt * (1. / 3.), dt * (1. / 3.), dt * (1. / 6.)};
-    int nc[3];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        npos[d] = wrap1(advance_pos(pos[d], v[d], ai), g.rlo[d], g.rhi[d], g.L[d]);
-        nc[d] = bin1(npos[d], g.plo[d], g.dxi[d], g.n[d]);
+    for (int d = 0; d < 3; d++) npos[d] = wrap1(advance_pos(pos[d], v[d], ai), g.rlo[d], g.rhi[d], g.L[d]);
+}
+
+// The move (-1, 0, 1) from cell index `from` to the cell of x along one
+// dimension of n cells; more than one cell sets bad.  With 2 cells both
+// neighbours are the same cell, reached by +1.
+__device__ __forceinline__ int move1(int from, double x, double plo, double dxi, int n, bool& bad)
+{
+    int to;
+    {
+#pragma clang fp contract(off)
+        to = nearest_cell_center_index((x - plo) * dxi);
     }
-    newcell = (nc[2] * g.n[1] + nc[1]) * g.n[0] + nc[0];
+    if (to < 0) to += n; // x = plo exactly belongs to the last cell
+    const int d = to - from;
+    if (d == 0) return 0;
+    if (d == 1 || d == 1 - n) return 1;
+    if (d == -1 || d == n - 1) return -1;
+    bad = true;
+    return 0;
 }
 
 // Three ways to map waves to cells (MODE).
@@ -357,6 +443,47 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
         return ((oz + kk) * PT::NBY + (oy + jj)) * PT::NBX + (ox + ii);
     };
+    // set this wave's cells of the grid (and the auxiliaries) that a later launch
+    // deposits into: the cells partition over the waves, so no fill launches are
+    // needed between the stages
+    if (a.gclear && inside_domain) {
+        const int n = (inside1 ? 2 : 1) * QG;
+        double* gc = a.gclear + (int64_t)cell * QG;
+        for (int e = lane; e < n; e += 64) gc[e] = e == 0 || e == QG ? a.m00 : 0.0;
+    }
+    if (s == 2 && a.clear_aux && inside_domain) {
+        const int n = (inside1 ? 2 : 1) * NAUX;
+        for (int e = lane; e < n; e += 64) a.aux[(int64_t)cell * NAUX + e] = 0.0;
+    }
+    if constexpr (s == 4) {
+        // compute_dt's conservative bound (Evolve.cpp:40-56) of this wave's cell:
+        // N_ii and Nbar_ii from the auxiliaries S_ii and M_ii
+        if (a.want_dt && inside_domain) {
+            double v = 0.0;
+            if (lane < NF) {
+                const double M = a.gin[(int64_t)cell * QG + herm_re_rt<NF>(lane)] - (lane == 0 ? a.m00 : 0.0);
+                const double sum = a.aux[(int64_t)cell * NAUX + lane];
+                v = fmax(fmax(0.5 * (sum + M), 0.5 * (sum - M)), a.m00);
+            }
+            v = fmax(v, __shfl_xor(v, 1));
+            if (NF == 3) v = fmax(v, __shfl_xor(v, 2));
+            if (lane == 0 && v > 0.0)
+                atomicMax(&a.red[DtRed::slot(blockIdx.x)],
+                          (unsigned long long)__double_as_longlong(v * a.dtp.vst_scale));
+        }
+    }
+    if constexpr (s == 0) {
+        // the end of the step: this launch neither reads the time nor dt, and the
+        // maxima are complete (stage 4 has ended)
+        if (a.step_end && blockIdx.x == 0 && wave == 0) {
+            const double h = next_dt(a.red, a.dtp, a.err);
+            if (lane == 0) {
+                a.scal[0] = advance_time(a.scal[0], a.scal[1]);
+                a.scal[1] = h;
+                *a.steps += 1;
+            }
+        }
+    }
     constexpr int GSH = s == 0 ? 0 : (NB * QG * (int)sizeof(T) + 7) / 8; // doubles of the staged box
     constexpr int per_wave = stage_lds_doubles_per_wave<NF, T, AUX>();
     static_assert(per_wave == 64 * 9 + 64 * NSR * (int)sizeof(T) / 8,
@@ -513,6 +640,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     const int bany = n0 > 0 ? beg : beg1; // a particle of the wave, for inactive lanes' loads
     // (one cell: the loop runs over the cell's run itself, base = beg + sbase)
     const int lo = CPW == 1 ? beg : 0, hi = CPW == 1 ? end : NSL;
+    int running = 0; // stage 1: lane 27 i + e holds the count of move e from the wave's cell i so far
     for (int base = lo; base < hi; base += 64) {
         const int sbase = base - lo;
         int64_t ip;
@@ -720,13 +848,40 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
                         else a.Y[(int64_t)c * a.np + ip] = Dep[c];
                     }
                 }
-                if (s == 1 && act) { // the end-of-step cell, for the sort before stage 4
-                    double v[3], npos[3];
+                if constexpr (s == 1) {
+                    // The sort plan's first part: the particle's move over the step
+                    // and its rank among the particles of its cell with that move,
+                    // in slot order (lane order within a chunk, chunks in order), so
+                    // that the sort is stable.  One pass per move present in the
+                    // chunk; most particles stay in their cell, so there are few.
+                    int e = 64;
+                    if (act) {
+                        double v[3], npos[3];
 #pragma unroll
-                    for (int d = 0; d < 3; d++) v[d] = double(pupv[d]) / double(pupt) * phys::c;
-                    int nc;
-                    end_position(pos, v, dt, g, npos, nc);
-                    a.newcell[ip] = nc;
+                        for (int d = 0; d < 3; d++) v[d] = double(pupv[d]) / double(pupt) * phys::c;
+                        end_position(pos, v, dt, g, npos);
+                        const int which = CPW == 2 && pcell != cell ? 1 : 0;
+                        bool bad = false;
+                        const int ex = move1(cx + which, npos[0], g.plo[0], g.dxi[0], g.n[0], bad);
+                        const int ey = move1(cy, npos[1], g.plo[1], g.dxi[1], g.n[1], bad);
+                        const int ez = move1(cz, npos[2], g.plo[2], g.dxi[2], g.n[2], bad);
+                        // only |p| > p_t outruns c dt < dx
+                        if (bad) atomicMin(a.err, status_word(a.cur.id[ip], EMU_ERR_MOVE));
+                        e = 27 * which + (ez + 1) * 9 + (ey + 1) * 3 + (ex + 1);
+                    }
+                    int myrank = 0;
+                    unsigned long long left = __ballot(act);
+                    while (left) {
+                        const int q = __builtin_amdgcn_readlane(e, __ffsll((long long)left) - 1);
+                        const unsigned long long msk = __ballot(e == q);
+                        if (e == q) myrank = __builtin_amdgcn_readlane(running, q) + __popcll(msk & ((1ull << lane) - 1ull));
+                        if (lane == q) running += __popcll(msk);
+                        left &= ~msk;
+                    }
+                    if (act) {
+                        a.rank[ip] = myrank;
+                        a.mv[ip] = (unsigned char)(e >= 27 ? e - 27 : e);
+                    }
                 }
             } else if (act) {
                 // y_{n+1} = acc + (dt/6) k4, then the post-step hook (main.cpp:155-199):
@@ -742,8 +897,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
                 double v[3], npos[3];
 #pragma unroll
                 for (int d = 0; d < 3; d++) v[d] = double(pupv[d]) / double(pupt) * phys::c;
-                int nc;
-                end_position(pos, v, dt, g, npos, nc);
+                end_position(pos, v, dt, g, npos);
                 const int64_t j = (int64_t)a.mbase[(int64_t)pcell * 27 + a.mv[ip]] + a.rank[ip];
                 if (j >= 0 && j < a.np) {
 #pragma unroll
@@ -868,6 +1022,9 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if constexpr (s == 1) {
+        if (inside_domain && lane < (inside1 ? 54 : 27)) a.mcount[(int64_t)cell * 27 + lane] = running;
     }
     if (!deposits) return;
     if constexpr (!MERGE) {

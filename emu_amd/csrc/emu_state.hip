@@ -3,13 +3,17 @@
 //
 // Per step (stage s reads the grid deposited from the stage-s state):
 //   stage 1..3 kernels (emu_stage.h): gather + Hamiltonian + commutator + RK
-//     update of the particle, then deposit of the next stage state into the
-//     other grid; stage 1 also bins each particle's end-of-step position;
-//   a stable counting sort plan by the new cell (ranks and bases);
-//   compute_dt reduction over the stage-4 deposit (main.cpp:193-197);
+//     update of the particle, then deposit of the next stage state into
+//     another grid; stage 1 also finds each particle's move over the step and
+//     its rank in it;
+//   a stable counting sort plan by the new cell (counts and bases);
 //   stage 4 kernel: y_{n+1}, positions, periodic shift, Renormalize (FP64),
-//     each particle written straight to its slot in the new cell order;
-//   the deposit of y_{n+1} that the next step's stage 1 reads.
+//     each particle written straight to its slot in the new cell order; and
+//     compute_dt's maximum over the stage-4 deposit (main.cpp:193-197);
+//   the deposit of y_{n+1} that the next step's stage 1 reads; and the next dt.
+// Seven launches, or six where one workgroup plans the sort.  Three grids take
+// turns, so that each stage sets to its base the one that a later stage
+// deposits into, in the same launch.
 //
 // The mesh holds, per cell and flavour component c, the combined fields
 //   M_c  = N_c - conj(Nbar)_c  (+ rho Ye/Mp dV on 00, the matter term)
@@ -54,110 +58,88 @@ __global__ void k_fill_grid(double* g, int64_t ncell, int Q, double m00, double*
 // particle's destination is base[old cell][e] + (its rank among the particles
 // of its old cell with the same e), which makes the order deterministic.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int move1(int from, int to, int n, int* bad)
-{
-    const int dd = pmod(to - from, n);
-    if (dd == 0) return 0;
-    if (dd == 1) return 1;
-    if (dd == n - 1) return -1;
-    *bad = 1;
-    return 0;
-}
+__device__ __forceinline__ int wrap_cell(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
-// One wave per old cell: move index and rank within (cell, move); m[c][e].
-// A move of more than one cell (only a particle with |p| > p_t can outrun
-// c dt < dx) is reported as EMU_ERR_MOVE with the particle's id.
-__global__ void k_move_ranks(const int* __restrict__ newcell, const int* __restrict__ cell_start,
-                             const int* __restrict__ cell_cnt, const int64_t* __restrict__ ids, Geom g,
-                             int* __restrict__ rank, unsigned char* __restrict__ mv, int* __restrict__ m,
-                             unsigned long long* err)
-{
-    const int c = blockIdx.x;
-    const int lane = threadIdx.x;
-    const int cx = c % g.n[0], cy = (c / g.n[0]) % g.n[1], cz = c / (g.n[0] * g.n[1]);
-    const int beg = cell_start[c], end = beg + cell_cnt[c];
-    int running = 0; // lane e (< 27) holds the running count of move e
-    for (int base = beg; base < end; base += 64) {
-        const int ip = base + lane;
-        const bool act = ip < end;
-        int e = 27;
-        if (act) {
-            const int t = newcell[ip];
-            const int tx = t % g.n[0], ty = (t / g.n[0]) % g.n[1], tz = t / (g.n[0] * g.n[1]);
-            int bad = 0;
-            const int ex = move1(cx, tx, g.n[0], &bad), ey = move1(cy, ty, g.n[1], &bad),
-                      ez = move1(cz, tz, g.n[2], &bad);
-            if (bad) atomicMin(err, status_word(ids[ip], EMU_ERR_MOVE));
-            e = (ez + 1) * 9 + (ey + 1) * 3 + (ex + 1);
-        }
-        // one pass per move present in the chunk (most particles stay in their
-        // cell, so there are few): the lanes of move q get ranks after the
-        // earlier chunks' particles of that move, in lane order
-        int myrank = 0;
-        unsigned long long left = __ballot(act);
-        while (left) {
-            const int q = __shfl(e, __ffsll((long long)left) - 1);
-            const unsigned long long msk = __ballot(act && e == q);
-            const int before = __shfl(running, q);
-            if (act && e == q) myrank = before + __popcll(msk & ((1ull << lane) - 1ull));
-            if (lane == q) running += __popcll(msk);
-            left &= ~msk;
-        }
-        if (act) {
-            rank[ip] = myrank;
-            mv[ip] = (unsigned char)e;
-        }
-    }
-    if (lane < 27) m[(int64_t)c * 27 + lane] = running;
-}
-
-__device__ __forceinline__ bool valid_move(int e, const Geom& g)
-{
-    const int ex = e % 3 - 1, ey = (e / 3) % 3 - 1, ez = e / 9 - 1;
-    const int ed[3] = {ex, ey, ez};
-    for (int d = 0; d < 3; d++) {
-        if (g.n[d] == 1 && ed[d] != 0) return false;
-        if (g.n[d] == 2 && ed[d] == -1) return false;
-    }
-    return true;
-}
-
-__device__ __forceinline__ int64_t source_of(int t, int e, const Geom& g)
+// f(e, source) for every move e that exists on the grid (a 1-cell dimension
+// has only move 0, a 2-cell one 0 and +1), with the cell that particles come
+// from into cell t by it; canonical order of e.
+template <typename F> __device__ __forceinline__ void for_moves(int t, const Geom& g, F&& f)
 {
     const int tx = t % g.n[0], ty = (t / g.n[0]) % g.n[1], tz = t / (g.n[0] * g.n[1]);
-    const int sx = pmod(tx - (e % 3 - 1), g.n[0]), sy = pmod(ty - ((e / 3) % 3 - 1), g.n[1]),
-              sz = pmod(tz - (e / 9 - 1), g.n[2]);
-    return ((int64_t)sz * g.n[1] + sy) * g.n[0] + sx;
+#pragma unroll
+    for (int ez = -1; ez <= 1; ez++)
+#pragma unroll
+        for (int ey = -1; ey <= 1; ey++)
+#pragma unroll
+            for (int ex = -1; ex <= 1; ex++) {
+                const int ed[3] = {ex, ey, ez};
+                bool ok = true;
+#pragma unroll
+                for (int d = 0; d < 3; d++) ok = ok && !(g.n[d] == 1 && ed[d] != 0) && !(g.n[d] == 2 && ed[d] == -1);
+                if (!ok) continue;
+                const int sx = wrap_cell(tx - ex, g.n[0]), sy = wrap_cell(ty - ey, g.n[1]), sz = wrap_cell(tz - ez, g.n[2]);
+                f((ez + 1) * 9 + (ey + 1) * 3 + (ex + 1), ((int64_t)sz * g.n[1] + sy) * g.n[0] + sx);
+            }
 }
 
-// cnt[t] = number of particles arriving in t, counts[t] = the slots they take
-// (cnt rounded up to a multiple of align); both 0 at t = ncell, for the scans.
-__global__ void k_new_counts(const int* __restrict__ m, Geom g, int64_t ncell, int align, int* __restrict__ counts,
-                             int* __restrict__ cnt)
+constexpr int kPlanBlock = 256;
+
+// base[source][e] for every source of target t, in canonical move order, from
+// the target's first slot.
+__device__ __forceinline__ void write_bases(int t, int first, const int* __restrict__ m, const Geom& g, int* __restrict__ base)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t > ncell) return;
+    int run = first;
+    for_moves(t, g, [&](int e, int64_t src) {
+        base[src * 27 + e] = run;
+        run += m[src * 27 + e];
+    });
+}
+
+// The sort plan, first part, one thread per target cell: cnt[t] = particles
+// arriving in t; start[t] = the first slot of its run (a multiple of align),
+// counted from the block's first; bsum[b] = the block's slots.  cnt[ncell] = 0
+// for the store's scan.  A grid of one block is planned here in full.
+__global__ __launch_bounds__(kPlanBlock) void k_plan_counts(const int* __restrict__ m, Geom g, int ncell, int align,
+                                                            int* __restrict__ start, int* __restrict__ cnt,
+                                                            int* __restrict__ bsum, int* __restrict__ base)
+{
+    using Scan = hipcub::BlockScan<int, kPlanBlock>;
+    __shared__ typename Scan::TempStorage tmp;
+    const int t = blockIdx.x * kPlanBlock + threadIdx.x;
     int n = 0;
-    if (t < ncell)
-        for (int e = 0; e < 27; e++)
-            if (valid_move(e, g)) n += m[source_of((int)t, e, g) * 27 + e];
-    cnt[t] = n;
-    counts[t] = (n + align - 1) / align * align;
+    if (t < ncell) for_moves(t, g, [&](int e, int64_t src) { n += m[src * 27 + e]; });
+    int first, total;
+    Scan(tmp).ExclusiveSum((n + align - 1) / align * align, first, total);
+    if (t <= ncell) cnt[t] = n;
+    if (t < ncell) start[t] = first;
+    if (gridDim.x > 1) {
+        if (threadIdx.x == 0) bsum[blockIdx.x] = total;
+    } else if (t < ncell) {
+        write_bases(t, first, m, g, base);
+    }
 }
 
-// base[s][e] for every source s = t - e, in canonical move order.
-__global__ void k_bases(const int* __restrict__ m, const int* __restrict__ new_start, Geom g, int64_t ncell,
-                        int* __restrict__ base)
+// The second part: every block sums the slots of the blocks before it (a few
+// thousand values at most), completes its cells' starts and writes the bases.
+// A scan kernel between the parts would be one more pass over the cells and two
+// more launches.
+__global__ __launch_bounds__(kPlanBlock) void k_plan_bases(const int* __restrict__ m, Geom g, int ncell,
+                                                           const int* __restrict__ bsum, int* __restrict__ start,
+                                                           int* __restrict__ base)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    using Reduce = hipcub::BlockReduce<int, kPlanBlock>;
+    __shared__ typename Reduce::TempStorage tmp;
+    __shared__ int before;
+    int s = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kPlanBlock) s += bsum[b];
+    s = Reduce(tmp).Sum(s);
+    if (threadIdx.x == 0) before = s;
+    __syncthreads();
+    const int t = blockIdx.x * kPlanBlock + threadIdx.x;
     if (t >= ncell) return;
-    int run = new_start[t];
-    for (int e = 0; e < 27; e++) {
-        if (!valid_move(e, g)) continue;
-        const int64_t sidx = source_of((int)t, e, g) * 27 + e;
-        base[sidx] = run;
-        run += m[sidx];
-    }
+    const int first = start[t] + before;
+    start[t] = first;
+    write_bases(t, first, m, g, base);
 }
 
 template <typename T> using Arrays = PArrays<T>;
@@ -217,52 +199,16 @@ __global__ void k_dt_reduce(const double* __restrict__ grid, const double* __res
         Vst = fmax(Vst, __shfl_xor(Vst, off));
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicMax(&red[0], (unsigned long long)__double_as_longlong(Vad > 0 ? Vad : 0.0));
-        atomicMax(&red[1], (unsigned long long)__double_as_longlong(Vst > 0 ? Vst : 0.0));
+        if (adaptive) atomicMax(&red[0], (unsigned long long)__double_as_longlong(Vad > 0 ? Vad : 0.0));
+        atomicMax(&red[DtRed::slot(blockIdx.x)], (unsigned long long)__double_as_longlong(Vst > 0 ? Vst : 0.0));
     }
 }
 
-struct DtParams {
-    double dt_translation, flavor_cfl, max_adaptive_speedup, Vvac_max, fixed_dt;
-    int use_flavor;
-};
-
-// main.cpp:193-198 and Evolve.cpp:57-88: the next dt from the reductions.
-__global__ void k_dt_finalize(const unsigned long long* red, DtParams p, double* dt_next, unsigned long long* err)
+// The starting dt, after a load.
+__global__ void k_dt_finalize(unsigned long long* red, DtParams p, double* dt, unsigned long long* err)
 {
-    if (threadIdx.x != 0) return;
-    if (p.fixed_dt > 0) { *dt_next = p.fixed_dt; return; }
-    double dt_flavor = 0.0;
-    if (p.use_flavor) {
-        const double vad = __longlong_as_double((long long)red[0]) + p.Vvac_max;
-        const double vst = __longlong_as_double((long long)red[1]) + p.Vvac_max;
-        const double dfa = phys::hbar / vad * p.flavor_cfl;
-        const double dfs = phys::hbar / vst * p.flavor_cfl;
-        dt_flavor = dfs;
-        if (p.max_adaptive_speedup > 1) dt_flavor = fmin(dfs * p.max_adaptive_speedup, dfa);
-    }
-    double dt = 0.0;
-    if (p.dt_translation != 0.0 && dt_flavor != 0.0) dt = fmin(p.dt_translation, dt_flavor);
-    else if (p.dt_translation != 0.0) dt = p.dt_translation;
-    else if (dt_flavor != 0.0) dt = dt_flavor;
-    else atomicMin(err, status_word_noindex(EMU_ERR_DT));
-    *dt_next = dt;
-}
-
-// End of step: particle time advanced by the four weighted stages, dt <- next.
-__global__ void k_step_end(double* time, double* dt, const double* dt_next, int64_t* steps)
-{
-#pragma clang fp contract(off)
-    if (threadIdx.x != 0) return;
-    const double h = *dt;
-    double t = *time;
-    t = h * (1. / 6.) * 1.0 + t;
-    t = h * (1. / 3.) * 1.0 + t;
-    t = h * (1. / 3.) * 1.0 + t;
-    t = h * (1. / 6.) * 1.0 + t;
-    *time = t;
-    *dt = *dt_next;
-    *steps += 1;
+    const double h = next_dt(red, p, err); // one wave
+    if (threadIdx.x == 0) *dt = h;
 }
 
 __global__ void k_fill_int(int* p, int64_t n, int v)
@@ -480,9 +426,8 @@ struct emu_state {
     // scratch
     void* Y = nullptr;
     void* acc = nullptr;
-    int* newcell = nullptr;
     int* rank = nullptr;
-    int* counts = nullptr;         // ncell + 1: the scan's input (padded counts)
+    int* counts = nullptr;         // ncell + 1: the scan's input (padded counts); a step's block sums
     int* cell_start = nullptr;     // ncell + 1
     int* new_start = nullptr;      // ncell + 1
     int* cell_cnt = nullptr;       // ncell + 1: particles per cell (current order)
@@ -490,15 +435,15 @@ struct emu_state {
     int* mcount = nullptr;         // [ncell][27] particles per (old cell, move)
     int* mbase = nullptr;          // [ncell][27] destination of the first of them
     unsigned char* mv = nullptr;   // move index per particle
-    double* grid[2] = {nullptr, nullptr};
+    double* grid[3] = {nullptr, nullptr, nullptr}; // [0] the current deposit, [1] at its base, [2] free
     double* aux = nullptr;
-    double* scal = nullptr;        // [0] time [1] dt [2] dt_next
+    double* scal = nullptr;        // [0] time [1] dt
     int64_t* steps = nullptr;
-    unsigned long long* red = nullptr; // [0..1] dt maxima, [2] error, [3] pupt min
+    unsigned long long* red = nullptr;   // [2] error, [3] pupt min, [4] weight maximum, [4..5] amplitude sums
+    unsigned long long* dtred = nullptr; // compute_dt's maxima (DtRed)
     void* cub_tmp = nullptr;
     size_t cub_bytes = 0;
     int cur = 0;      // which persistent copy is current
-    int gcur = 0;     // grid holding the deposit of the current state
     bool evolved = false; // a step was taken since the last load
     double Vvac_max = 0.0;
     double m00 = 0.0;
@@ -513,14 +458,18 @@ struct emu_state {
     int profile = 0;
     struct Mark { int k; hipEvent_t a, b; };
     std::vector<Mark> marks;
-    // the sort plan runs on a stream of its own, beside stages 2 and 3 (it
-    // needs stage 1's end-of-step cells, and only stage 4 reads it), and so
-    // does compute_dt, beside stage 4 and the step-end deposit
+    // on grids of more than kInlinePlanCells cells the sort plan runs on a stream
+    // of its own, beside stages 2 and 3 (it needs stage 1's moves, and only
+    // stage 4 reads it)
     hipStream_t side = nullptr;
-    hipEvent_t ev_stage1 = nullptr, ev_plan = nullptr, ev_stage3 = nullptr, ev_dt = nullptr;
+    hipEvent_t ev_stage1 = nullptr, ev_plan = nullptr;
 };
 
 namespace {
+
+// Up to here the plan's two small launches cost less in line than the event
+// pairs and the second stream that hide them.
+constexpr int64_t kInlinePlanCells = 32768;
 
 template <typename T> Arrays<T> arrays_of(emu_state* st, int copy)
 {
@@ -536,9 +485,6 @@ template <typename T> Arrays<T> arrays_of(emu_state* st, int copy)
     A.f = (T*)b;
     return A;
 }
-
-// The ids of the current copy (placed after the positions in either precision).
-const int64_t* current_ids(emu_state* st) { return arrays_of<double>(st, st->cur).id; }
 
 size_t persistent_bytes(int64_t np, int nh, size_t tsize)
 {
@@ -627,23 +573,59 @@ template <int NF, typename T> void launch_stage_shape(emu_state* st, StageArgs<T
     else launch_stage_t<NF, T, 3, 3, 3>(st, a);
 }
 
+DtParams dt_params(const emu_state* st, double fixed_dt)
+{
+    const emu_ctx* ctx = st->ctx;
+    const emu_params& p = ctx->p;
+    DtParams dp;
+    dp.dt_translation = p.cfl_factor > 0.0
+                            ? std::min(std::min(ctx->g.dx[0], ctx->g.dx[1]), ctx->g.dx[2]) / phys::c * p.cfl_factor
+                            : 0.0;
+    dp.flavor_cfl = p.flavor_cfl_factor;
+    dp.max_adaptive_speedup = p.max_adaptive_speedup;
+    dp.Vvac_max = st->Vvac_max;
+    dp.fixed_dt = fixed_dt;
+    dp.use_flavor = p.flavor_cfl_factor > 0.0;
+    dp.vst_scale = 2.0 * st->nf * M_SQRT2 * phys::GF / (ctx->g.cell_volume * st->nscale);
+    return dp;
+}
+
+// What a launch does besides its stage.
+struct StageExtra {
+    bool want_aux = false;     // deposit the compute_dt auxiliaries
+    double* gclear = nullptr;  // grid to set to its base
+    bool clear_aux = false;
+    bool want_dt = false;      // stage 4: the conservative flavour bound
+    bool step_end = false;     // stage 0: the next dt and the step's end
+    double fixed_dt = 0.0;
+};
+
 template <typename T>
-StageArgs<T> stage_args(emu_state* st, int stage, const double* gin, double* gout, bool want_aux)
+StageArgs<T> stage_args(emu_state* st, int stage, const double* gin, double* gout, const StageExtra& x)
 {
     StageArgs<T> a;
     a.cur = arrays_of<T>(st, st->cur);
     a.dst = arrays_of<T>(st, 1 - st->cur);
     a.Y = (T*)st->Y;
     a.acc = (T*)st->acc;
-    a.newcell = st->newcell;
-    a.mbase = st->mbase;
     a.rank = st->rank;
     a.mv = st->mv;
+    a.mcount = st->mcount;
+    a.mbase = st->mbase;
     a.cell_start = st->cell_start;
     a.cell_cnt = st->cell_cnt;
     a.gin = gin;
     a.gout = gout;
     a.aux = st->aux;
+    a.gclear = x.gclear;
+    a.clear_aux = x.clear_aux;
+    a.m00 = st->m00 * st->nscale;
+    a.want_dt = x.want_dt;
+    a.red = st->dtred;
+    a.step_end = x.step_end;
+    a.dtp = dt_params(st, x.fixed_dt);
+    a.scal = st->scal;
+    a.steps = st->steps;
     a.dt = st->scal + 1;
     a.err = st->red + 2;
     a.np = st->cap;
@@ -653,7 +635,7 @@ StageArgs<T> stage_args(emu_state* st, int stage, const double* gin, double* gou
     // where the adaptive bound is used (max_adaptive_speedup > 1).  FP64 deposits
     // the full set either way: measured at 64^3 x 92, its auxiliary stage ran
     // 2% slower with the diagonal sums alone (FP32-bulk's 1% faster).
-    a.want_aux = want_aux ? (st->ctx->p.max_adaptive_speedup > 1 || sizeof(T) == 8 ? 2 : 1) : 0;
+    a.want_aux = x.want_aux ? (st->ctx->p.max_adaptive_speedup > 1 || sizeof(T) == 8 ? 2 : 1) : 0;
     a.blocks_per_xcd = 0;
     a.g = st->ctx->g;
     const emu_ctx* ctx = st->ctx;
@@ -663,14 +645,14 @@ StageArgs<T> stage_args(emu_state* st, int stage, const double* gin, double* gou
     return a;
 }
 
-void launch_stage(emu_state* st, int stage, const double* gin, double* gout, bool want_aux)
+void launch_stage(emu_state* st, int stage, const double* gin, double* gout, const StageExtra& x)
 {
     if (st->precision == EMU_FP32_BULK) {
-        auto a = stage_args<float>(st, stage, gin, gout, want_aux);
+        auto a = stage_args<float>(st, stage, gin, gout, x);
         if (st->nf == 2) launch_stage_shape<2, float>(st, a);
         else launch_stage_shape<3, float>(st, a);
     } else {
-        auto a = stage_args<double>(st, stage, gin, gout, want_aux);
+        auto a = stage_args<double>(st, stage, gin, gout, x);
         if (st->nf == 2) launch_stage_shape<2, double>(st, a);
         else launch_stage_shape<3, double>(st, a);
     }
@@ -682,32 +664,24 @@ void fill_grid(emu_state* st, double* g, bool with_aux)
                        st->ncell, st->QG, st->m00 * st->nscale, with_aux ? st->aux : nullptr, st->naux);
 }
 
-int dt_from_grid(emu_state* st, const double* g, double fixed_dt, hipStream_t s = nullptr)
+// compute_dt's maxima over the cells of grid g and the auxiliaries, both bounds
+void dt_reduce(emu_state* st, const double* g)
 {
     emu_ctx* ctx = st->ctx;
-    const emu_params& p = ctx->p;
-    if (!s) s = ctx->stream;
-    hipLaunchKernelGGL(k_fill_u64v, dim3(1), dim3(64), 0, s, st->red, 2, 0ull);
-    const bool use_flavor = p.flavor_cfl_factor > 0.0;
-    const int adaptive = p.max_adaptive_speedup > 1 ? 1 : 0;
-    if (use_flavor && fixed_dt <= 0) {
-        if (st->nf == 2)
-            hipLaunchKernelGGL(k_dt_reduce<2>, dim3(grid_blocks(st->ncell)), dim3(256), 0, s, g, st->aux,
-                               st->ncell, ctx->g.cell_volume * st->nscale, st->m00 * st->nscale, adaptive, st->red);
-        else
-            hipLaunchKernelGGL(k_dt_reduce<3>, dim3(grid_blocks(st->ncell)), dim3(256), 0, s, g, st->aux,
-                               st->ncell, ctx->g.cell_volume * st->nscale, st->m00 * st->nscale, adaptive, st->red);
-    }
-    DtParams dp;
-    dp.dt_translation = p.cfl_factor > 0.0
-                            ? std::min(std::min(ctx->g.dx[0], ctx->g.dx[1]), ctx->g.dx[2]) / phys::c * p.cfl_factor
-                            : 0.0;
-    dp.flavor_cfl = p.flavor_cfl_factor;
-    dp.max_adaptive_speedup = p.max_adaptive_speedup;
-    dp.Vvac_max = st->Vvac_max;
-    dp.fixed_dt = fixed_dt;
-    dp.use_flavor = use_flavor;
-    hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(64), 0, s, st->red, dp, st->scal + 2, st->red + 2);
+    const int adaptive = ctx->p.max_adaptive_speedup > 1 ? 1 : 0;
+    const double vol = ctx->g.cell_volume * st->nscale, m00 = st->m00 * st->nscale;
+    const dim3 grid(grid_blocks(st->ncell)), block(256);
+    if (st->nf == 2) hipLaunchKernelGGL(k_dt_reduce<2>, grid, block, 0, ctx->stream, g, st->aux, st->ncell, vol, m00, adaptive, st->dtred);
+    else hipLaunchKernelGGL(k_dt_reduce<3>, grid, block, 0, ctx->stream, g, st->aux, st->ncell, vol, m00, adaptive, st->dtred);
+}
+
+// the starting dt (main.cpp:206) from grid g, into scal[1]
+int starting_dt(emu_state* st, const double* g)
+{
+    emu_ctx* ctx = st->ctx;
+    if (ctx->p.flavor_cfl_factor > 0.0) dt_reduce(st, g);
+    hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(64), 0, ctx->stream, st->dtred, dt_params(st, 0.0), st->scal + 1,
+                       st->red + 2);
     EMU_LAUNCH_CHECK(ctx, "compute_dt");
     return EMU_OK;
 }
@@ -759,7 +733,6 @@ extern "C" int emu_state_create(emu_ctx* ctx, int64_t np, int precision, emu_sta
     bool ok = hipMalloc(&st->block[0], pb) == hipSuccess && hipMalloc(&st->block[1], pb) == hipSuccess &&
               hipMalloc(&st->Y, (size_t)npa * 2 * st->nh * st->tsize) == hipSuccess &&
               hipMalloc(&st->acc, (size_t)npa * 2 * st->nh * st->tsize) == hipSuccess &&
-              hipMalloc(&st->newcell, (size_t)npa * sizeof(int)) == hipSuccess &&
               hipMalloc(&st->rank, (size_t)npa * sizeof(int)) == hipSuccess &&
               hipMalloc(&st->counts, (size_t)(st->ncell + 1) * sizeof(int)) == hipSuccess &&
               hipMalloc(&st->cell_start, (size_t)(st->ncell + 1) * sizeof(int)) == hipSuccess &&
@@ -771,16 +744,16 @@ extern "C" int emu_state_create(emu_ctx* ctx, int64_t np, int precision, emu_sta
               hipMalloc(&st->mv, (size_t)npa) == hipSuccess &&
               hipMalloc(&st->grid[0], (size_t)st->ncell * st->QG * sizeof(double)) == hipSuccess &&
               hipMalloc(&st->grid[1], (size_t)st->ncell * st->QG * sizeof(double)) == hipSuccess &&
+              hipMalloc(&st->grid[2], (size_t)st->ncell * st->QG * sizeof(double)) == hipSuccess &&
               hipMalloc(&st->aux, (size_t)st->ncell * st->naux * sizeof(double)) == hipSuccess &&
               hipMalloc(&st->scal, 4 * sizeof(double)) == hipSuccess &&
               hipMalloc(&st->steps, sizeof(int64_t)) == hipSuccess &&
-              hipMalloc(&st->red, 8 * sizeof(unsigned long long)) == hipSuccess;
+              hipMalloc(&st->red, 8 * sizeof(unsigned long long)) == hipSuccess &&
+              hipMalloc(&st->dtred, DtRed::words * sizeof(unsigned long long)) == hipSuccess;
     // default priority, and no implicit synchronisation with the legacy stream
     ok = ok && hipStreamCreateWithFlags(&st->side, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&st->ev_stage1, hipEventDisableTiming) == hipSuccess &&
-         hipEventCreateWithFlags(&st->ev_plan, hipEventDisableTiming) == hipSuccess &&
-         hipEventCreateWithFlags(&st->ev_stage3, hipEventDisableTiming) == hipSuccess &&
-         hipEventCreateWithFlags(&st->ev_dt, hipEventDisableTiming) == hipSuccess;
+         hipEventCreateWithFlags(&st->ev_plan, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
         emu_state_destroy(st);
         return set_error(ctx, EMU_ERR_NOMEM, "state allocation failed");
@@ -792,10 +765,10 @@ extern "C" int emu_state_create(emu_ctx* ctx, int64_t np, int precision, emu_sta
 extern "C" int emu_state_destroy(emu_state* st)
 {
     if (!st) return EMU_OK;
-    void* ptrs[] = {st->block[0], st->block[1], st->Y,        st->acc,     st->newcell, st->rank,
-                    st->counts,   st->cell_start, st->new_start, st->cell_cnt, st->new_cnt, st->mcount,
-                    st->mbase,    st->mv,         st->grid[0], st->grid[1], st->aux,
-                    st->scal,     st->steps,      st->red,     st->cub_tmp};
+    void* ptrs[] = {st->block[0], st->block[1],   st->Y,         st->acc,      st->rank,    st->counts, st->cell_start,
+                    st->new_start, st->cell_cnt,  st->new_cnt,   st->mcount,   st->mbase,   st->mv,     st->grid[0],
+                    st->grid[1],  st->grid[2],    st->aux,       st->scal,     st->steps,   st->red,    st->cub_tmp,
+                    st->dtred};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& m : st->marks) {
@@ -806,7 +779,7 @@ extern "C" int emu_state_destroy(emu_state* st)
         (void)hipStreamSynchronize(st->side);
         (void)hipStreamDestroy(st->side);
     }
-    for (hipEvent_t ev : {st->ev_stage1, st->ev_plan, st->ev_stage3, st->ev_dt})
+    for (hipEvent_t ev : {st->ev_stage1, st->ev_plan})
         if (ev) (void)hipEventDestroy(ev);
     delete st;
     return EMU_OK;
@@ -817,9 +790,10 @@ template <typename T> static int load_t(emu_state* st, const PView& P, const int
     emu_ctx* ctx = st->ctx;
     hipStream_t s = ctx->stream;
     const int64_t np = st->np;
+    int* keys = (int*)st->Y; // each particle's cell: the stage state is free until the first step
     hipLaunchKernelGGL(k_fill_int, dim3(grid_blocks(st->ncell + 1)), dim3(256), 0, s, st->counts, st->ncell + 1, 0);
     if (np > 0)
-        hipLaunchKernelGGL(k_bin_input, dim3(grid_blocks(np)), dim3(256), 0, s, P, ctx->g, st->newcell, st->counts);
+        hipLaunchKernelGGL(k_bin_input, dim3(grid_blocks(np)), dim3(256), 0, s, P, ctx->g, keys, st->counts);
     // the cells' first positions back to back (new_start, scratch here), then
     // their padded slot runs (cell_start)
     int e = scan_counts(st, st->counts, st->new_start);
@@ -852,10 +826,10 @@ template <typename T> static int load_t(emu_state* st, const PView& P, const int
     int end_bit = 1;
     while ((1ll << end_bit) < st->ncell) end_bit++;
     size_t need = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, need, st->newcell, keys_out, st->rank, order, (int)np, 0, end_bit,
+    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, need, keys, keys_out, st->rank, order, (int)np, 0, end_bit,
                                              s);
     if (ensure_cub(st, need)) e = set_error(ctx, EMU_ERR_NOMEM, "radix sort scratch");
-    if (!e && hipcub::DeviceRadixSort::SortPairs(st->cub_tmp, st->cub_bytes, st->newcell, keys_out, st->rank, order,
+    if (!e && hipcub::DeviceRadixSort::SortPairs(st->cub_tmp, st->cub_bytes, keys, keys_out, st->rank, order,
                                                  (int)np, 0, end_bit, s) != hipSuccess)
         e = set_error(ctx, EMU_ERR_HIP, "radix sort");
     if (!e) {
@@ -910,14 +884,16 @@ extern "C" int emu_state_load(emu_state* st, const emu_particles* parts, const i
     double sc[4] = {t0, 0.0, 0.0, 0.0};
     EMU_HIP(ctx, hipMemcpyAsync(st->scal, sc, sizeof sc, hipMemcpyHostToDevice, s));
     EMU_HIP(ctx, hipMemsetAsync(st->steps, 0, sizeof(int64_t), s));
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, s, (int*)st->dtred, (int64_t)2 * DtRed::words, 0);
     hipLaunchKernelGGL(k_fill_u64v, dim3(1), dim3(64), 0, s, st->red + 2, 1, ~0ull);
     // initial deposit (main.cpp:118) and starting dt (main.cpp:206)
-    st->gcur = 0;
     fill_grid(st, st->grid[0], true);
-    launch_stage(st, 0, nullptr, st->grid[0], true);
-    e = dt_from_grid(st, st->grid[0], 0.0);
+    fill_grid(st, st->grid[1], false);
+    StageExtra x;
+    x.want_aux = true;
+    launch_stage(st, 0, nullptr, st->grid[0], x);
+    e = starting_dt(st, st->grid[0]);
     if (e) return e;
-    EMU_HIP(ctx, hipMemcpyAsync(st->scal + 1, st->scal + 2, sizeof(double), hipMemcpyDeviceToDevice, s));
     EMU_HIP(ctx, hipStreamSynchronize(s));
     st->evolved = false;
     return EMU_OK;
@@ -931,11 +907,9 @@ extern "C" int emu_state_set_vvac_max(emu_state* st, double vvac_max)
     st->Vvac_max = vvac_max;
     // grid[0] (and aux) still hold the load's deposit: the starting dt again
     // (main.cpp:206) with the new value
-    const int e = dt_from_grid(st, st->grid[0], 0.0);
+    const int e = starting_dt(st, st->grid[0]);
     if (e) return e;
-    hipStream_t s = ctx->stream;
-    EMU_HIP(ctx, hipMemcpyAsync(st->scal + 1, st->scal + 2, sizeof(double), hipMemcpyDeviceToDevice, s));
-    EMU_HIP(ctx, hipStreamSynchronize(s));
+    EMU_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return EMU_OK;
 }
 
@@ -986,78 +960,66 @@ extern "C" int emu_state_evolve(emu_state* st, int nsteps, double fixed_dt)
     emu_ctx* ctx = st->ctx;
     hipStream_t s = ctx->stream;
     const Geom& g = ctx->g;
-    hipLaunchKernelGGL(k_fill_int, dim3(grid_blocks(st->ncell + 1)), dim3(256), 0, s, st->counts, st->ncell + 1, 0);
     // the deterministic sort assumes moves of at most one cell per step
     if (ctx->p.cfl_factor <= 0.0 || ctx->p.cfl_factor >= 1.0)
         if (fixed_dt <= 0 || fixed_dt * phys::c >= std::min(std::min(g.dx[0], g.dx[1]), g.dx[2]))
             return set_error(ctx, EMU_ERR_MOVE, "fused step needs c*dt < dx (0 < cfl_factor < 1)");
     if (fixed_dt > 0) EMU_HIP(ctx, hipMemcpyAsync(st->scal + 1, &fixed_dt, sizeof(double), hipMemcpyHostToDevice, s));
     if (nsteps > 0) st->evolved = true;
+    const bool flavor_dt = ctx->p.flavor_cfl_factor > 0.0 && fixed_dt <= 0;
+    const bool adaptive = flavor_dt && ctx->p.max_adaptive_speedup > 1;
+    const int ncell = (int)st->ncell, plan_blocks = (ncell + kPlanBlock) / kPlanBlock; // a thread for cell ncell too
+    const bool beside = st->ncell > kInlinePlanCells;
     for (int step = 0; step < nsteps; step++) {
-        double* A = st->grid[st->gcur];     // holds the deposit of y_n
-        double* B = st->grid[1 - st->gcur];
-        const bool want_aux = ctx->p.flavor_cfl_factor > 0.0 && fixed_dt <= 0;
-        ev_record(st, 1, true);
-        fill_grid(st, B, false);
-        ev_record(st, 1, false);
-        ev_record(st, 0, true);
-        launch_stage(st, 1, A, B, false);   // also bins the end-of-step positions
-        ev_record(st, 0, false);
-        // stable counting-sort plan by the new cell, on the side stream while
-        // stages 2 and 3 run (it reads stage 1's cells and the current run
-        // table; it writes only the plan, which stage 4 waits for)
-        hipStream_t ss = st->side;
-        EMU_HIP(ctx, hipEventRecord(st->ev_stage1, s));
-        EMU_HIP(ctx, hipStreamWaitEvent(ss, st->ev_stage1, 0));
+        // the grids' turns: A holds the deposit of y_n, B is at its base, C free
+        double *A = st->grid[0], *B = st->grid[1], *C = st->grid[2];
+        auto stage = [&](int k, const double* gin, double* gout, const StageExtra& x) {
+            ev_record(st, 0, true);
+            launch_stage(st, k, gin, gout, x);
+            ev_record(st, 0, false);
+        };
+        StageExtra x1, x2, x3, x4, x0;
+        x1.gclear = C;
+        stage(1, A, B, x1); // also the moves over the step
+        // the stable counting-sort plan by the new cell
+        hipStream_t ss = beside ? st->side : s;
+        if (beside) {
+            EMU_HIP(ctx, hipEventRecord(st->ev_stage1, s));
+            EMU_HIP(ctx, hipStreamWaitEvent(ss, st->ev_stage1, 0));
+        }
         ev_record(st, 2, true, ss);
-        hipLaunchKernelGGL(k_move_ranks, dim3((unsigned)st->ncell), dim3(64), 0, ss, st->newcell, st->cell_start,
-                           st->cell_cnt, current_ids(st), ctx->g, st->rank, st->mv, st->mcount, st->red + 2);
-        hipLaunchKernelGGL(k_new_counts, dim3(grid_blocks(st->ncell + 1)), dim3(256), 0, ss, st->mcount, ctx->g,
-                           st->ncell, st->align, st->counts, st->new_cnt);
-        int e = scan_counts(st, st->counts, st->new_start, ss);
-        if (e) return e;
-        hipLaunchKernelGGL(k_bases, dim3(grid_blocks(st->ncell)), dim3(256), 0, ss, st->mcount, st->new_start, ctx->g,
-                           st->ncell, st->mbase);
+        hipLaunchKernelGGL(k_plan_counts, dim3(plan_blocks), dim3(kPlanBlock), 0, ss, st->mcount, g, ncell, st->align,
+                           st->new_start, st->new_cnt, st->counts, st->mbase);
+        if (plan_blocks > 1)
+            hipLaunchKernelGGL(k_plan_bases, dim3(plan_blocks), dim3(kPlanBlock), 0, ss, st->mcount, g, ncell,
+                               st->counts, st->new_start, st->mbase);
         ev_record(st, 2, false, ss);
-        EMU_HIP(ctx, hipEventRecord(st->ev_plan, ss));
-        ev_record(st, 1, true);
-        fill_grid(st, A, false);
-        ev_record(st, 1, false);
-        ev_record(st, 0, true);
-        launch_stage(st, 2, B, A, false);
-        ev_record(st, 0, false);
-        ev_record(st, 1, true);
-        fill_grid(st, B, want_aux);
-        ev_record(st, 1, false);
-        ev_record(st, 0, true);
-        launch_stage(st, 3, A, B, want_aux);
-        ev_record(st, 0, false);
-        // compute_dt from stage 3's deposit, also on the side stream: it reads B
-        // beside stage 4 and writes the next dt, which k_step_end waits for
-        EMU_HIP(ctx, hipEventRecord(st->ev_stage3, s));
-        EMU_HIP(ctx, hipStreamWaitEvent(ss, st->ev_stage3, 0));
-        ev_record(st, 3, true, ss);
-        e = dt_from_grid(st, B, fixed_dt, ss);
-        ev_record(st, 3, false, ss);
-        if (e) return e;
-        EMU_HIP(ctx, hipEventRecord(st->ev_dt, ss));
-        EMU_HIP(ctx, hipStreamWaitEvent(s, st->ev_plan, 0));
-        ev_record(st, 0, true);
-        launch_stage(st, 4, B, nullptr, false); // writes y_{n+1} into the other copy, new order
-        ev_record(st, 0, false);
+        if (beside) EMU_HIP(ctx, hipEventRecord(st->ev_plan, ss));
+        x2.gclear = A;
+        x2.clear_aux = flavor_dt;
+        stage(2, B, C, x2);
+        x3.gclear = B;
+        x3.want_aux = flavor_dt;
+        stage(3, C, A, x3);
+        if (adaptive) {
+            ev_record(st, 3, true);
+            dt_reduce(st, A);
+            ev_record(st, 3, false);
+        }
+        if (beside) EMU_HIP(ctx, hipStreamWaitEvent(s, st->ev_plan, 0));
+        x4.gclear = C;
+        x4.want_dt = flavor_dt && !adaptive;
+        stage(4, A, nullptr, x4); // writes y_{n+1} into the other copy, new order
         st->cur = 1 - st->cur;
         std::swap(st->cell_start, st->new_start);
         std::swap(st->cell_cnt, st->new_cnt);
-        // deposit of y_{n+1} for the next step's stage 1
-        ev_record(st, 1, true);
-        fill_grid(st, A, false);
-        ev_record(st, 1, false);
-        ev_record(st, 0, true);
-        launch_stage(st, 0, nullptr, A, false);
-        ev_record(st, 0, false);
-        EMU_HIP(ctx, hipStreamWaitEvent(s, st->ev_dt, 0));
-        hipLaunchKernelGGL(k_step_end, dim3(1), dim3(64), 0, s, st->scal, st->scal + 1, st->scal + 2, st->steps);
-        if (fixed_dt > 0) EMU_HIP(ctx, hipMemcpyAsync(st->scal + 1, &fixed_dt, sizeof(double), hipMemcpyHostToDevice, s));
+        // deposit of y_{n+1} for the next step's stage 1, and the next dt
+        x0.step_end = true;
+        x0.fixed_dt = fixed_dt;
+        stage(0, nullptr, B, x0);
+        st->grid[0] = B;
+        st->grid[1] = C;
+        st->grid[2] = A;
         EMU_LAUNCH_CHECK(ctx, "state_evolve");
     }
     return EMU_OK;
