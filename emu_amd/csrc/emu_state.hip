@@ -253,28 +253,117 @@ __global__ void k_pad_counts(int* __restrict__ counts, int* __restrict__ cnt, in
 // Load: the j-th particle in (cell, input index) order is input particle
 // order[j] of cell key[j]; it takes slot start[key] + (j - ustart[key]), where
 // ustart are the cells' first positions back to back and start their slots.
+__global__ void k_load_slots(const int* __restrict__ order, const int* __restrict__ key, const int* __restrict__ start,
+                             const int* __restrict__ ustart, int64_t np, int* __restrict__ slot)
+{
+    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < np; j += (int64_t)gridDim.x * blockDim.x) {
+        const int c = key[j];
+        slot[order[j]] = start[c] + ((int)j - ustart[c]);
+    }
+}
+
+// A loaded particle as one record of 8-byte words: position, id, then in T
+// pup[4], N, Nbar, L, Lbar and the flavour rows.  A record has exactly the bytes
+// that the particle takes in a copy of the state's arrays.
+template <int NF, typename T> struct LoadRec {
+    static constexpr int nh = NH<NF>, N = 4, L = 6, F = 8; // T entries after the 4 words
+    static constexpr int words = 4 + (8 + 2 * nh) * (int)sizeof(T) / 8;
+    static constexpr int row = words | 1; // LDS row stride: odd, so that rows spread over the banks
+    static constexpr int waves = 2;       // per workgroup, 2 x 64 rows of LDS (32 KB at most)
+};
+
+// The load goes through records because the caller's particles come in their
+// own order (a run under way has scattered directions): reading every array
+// through the sort order fetched a cache line per value (12 ms at 24.1 M
+// particles).  Here a wave reads its 64 particles coalesced, transposes them in
+// LDS and writes each record in one piece to its slot; k_load_unpack then turns
+// the records, in slot order, into the state's arrays (together 5.1 ms in
+// FP32-bulk, 8.0 in FP64).
 template <int NF, typename T>
-__global__ void k_load(PView P, const int64_t* ids, const int* __restrict__ order, const int* __restrict__ key,
-                       const int* __restrict__ start, const int* __restrict__ ustart, Arrays<T> dst, int64_t np,
-                       int64_t stride, double nscale)
+__global__ __launch_bounds__((64 * LoadRec<NF, T>::waves)) void k_load_pack(PView P, const int64_t* __restrict__ ids,
+                                                                            const int* __restrict__ slot,
+                                                                            int64_t* __restrict__ rec, double nscale)
 {
     using I = PIdx<NF>;
-    constexpr int nh = NH<NF>;
-    for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < np; j += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t ip = order[j];
-        const int c = key[j];
-        const int64_t k = start[c] + (j - ustart[c]);
-        for (int d = 0; d < 3; d++) dst.pos[d][k] = P.pos[d][ip];
-        for (int d = 0; d < 4; d++) dst.pup[d][k] = T(P.r[I::pupx + d][ip]);
-        dst.Nn[0][k] = T(P.r[I::N][ip] * nscale);
-        dst.Nn[1][k] = T(P.r[I::Nbar][ip] * nscale);
-        dst.Ll[0][k] = T(P.r[I::L][ip]);
-        dst.Ll[1][k] = T(P.r[I::Lbar][ip]);
-        dst.id[k] = ids ? ids[ip] : ip;
-        for (int c2 = 0; c2 < nh; c2++) {
-            dst.f[(int64_t)c2 * stride + k] = T(P.r[I::f + c2][ip]);
-            dst.f[(int64_t)(nh + c2) * stride + k] = T(P.r[I::fbar + c2][ip]);
+    using R = LoadRec<NF, T>;
+    constexpr int nh = R::nh;
+    __shared__ int64_t lds[64 * R::waves * R::row];
+    const int lane = threadIdx.x & 63;
+    int64_t* wl = lds + (threadIdx.x - lane) * R::row;
+    const int64_t ip = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const bool act = ip < P.np;
+    const int64_t ipl = act ? ip : P.np - 1;
+    const int k = act ? slot[ipl] : -1;
+    {
+        int64_t* r = wl + lane * R::row;
+        T* t = (T*)(r + 4);
+        for (int d = 0; d < 3; d++) r[d] = __double_as_longlong(P.pos[d][ipl]);
+        r[3] = ids ? ids[ipl] : ipl;
+        for (int d = 0; d < 4; d++) t[d] = T(P.r[I::pupx + d][ipl]);
+        t[R::N] = T(P.r[I::N][ipl] * nscale);
+        t[R::N + 1] = T(P.r[I::Nbar][ipl] * nscale);
+        t[R::L] = T(P.r[I::L][ipl]);
+        t[R::L + 1] = T(P.r[I::Lbar][ipl]);
+#pragma unroll
+        for (int c = 0; c < nh; c++) {
+            t[R::F + c] = T(P.r[I::f + c][ipl]);
+            t[R::F + nh + c] = T(P.r[I::fbar + c][ipl]);
         }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int j = 0; j < R::words; j++) {
+        const int e = j * 64 + lane, r = e / R::words, w = e - r * R::words;
+        const int dst = __shfl(k, r);
+        if (dst >= 0) rec[(int64_t)dst * R::words + w] = wl[r * R::row + w];
+    }
+}
+
+// The records of all `cap` slots into the state's arrays (slots between the
+// cells' runs hold nothing, before and after).
+template <int NF, typename T>
+__global__ __launch_bounds__((64 * LoadRec<NF, T>::waves)) void k_load_unpack(const int64_t* __restrict__ rec,
+                                                                              Arrays<T> dst, int64_t cap)
+{
+    using R = LoadRec<NF, T>;
+    constexpr int nh = R::nh;
+    __shared__ int64_t lds[64 * R::waves * R::row];
+    const int lane = threadIdx.x & 63;
+    int64_t* wl = lds + (threadIdx.x - lane) * R::row;
+    const int64_t k0 = blockIdx.x * (int64_t)blockDim.x + (threadIdx.x - lane), k = k0 + lane;
+    const int64_t n = (cap - k0 < 64 ? cap - k0 : 64) * R::words; // words of this wave's records
+#pragma unroll
+    for (int j = 0; j < R::words; j++) {
+        const int e = j * 64 + lane, r = e / R::words, w = e - r * R::words;
+        if (e < n) wl[r * R::row + w] = rec[k0 * R::words + e];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (k >= cap) return;
+    const int64_t* r = wl + lane * R::row;
+    const T* t = (const T*)(r + 4);
+    for (int d = 0; d < 3; d++) dst.pos[d][k] = __longlong_as_double(r[d]);
+    dst.id[k] = r[3];
+    for (int d = 0; d < 4; d++) dst.pup[d][k] = t[d];
+    for (int d = 0; d < 2; d++) dst.Nn[d][k] = t[R::N + d];
+    for (int d = 0; d < 2; d++) dst.Ll[d][k] = t[R::L + d];
+#pragma unroll
+    for (int c = 0; c < 2 * nh; c++) dst.f[(int64_t)c * cap + k] = t[R::F + c];
+}
+
+// Load: the scalars of a fresh state.
+__global__ void k_load_scalars(double* scal, const double* time, int64_t* steps, unsigned long long* err,
+                               unsigned long long* dtred)
+{
+    for (int i = threadIdx.x; i < DtRed::words; i += blockDim.x) dtred[i] = 0;
+    if (threadIdx.x == 0) {
+        scal[0] = time ? *time : 0.0; // all particles share it (main.cpp:101-110)
+        scal[1] = 0.0;
+        *steps = 0;
+        *err = ~0ull;
     }
 }
 
@@ -312,25 +401,32 @@ __global__ void k_store(Arrays<T> src, PView P, int64_t* ids, const double* time
     }
 }
 
-// max(|N|, |Nbar|) as the bit pattern of a non-negative double (those order
-// like unsigned integers)
-__global__ void k_absmax2(const double* __restrict__ a, const double* __restrict__ b, int64_t np,
-                          unsigned long long* red)
+// Load: red[0] = min pupt and red[1] = max(|N|, |Nbar|) as the bit patterns of
+// non-negative doubles (those order like unsigned integers).
+__global__ void k_load_ranges(const double* __restrict__ pupt, const double* __restrict__ N,
+                              const double* __restrict__ Nbar, int64_t np, unsigned long long* red)
 {
-    double v = 0.0;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < np; t += (int64_t)gridDim.x * blockDim.x)
-        v = fmax(v, fmax(fabs(a[t]), fabs(b[t])));
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(red, (unsigned long long)__double_as_longlong(v));
+    double lo = INFINITY, hi = 0.0;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < np; t += (int64_t)gridDim.x * blockDim.x) {
+        lo = fmin(lo, pupt[t]);
+        hi = fmax(hi, fmax(fabs(N[t]), fabs(Nbar[t])));
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, off));
+        hi = fmax(hi, __shfl_xor(hi, off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMin(&red[0], (unsigned long long)__double_as_longlong(lo));
+        atomicMax(&red[1], (unsigned long long)__double_as_longlong(hi));
+    }
 }
 
-__global__ void k_min_pupt_t(const double* __restrict__ pupt, int64_t np, unsigned long long* red)
+__global__ void k_load_ranges_init(unsigned long long* red)
 {
-    double v = INFINITY;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < np; t += (int64_t)gridDim.x * blockDim.x)
-        v = fmin(v, pupt[t]);
-    for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off));
-    if ((threadIdx.x & 63) == 0) atomicMin(red, (unsigned long long)__double_as_longlong(v));
+    if (threadIdx.x == 0) {
+        red[0] = ~0ull >> 1;
+        red[1] = 0;
+    }
 }
 
 // Diagnostic: per cell N_01 = sum_p w N f01 and Nbar_01 (Re, Im), deposited
@@ -790,10 +886,16 @@ template <typename T> static int load_t(emu_state* st, const PView& P, const int
     emu_ctx* ctx = st->ctx;
     hipStream_t s = ctx->stream;
     const int64_t np = st->np;
-    int* keys = (int*)st->Y; // each particle's cell: the stage state is free until the first step
+    // scratch: the stage state's and the accumulator's arrays, free until the
+    // first step (at least 32 bytes per slot each), and the other copy's block
+    int* cells = (int*)st->Y;
+    int* keys = cells + st->cap;
+    int* iota = keys + st->cap;
+    int* order = (int*)st->acc;
+    int* slot = order + st->cap;
     hipLaunchKernelGGL(k_fill_int, dim3(grid_blocks(st->ncell + 1)), dim3(256), 0, s, st->counts, st->ncell + 1, 0);
     if (np > 0)
-        hipLaunchKernelGGL(k_bin_input, dim3(grid_blocks(np)), dim3(256), 0, s, P, ctx->g, keys, st->counts);
+        hipLaunchKernelGGL(k_bin_input, dim3(grid_blocks(np)), dim3(256), 0, s, P, ctx->g, cells, st->counts);
     // the cells' first positions back to back (new_start, scratch here), then
     // their padded slot runs (cell_start)
     int e = scan_counts(st, st->counts, st->new_start);
@@ -803,76 +905,58 @@ template <typename T> static int load_t(emu_state* st, const PView& P, const int
     e = scan_counts(st, st->counts, st->cell_start);
     if (e) return e;
     if (np == 0) return EMU_OK;
-    st->nscale = 1.0;
-    if (st->precision == EMU_FP32_BULK) {
-        using I2 = PIdx<2>;
-        const int iN = I2::N, iNb = st->nf == 2 ? PIdx<2>::Nbar : PIdx<3>::Nbar;
-        hipLaunchKernelGGL(k_fill_u64v, dim3(1), dim3(64), 0, s, st->red + 4, 1, 0ull);
-        hipLaunchKernelGGL(k_absmax2, dim3(std::min(grid_blocks(np), 1024u)), dim3(256), 0, s, P.r[iN], P.r[iNb], np, st->red + 4);
-        unsigned long long h = 0;
-        EMU_HIP(ctx, hipMemcpyAsync(&h, st->red + 4, 8, hipMemcpyDeviceToHost, s));
-        EMU_HIP(ctx, hipStreamSynchronize(s));
-        double nmax;
-        std::memcpy(&nmax, &h, 8);
-        if (nmax > 0.0 && std::isfinite(nmax)) st->nscale = std::ldexp(1.0, -std::ilogb(nmax));
-    }
-    // stable radix sort of (cell, input index): sorted slot j <- input order[j]
-    int *keys_out = nullptr, *order = nullptr;
-    if (hipMalloc(&keys_out, np * sizeof(int)) != hipSuccess || hipMalloc(&order, np * sizeof(int)) != hipSuccess) {
-        if (keys_out) (void)hipFree(keys_out);
-        return set_error(ctx, EMU_ERR_NOMEM, "load sort scratch");
-    }
-    hipLaunchKernelGGL(k_iota, dim3(grid_blocks(np)), dim3(256), 0, s, st->rank, np);
+    // stable radix sort of (cell, input index)
+    hipLaunchKernelGGL(k_iota, dim3(grid_blocks(np)), dim3(256), 0, s, iota, np);
     int end_bit = 1;
     while ((1ll << end_bit) < st->ncell) end_bit++;
     size_t need = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, need, keys, keys_out, st->rank, order, (int)np, 0, end_bit,
-                                             s);
-    if (ensure_cub(st, need)) e = set_error(ctx, EMU_ERR_NOMEM, "radix sort scratch");
-    if (!e && hipcub::DeviceRadixSort::SortPairs(st->cub_tmp, st->cub_bytes, keys, keys_out, st->rank, order,
-                                                 (int)np, 0, end_bit, s) != hipSuccess)
-        e = set_error(ctx, EMU_ERR_HIP, "radix sort");
-    if (!e) {
-        Arrays<T> A = arrays_of<T>(st, st->cur);
-        if (st->nf == 2)
-            hipLaunchKernelGGL((k_load<2, T>), dim3(grid_blocks(np)), dim3(256), 0, s, P, ids, order, keys_out,
-                               st->cell_start, st->new_start, A, np, st->cap, st->nscale);
-        else
-            hipLaunchKernelGGL((k_load<3, T>), dim3(grid_blocks(np)), dim3(256), 0, s, P, ids, order, keys_out,
-                               st->cell_start, st->new_start, A, np, st->cap, st->nscale);
-        if (hipGetLastError() != hipSuccess) e = set_error(ctx, EMU_ERR_HIP, "state_load");
+    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, need, cells, keys, iota, order, (int)np, 0, end_bit, s);
+    if (ensure_cub(st, need)) return set_error(ctx, EMU_ERR_NOMEM, "radix sort scratch");
+    if (hipcub::DeviceRadixSort::SortPairs(st->cub_tmp, st->cub_bytes, cells, keys, iota, order, (int)np, 0, end_bit,
+                                           s) != hipSuccess)
+        return set_error(ctx, EMU_ERR_HIP, "radix sort");
+    hipLaunchKernelGGL(k_load_slots, dim3(grid_blocks(np)), dim3(256), 0, s, order, keys, st->cell_start, st->new_start,
+                       np, slot);
+    const Arrays<T> A = arrays_of<T>(st, st->cur);
+    int64_t* rec = (int64_t*)st->block[1 - st->cur];
+    const unsigned block = 64 * LoadRec<2, T>::waves;
+    const dim3 gp((unsigned)((np + block - 1) / block)), gu((unsigned)((st->cap + block - 1) / block));
+    if (st->nf == 2) {
+        hipLaunchKernelGGL((k_load_pack<2, T>), gp, dim3(block), 0, s, P, ids, slot, rec, st->nscale);
+        hipLaunchKernelGGL((k_load_unpack<2, T>), gu, dim3(block), 0, s, rec, A, st->cap);
+    } else {
+        hipLaunchKernelGGL((k_load_pack<3, T>), gp, dim3(block), 0, s, P, ids, slot, rec, st->nscale);
+        hipLaunchKernelGGL((k_load_unpack<3, T>), gu, dim3(block), 0, s, rec, A, st->cap);
     }
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(keys_out);
-    (void)hipFree(order);
-    return e;
+    EMU_LAUNCH_CHECK(ctx, "state_load");
+    return EMU_OK;
 }
 
 extern "C" int emu_state_load(emu_state* st, const emu_particles* parts, const int64_t* ids)
 {
     if (!st || !parts || parts->np != st->np) return EMU_ERR_ARG;
     emu_ctx* ctx = st->ctx;
+    hipStream_t s = ctx->stream;
     PView P;
     P.np = parts->np;
     const int na = 12 + 2 * st->nh;
     for (int d = 0; d < 3; d++) P.pos[d] = parts->pos[d];
     for (int k = 0; k < EMU_MAX_ATTRIBS; k++) P.r[k] = k < na ? parts->rdata[k] : nullptr;
+    // the least energy and the largest weight
+    hipLaunchKernelGGL(k_load_ranges_init, dim3(1), dim3(64), 0, s, st->red + 3);
+    if (st->np > 0)
+        hipLaunchKernelGGL(k_load_ranges, dim3(std::min(grid_blocks(st->np), 1024u)), dim3(256), 0, s,
+                           P.r[PIdx<2>::pupt], P.r[PIdx<2>::N], P.r[st->nf == 2 ? (int)PIdx<2>::Nbar : (int)PIdx<3>::Nbar],
+                           st->np, st->red + 3);
+    double range[2];
+    EMU_HIP(ctx, hipMemcpyAsync(range, st->red + 3, sizeof range, hipMemcpyDeviceToHost, s));
+    EMU_HIP(ctx, hipStreamSynchronize(s));
+    const double pupt_min = range[0], nmax = range[1];
+    st->nscale = 1.0;
+    if (st->precision == EMU_FP32_BULK && nmax > 0.0 && std::isfinite(nmax)) st->nscale = std::ldexp(1.0, -std::ilogb(nmax));
     int e = st->precision == EMU_FP32_BULK ? load_t<float>(st, P, ids) : load_t<double>(st, P, ids);
     if (e) return e;
-    hipStream_t s = ctx->stream;
-    // time of the particles (all particles share it; main.cpp:101-110)
-    double t0 = 0.0;
-    if (st->np > 0) EMU_HIP(ctx, hipMemcpyAsync(&t0, parts->rdata[PIdx<2>::time], sizeof(double), hipMemcpyDeviceToHost, s));
     // Vvac_max from the minimum energy (FlavoredNeutrinoContainerInit.cpp:657-660)
-    hipLaunchKernelGGL(k_fill_u64v, dim3(1), dim3(64), 0, s, st->red, 4, ~0ull >> 1);
-    if (st->np > 0)
-        hipLaunchKernelGGL(k_min_pupt_t, dim3(std::min(grid_blocks(st->np), 1024u)), dim3(256), 0, s, parts->rdata[PIdx<2>::pupt], st->np,
-                           st->red + 3);
-    unsigned long long h;
-    EMU_HIP(ctx, hipMemcpyAsync(&h, st->red + 3, 8, hipMemcpyDeviceToHost, s));
-    EMU_HIP(ctx, hipStreamSynchronize(s));
-    double pupt_min;
-    std::memcpy(&pupt_min, &h, 8);
     double d[9] = {0};
     if (st->nf == 2) {
         for (int i = 0; i < 2; i++) d[herm_re<2>(i, i)] = ctx->p.mass[i] * ctx->p.mass[i];
@@ -881,11 +965,8 @@ extern "C" int emu_state_load(emu_state* st, const emu_particles* parts, const i
         for (int i = 0; i < 3; i++) d[herm_re<3>(i, i)] = ctx->p.mass[i] * ctx->p.mass[i];
         st->Vvac_max = std::sqrt(su_mag2<3, double>(d)) * phys::c4 / pupt_min;
     }
-    double sc[4] = {t0, 0.0, 0.0, 0.0};
-    EMU_HIP(ctx, hipMemcpyAsync(st->scal, sc, sizeof sc, hipMemcpyHostToDevice, s));
-    EMU_HIP(ctx, hipMemsetAsync(st->steps, 0, sizeof(int64_t), s));
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(256), 0, s, (int*)st->dtred, (int64_t)2 * DtRed::words, 0);
-    hipLaunchKernelGGL(k_fill_u64v, dim3(1), dim3(64), 0, s, st->red + 2, 1, ~0ull);
+    hipLaunchKernelGGL(k_load_scalars, dim3(1), dim3(256), 0, s, st->scal, st->np > 0 ? P.r[PIdx<2>::time] : nullptr,
+                       st->steps, st->red + 2, st->dtred);
     // initial deposit (main.cpp:118) and starting dt (main.cpp:206)
     fill_grid(st, st->grid[0], true);
     fill_grid(st, st->grid[1], false);
