@@ -30,25 +30,26 @@ namespace emu {
 typedef double mf_d4 __attribute__((ext_vector_type(4)));
 typedef float mf_f4 __attribute__((ext_vector_type(4)));
 
-// One 16x16x4 matrix-core step in the precision of T.  Element r of lane l of
-// the result holds row 4r + l/16 (f64) or 4(l/16) + r (f32), column l%16.
-template <typename T> struct Mfma;
-template <> struct Mfma<double> {
-    typedef mf_d4 acc_t;
-    static __device__ __forceinline__ acc_t step(double a, double b, acc_t c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int r, int lane) { return 4 * r + (lane >> 4); }
-};
-template <> struct Mfma<float> {
-    typedef mf_f4 acc_t;
-    static __device__ __forceinline__ acc_t step(float a, float b, acc_t c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int r, int lane) { return 4 * (lane >> 4) + r; }
-};
+// Transpose of a 4 x 4 block of 16-lane rows: row i of register k <-> row k of
+// register i.
+__device__ __forceinline__ void transpose_rows(float& a, float& b, float& c, float& d)
+{
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    auto swap32 = [](float& x, float& y) { // upper half of x <-> lower half of y
+        const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+        x = __uint_as_float(r[0]);
+        y = __uint_as_float(r[1]);
+    };
+    auto swap16 = [](float& x, float& y) { // odd rows of x <-> even rows of y
+        const u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+        x = __uint_as_float(r[0]);
+        y = __uint_as_float(r[1]);
+    };
+    swap32(a, c);
+    swap32(b, d);
+    swap16(a, b);
+    swap16(c, d);
+}
 
 template <typename T> struct PArrays {
     double* pos[3];
@@ -555,6 +556,17 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         tdx[m][1] = 3 + (WY == 1 ? 1 : jj);
         tdx[m][2] = 6 + (WZ == 1 ? 1 : kk);
     }
+    // FP32-bulk's gather: this lane's entry of A at step k, row i = l%16 (group
+    // i%4, component i/4 of the step's four), neighbour t = 4k + l/16 (past the
+    // last one: any in-range entry, its weight is zero; rows past NH feed results
+    // that are dropped)
+    constexpr int KG = sizeof(T) == 4 && s != 0 ? (NT + 3) / 4 : 1;
+    int goff[KG];
+#pragma unroll
+    for (int k = 0; k < KG; k++) {
+        const int t = 4 * k + (lane >> 4);
+        goff[k] = box_of(t < NT ? t : NT - 1) * QG + (lane & 3) * nh + ((lane & 15) >> 2);
+    }
     // The last columns, when at most 8 remain past the 16-column tiles (NF = 3:
     // 36 = 2 x 16 + 4 without the auxiliaries, 39 = 2 x 16 + 7 with the
     // diagonal ones), run as 4-column tiles on the 4-block 4x4x4 form instead:
@@ -697,8 +709,71 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         } else {
             // ---- gather on the matrix cores, 16 particles per tile
             T inside[nh];
-            {
-                using MF = Mfma<T>;
+            const int ntile = CPW == 1 ? (min(64, end - base) + 15) >> 4 : min(4, (NSL + 15 - sbase) >> 4);
+            if constexpr (sizeof(T) == 4) {
+                // FP32-bulk: per tile of 16 particles the product is G^T W.  A's rows
+                // are 4 components x the 4 field groups, K the neighbours (4 per
+                // step), B's columns the particles, so that a lane's four results are
+                // the four groups of one component of one particle, and contracting
+                // them with s is 3 FMAs in the lane: 7 steps per 4 components
+                // (ceil(27 / 4)) instead of 27 steps whose 16 columns hold NH.
+                // The particle's own lane forms its 27 weights once; a transpose of
+                // 16-lane rows turns four of them into the operands of all four
+                // tiles, and another returns the results, without LDS.
+                constexpr int KK = (NT + 3) / 4, MG = (nh + 3) / 4;
+                const int c16 = lane & 15;
+                T w[4 * KK];
+                {
+                    T fx[3], fyz[3][3];
+#pragma unroll
+                    for (int ii = 0; ii < 3; ii++) fx[ii] = T(wd[0][ii]);
+#pragma unroll
+                    for (int kk = 0; kk < 3; kk++)
+#pragma unroll
+                        for (int jj = 0; jj < 3; jj++) fyz[kk][jj] = T(wd[1][jj]) * T(wd[2][kk]);
+#pragma unroll
+                    for (int t = 0; t < 4 * KK; t++) {
+                        const int ii = WX == 1 ? 1 : t % WX, jj = WY == 1 ? 1 : (t / WX) % WY,
+                                  kk = WZ == 1 ? 1 : (t / (WX * WY)) % 3;
+                        w[t] = t < NT ? fx[ii] * fyz[kk][jj] : T(0);
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < KK; k++) transpose_rows(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+                // w[4 k + m] now holds tile m's operand of step k
+                T res[4 * MG][4];
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+#pragma unroll
+                    for (int c = 0; c < MG; c++) res[c][m] = T(0);
+                    if (m < ntile) {
+                        // the tile's cell's neighbourhood: the second cell's box is one
+                        // column further along x (box rows of QG values)
+                        const T* Gt = Gs + (CPW == 2 && (sbase >> 4) + m >= T0 ? QG : 0);
+                        const T* vp = Src + (16 * m + c16) * NSR + nh;
+                        const T v0 = vp[0], v1 = vp[1], v2 = vp[2];
+                        mf_f4 acc_g[MG];
+#pragma unroll
+                        for (int c = 0; c < MG; c++) acc_g[c] = mf_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int k = 0; k < KK; k++)
+#pragma unroll
+                            for (int c = 0; c < MG; c++)
+                                acc_g[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(Gt[goff[k] + 4 * c], w[4 * k + m],
+                                                                                acc_g[c], 0, 0, 0);
+#pragma unroll
+                        for (int c = 0; c < MG; c++)
+                            res[c][m] = acc_g[c][0] - v0 * acc_g[c][1] - v1 * acc_g[c][2] - v2 * acc_g[c][3];
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < MG; c++) {
+                    transpose_rows(res[c][0], res[c][1], res[c][2], res[c][3]);
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (4 * c + j < nh) inside[4 * c + j] = res[c][j];
+                }
+            } else {
                 const int g4 = lane >> 4, c16 = lane & 15;
                 // B columns past NH only feed result columns that are dropped, so
                 // every lane reads an in-range entry, unmasked
@@ -710,13 +785,9 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
                     const int c = 4 * cb + (lane & 3);
                     cqb[cb] = g4 * nh + (c < nh ? c : nh - 1);
                 }
-                const int ntile = CPW == 1 ? (min(64, end - base) + 15) >> 4 : min(4, (NSL + 15 - sbase) >> 4);
 #pragma unroll 1
                 for (int m = 0; m < ntile; m++) {
                     const int p = 16 * m + c16; // the particle of this lane's A rows
-                    // the tile's cell's neighbourhood: the second cell's box is one
-                    // column further along x (box rows of QG values)
-                    const T* Gt = Gs + (CPW == 2 && (sbase >> 4) + m >= T0 ? QG : 0);
                     double w3[9];
 #pragma unroll
                     for (int e = 0; e < 9; e++) w3[e] = Wf[p * 9 + e];
@@ -724,9 +795,6 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
                     const T v0 = vp[0], v1 = vp[1], v2 = vp[2];
                     const T sg = g4 == 0 ? T(1) : (g4 == 1 ? -v0 : (g4 == 2 ? -v1 : -v2));
                     // A = (w_x s_g) (w_y w_z): 3 + WY WZ products, then one per target
-                    // (FP32-bulk forms w_y w_z in FP32 from the rounded factors, one
-                    // conversion per factor instead of one per product: the A
-                    // operand is FP32 either way)
                     T ax[WX], ayz[WY * WZ];
 #pragma unroll
                     for (int ii = 0; ii < WX; ii++) ax[ii] = T(w3[WX == 1 ? 1 : ii]) * sg;
@@ -734,46 +802,29 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
                     for (int kk = 0; kk < WZ; kk++)
 #pragma unroll
                         for (int jj = 0; jj < WY; jj++)
-                            ayz[kk * WY + jj] = sizeof(T) == 4
-                                                     ? T(w3[3 + (WY == 1 ? 1 : jj)]) * T(w3[6 + (WZ == 1 ? 1 : kk)])
-                                                     : T(w3[3 + (WY == 1 ? 1 : jj)] * w3[6 + (WZ == 1 ? 1 : kk)]);
-                    if constexpr (sizeof(T) == 8) {
-                        // FP64: the NH result columns in blocks of 4 on the 4-block
-                        // 4x4x4 form (16 cycles each): 3 blocks instead of one 16-column
-                        // 16x16x4 (64 cycles) at NF = 3.  Block b is particles
-                        // 16m + 4b .. +3; A[b][i][k] sits in lane 16k + 4b + i, which is
-                        // the same particle and group as the 16x16x4 operand above;
-                        // B[b][k][j] in lane 16k + 4b + j; D[b][i][j] in lane 16i + 4b + j.
-                        double accb[NCB];
+                            ayz[kk * WY + jj] = T(w3[3 + (WY == 1 ? 1 : jj)] * w3[6 + (WZ == 1 ? 1 : kk)]);
+                    // FP64: the NH result columns in blocks of 4 on the 4-block
+                    // 4x4x4 form (16 cycles each): 3 blocks instead of one 16-column
+                    // 16x16x4 (64 cycles) at NF = 3.  Block b is particles
+                    // 16m + 4b .. +3; A[b][i][k] sits in lane 16k + 4b + i, which is
+                    // the same particle and group as the 16x16x4 operand above;
+                    // B[b][k][j] in lane 16k + 4b + j; D[b][i][j] in lane 16i + 4b + j.
+                    double accb[NCB];
 #pragma unroll
-                        for (int cb = 0; cb < NCB; cb++) accb[cb] = 0.0;
+                    for (int cb = 0; cb < NCB; cb++) accb[cb] = 0.0;
 #pragma unroll
-                        for (int t = 0; t < NT; t++) {
-                            const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
-                            const T A = ax[ii] * ayz[kk * WY + jj];
+                    for (int t = 0; t < NT; t++) {
+                        const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
+                        const T A = ax[ii] * ayz[kk * WY + jj];
 #pragma unroll
-                            for (int cb = 0; cb < NCB; cb++)
-                                accb[cb] = __builtin_amdgcn_mfma_f64_4x4x4f64(A, Gt[box_of(t) * QG + cqb[cb]], accb[cb], 0, 0, 0);
-                        }
-                        const int pr = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4);
+                        for (int cb = 0; cb < NCB; cb++)
+                            accb[cb] = __builtin_amdgcn_mfma_f64_4x4x4f64(A, Gs[box_of(t) * QG + cqb[cb]], accb[cb], 0, 0, 0);
+                    }
+                    const int pr = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4);
 #pragma unroll
-                        for (int cb = 0; cb < NCB; cb++) {
-                            const int c = 4 * cb + (lane & 3);
-                            if (c < nh) Src[pr * NSR + c] = T(accb[cb]);
-                        }
-                    } else {
-                        typename MF::acc_t accg = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-                        for (int t = 0; t < NT; t++) {
-                            const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
-                            const T A = ax[ii] * ayz[kk * WY + jj];
-                            const T B = Gt[box_of(t) * QG + cq];
-                            accg = MF::step(A, B, accg);
-                        }
-                        if (c16 < nh) {
-#pragma unroll
-                            for (int r = 0; r < 4; r++) Src[(16 * m + MF::row(r, lane)) * NSR + c16] = accg[r];
-                        }
+                    for (int cb = 0; cb < NCB; cb++) {
+                        const int c = 4 * cb + (lane & 3);
+                        if (c < nh) Src[pr * NSR + c] = T(accb[cb]);
                     }
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
