@@ -365,6 +365,11 @@ template <typename T, int S, int AUX> constexpr int stage_mode()
 // 2-wave workgroups, 7 with single waves)
 template <int MODE, int AUX> constexpr int stage_waves_per_block() { return MODE == 2 ? 4 : (AUX != 0 ? 1 : 2); }
 
+// Columns of patches (k_stage); at 64^3 x 92, NF = 3, ms per step of the five
+// launches, FP32-bulk and FP64: plain order 13.77 / 22.2, 4 x 4 13.27 / 21.4, 4 x 8
+// 13.14 / 21.3, 8 x 8 13.14 / 21.4, 2 x 2 13.33 / 21.5, 4 x 4 rows taken whole 13.41 / 21.8.
+constexpr int kTileY = 4, kTileZ = 8;
+
 // S: 0 = deposit only (the step's result, or the initial state), 1..4 = RK
 // stage; AUX: also deposit the compute_dt auxiliaries (S = 0 or 3; 1 or 2 as
 // for aux_columns).
@@ -408,7 +413,24 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     // PM: the block's patch; otherwise this wave's patch of CPW cells, WPB consecutive per block
     const int patch = __builtin_amdgcn_readfirstlane(PM ? bgroup : bgroup * WPB + wave);
     if (patch >= npx * npy * npz) return; // uniform over the workgroup (PM) or the wave
-    const int bx = (patch % npx) * PT::PX, by = ((patch / npx) % npy) * PT::PY, bz = (patch / (npx * npy)) * PT::PZ;
+    // Patches are taken in columns of kTileY x kTileZ along x: the waves in flight on
+    // an XCD then hold neighbours in all three dimensions, so that what they
+    // exchange (stage 4's particles for a neighbour's lines, the deposits on
+    // shared cells, the neighbourhood fields) meets in its L2 and in the memory-side
+    // cache.  In plain x, y, z order the z neighbours are a plane apart and stage 4's
+    // lines were written to memory in parts.
+    int bx, by, bz;
+    {
+        const int slab = npx * npy * kTileZ, tz = patch / slab;
+        int r = patch - tz * slab;
+        const int hz = min(kTileZ, npz - tz * kTileZ), rows = npx * kTileY * hz, ty = r / rows;
+        r -= ty * rows;
+        const int hy = min(kTileY, npy - ty * kTileY), x = r / (hy * hz);
+        r -= x * hy * hz;
+        bx = x * PT::PX;
+        by = (ty * kTileY + r % hy) * PT::PY;
+        bz = (tz * kTileZ + r / hy) * PT::PZ;
+    }
     const int pw = PM ? wave : 0; // this wave's cell within the patch
     const int ox = pw % PT::PX, oy = (pw / PT::PX) % PT::PY, oz = pw / (PT::PX * PT::PY);
     const int cx = bx + ox, cy = by + oy, cz = bz + oz;
