@@ -256,29 +256,29 @@ __device__ __forceinline__ int move1(int from, double x, double plo, double dxi,
     return 0;
 }
 
-// Three ways to map waves to cells (MODE).
+// Ways to map waves to cells (MODE).
 //  0: every wave is its own patch of one cell (box = its 27 neighbours; two
 //     cells in FP32-bulk, below), stages its own box and flushes its deposit
 //     directly: no workgroup barrier.
-//  1: the WPB waves of a workgroup take a patch of WPB cells (2 along x, then
+//  2: the WPB waves of a workgroup take a patch of WPB cells (2 along x, then
 //     2 along y, when the stencil is 3 wide there, else along z); the patch's
 //     neighbourhood box (PX + WX - 1) x (PY + WY - 1) x (PZ + WZ - 1) is staged
-//     once for all of them (one barrier), and each wave flushes directly.
-//  2: as 1, and the deposits are also summed over the box in LDS before one
-//     set of global atomics (56% fewer for a 2 x 2 patch at the 3-D stencil),
-//     at the cost of two more barriers.
-// PM (a shared patch) is MODE >= 1.  In MODE 0 a wave may also take CPW = 2
+//     once for all of them, and the deposits are summed over the box in LDS
+//     before one set of global atomics (56% fewer for a 2 x 2 patch at the 3-D
+//     stencil).
+//  3: the WPB waves of a workgroup share one cell, 64 particles each in turn,
+//     with the box staged once and the deposits summed in LDS as in 2: for grids
+//     with too few cells to fill the chip and several chunks per cell.
+// PM (a shared patch) is MODE >= 2.  In MODE 0 a wave may also take CPW = 2
 // cells, x-adjacent, as one patch: their particles form one list of 16-particle
 // tiles (the first cell's, then the second's), so that a cell of 92 particles no
 // longer leaves 36 of a chunk's 64 lanes idle, and the wave stages the two
 // cells' 4 x 3 x 3 box once.
-template <int WX, int WY, int WZ, int WPB, bool PM, int CPW = 1> struct Patch {
-    static_assert(CPW == 1 || (CPW == 2 && !PM && WX == 3), "two cells per wave: MODE 0, along a 3-wide x");
-    static constexpr int PX = (PM || CPW == 2) && WX == 3 ? 2 : 1;
-    static constexpr int PY = PM && WY == 3 && WPB >= 2 * PX ? 2 : 1;
-    static constexpr int PZ = PM ? WPB / (PX * PY) : 1;
-    static constexpr int CELLS = PM ? WPB : CPW; // cells of one patch
-    static_assert(PX * PY * PZ == CELLS, "a patch holds one cell per wave, or the wave's CPW cells");
+template <int WX, int WY, int WZ, int CELLS> struct Patch {
+    static constexpr int PX = WX == 3 && CELLS >= 2 ? 2 : 1;
+    static constexpr int PY = WY == 3 && CELLS >= 2 * PX ? 2 : 1;
+    static constexpr int PZ = CELLS / (PX * PY);
+    static_assert(PX * PY * PZ == CELLS, "cells of one patch");
     static constexpr int NBX = PX + WX - 1, NBY = PY + WY - 1, NBZ = PZ + WZ - 1;
     static constexpr int NB = NBX * NBY * NBZ;
 };
@@ -315,13 +315,6 @@ template <int NF, typename T, int AUX> constexpr int stage_lds_doubles_per_wave(
     return 64 * 9 + 64 * stage_source_row<NF>(AUX) * (int)sizeof(T) / 8;
 }
 
-// LDS of the table of the neighbourhood box's cell indices (NB ints), in
-// doubles: one per workgroup (PM) or per wave.
-template <int WX, int WY, int WZ, int WPB, bool PM, int CPW> constexpr int stage_lds_ctab_doubles()
-{
-    return (Patch<WX, WY, WZ, WPB, PM, CPW>::NB + 1) / 2;
-}
-
 // cells per wave: two in FP32-bulk's independent-wave launches of the 3-D
 // stencil (its 4 x 3 x 3 box still fits three waves per SIMD in LDS; FP64's
 // would not fit two)
@@ -330,24 +323,26 @@ template <typename T, int WX, int MODE> constexpr int stage_cells_per_wave()
     return MODE == 0 && sizeof(T) == 4 && WX == 3 ? 2 : 1;
 }
 
-// LDS of a workgroup, in doubles.  The cell tables come first.  PM: then the
-// staged neighbourhood box (gather stages, NB x 4 NH values of T) and the
-// waves' regions; with the merge (MODE 2) the deposit's merge buffer (NB x
-// deposited columns, double) reuses that space once every wave is done with
-// it.  Without PM: per wave, its own box and its region.  The host sizes the
-// launch with this function.
+template <typename T, int WX, int WY, int WZ, int WPB, int MODE>
+using StagePatch = Patch<WX, WY, WZ, (MODE == 2 ? WPB : stage_cells_per_wave<T, WX, MODE>())>;
+
+// LDS of a workgroup, in doubles.  The tables of the box's cell indices (NB ints)
+// come first.  PM: then the staged neighbourhood box (gather stages, NB x 4 NH
+// values of T) and the waves' regions; the deposit's merge buffer (NB x deposited
+// columns, double) reuses that space once every wave is done with it.  Without
+// PM: per wave, its own box and its region.  The host sizes the launch with this
+// function.
 template <int NF, typename T, int WX, int WY, int WZ, int WPB, int S, int AUX, int MODE>
 constexpr int stage_lds_doubles_per_block()
 {
-    constexpr bool PM = MODE >= 1;
-    constexpr int CPW = stage_cells_per_wave<T, WX, MODE>();
+    constexpr bool PM = MODE >= 2;
     constexpr int nh = NF * NF;
-    constexpr int NB = Patch<WX, WY, WZ, WPB, PM, CPW>::NB;
-    constexpr int ct = (PM ? 1 : WPB) * stage_lds_ctab_doubles<WX, WY, WZ, WPB, PM, CPW>();
+    constexpr int NB = StagePatch<T, WX, WY, WZ, WPB, MODE>::NB;
+    constexpr int ct = (PM ? 1 : WPB) * ((NB + 1) / 2);
     constexpr int gsh = S == 0 ? 0 : (NB * 4 * nh * (int)sizeof(T) + 7) / 8;
     if (!PM) return ct + WPB * (gsh + stage_lds_doubles_per_wave<NF, T, AUX>());
     constexpr int work = gsh + WPB * stage_lds_doubles_per_wave<NF, T, AUX>();
-    constexpr int merge = MODE == 2 && S <= 3 ? NB * (4 * nh + aux_columns<NF>(AUX)) : 0;
+    constexpr int merge = S <= 3 ? NB * (4 * nh + aux_columns<NF>(AUX)) : 0;
     return ct + (work > merge ? work : merge);
 }
 
@@ -359,11 +354,11 @@ template <typename T, int S, int AUX> constexpr int stage_mode()
 {
     return S == 0 || (S == 4 && sizeof(T) == 4) ? 2 : 0;
 }
-// waves per workgroup: a patch of 4 (MODE 2); otherwise 2, or 1 for the launches
+// waves per workgroup: 4 (MODE 2 and 3); otherwise 2, or 1 for the launches
 // with the compute_dt auxiliaries, whose larger LDS rows would otherwise leave
 // a CU a whole 2-wave workgroup short (FP64 at 64^3 x 92: 6 waves per CU with
 // 2-wave workgroups, 7 with single waves)
-template <int MODE, int AUX> constexpr int stage_waves_per_block() { return MODE == 2 ? 4 : (AUX != 0 ? 1 : 2); }
+template <int MODE, int AUX> constexpr int stage_waves_per_block() { return MODE >= 2 ? 4 : (AUX != 0 ? 1 : 2); }
 
 // Columns of patches (k_stage); at 64^3 x 92, NF = 3, ms per step of the five
 // launches, FP32-bulk and FP64: plain order 13.77 / 22.2, 4 x 4 13.27 / 21.4, 4 x 8
@@ -376,8 +371,8 @@ constexpr int kTileY = 4, kTileZ = 8;
 template <int NF, typename T, int WX, int WY, int WZ, int WPB, int S, int AUX, int MODE>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2))) void k_stage(StageArgs<T> a)
 {
-    constexpr bool PM = MODE >= 1;    // the workgroup shares one patch and its staged box
-    constexpr bool MERGE = MODE == 2; // and merges its deposits in LDS
+    constexpr bool PM = MODE >= 2;    // the workgroup shares one patch and its staged box, and merges its deposits in LDS
+    constexpr bool SPLIT = MODE == 3; // the patch is one cell, whose chunks the waves take in turn
     constexpr int nh = NH<NF>;
     constexpr int QG = 4 * nh;
     constexpr int NT = WX * WY * WZ;        // target cells of a source cell
@@ -401,7 +396,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     constexpr int s = S;
     constexpr bool aux = AUX != 0;
     constexpr int CPW = stage_cells_per_wave<T, WX, MODE>();
-    using PT = Patch<WX, WY, WZ, WPB, PM, CPW>;
+    using PT = StagePatch<T, WX, WY, WZ, WPB, MODE>;
     constexpr int NB = PT::NB;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
@@ -431,7 +426,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         by = (ty * kTileY + r % hy) * PT::PY;
         bz = (tz * kTileZ + r / hy) * PT::PZ;
     }
-    const int pw = PM ? wave : 0; // this wave's cell within the patch
+    const int pw = PM && !SPLIT ? wave : 0; // this wave's cell within the patch
     const int ox = pw % PT::PX, oy = (pw / PT::PX) % PT::PY, oz = pw / (PT::PX * PT::PY);
     const int cx = bx + ox, cy = by + oy, cz = bz + oz;
     // a wave whose cell lies outside the domain (a partial patch) or holds no
@@ -469,19 +464,20 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     // set this wave's cells of the grid (and the auxiliaries) that a later launch
     // deposits into: the cells partition over the waves, so no fill launches are
     // needed between the stages
-    if (a.gclear && inside_domain) {
+    const bool owner = inside_domain && (!SPLIT || wave == 0); // of the cell's own values
+    if (a.gclear && owner) {
         const int n = (inside1 ? 2 : 1) * QG;
         double* gc = a.gclear + (int64_t)cell * QG;
         for (int e = lane; e < n; e += 64) gc[e] = e == 0 || e == QG ? a.m00 : 0.0;
     }
-    if (s == 2 && a.clear_aux && inside_domain) {
+    if (s == 2 && a.clear_aux && owner) {
         const int n = (inside1 ? 2 : 1) * NAUX;
         for (int e = lane; e < n; e += 64) a.aux[(int64_t)cell * NAUX + e] = 0.0;
     }
     if constexpr (s == 4) {
         // compute_dt's conservative bound (Evolve.cpp:40-56) of this wave's cell:
         // N_ii and Nbar_ii from the auxiliaries S_ii and M_ii
-        if (a.want_dt && inside_domain) {
+        if (a.want_dt && owner) {
             double v = 0.0;
             if (lane < NF) {
                 const double M = a.gin[(int64_t)cell * QG + herm_re_rt<NF>(lane)] - (lane == 0 ? a.m00 : 0.0);
@@ -511,7 +507,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     constexpr int per_wave = stage_lds_doubles_per_wave<NF, T, AUX>();
     static_assert(per_wave == 64 * 9 + 64 * NSR * (int)sizeof(T) / 8,
                   "LDS layout and its size function disagree");
-    constexpr int CT = stage_lds_ctab_doubles<WX, WY, WZ, WPB, PM, CPW>();
+    constexpr int CT = (NB + 1) / 2;
     // [NB] the box's cell indices: the block's, or this wave's
     int* ctab = (int*)(PM ? lds : lds + wave * CT);
     double* lw = lds + (PM ? CT : WPB * CT);
@@ -675,7 +671,12 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     // (one cell: the loop runs over the cell's run itself, base = beg + sbase)
     const int lo = CPW == 1 ? beg : 0, hi = CPW == 1 ? end : NSL;
     int running = 0; // stage 1: lane 27 i + e holds the count of move e from the wave's cell i so far
-    for (int base = lo; base < hi; base += 64) {
+    int seen = 0;    // (SPLIT: of the workgroup's finished rounds)
+    // SPLIT, stage 1: the waves stay together (their ranks follow from each other's
+    // counts), so a round runs for all of them; a wave past the end has no active lane
+    __shared__ int moves[SPLIT && s == 1 ? WPB * 27 : 1];
+    const int first = SPLIT ? 64 * wave : 0;
+    for (int base = lo + first; (SPLIT && s == 1 ? base - first : base) < hi; base += SPLIT ? 64 * WPB : 64) {
         const int sbase = base - lo;
         int64_t ip;
         bool act;
@@ -951,6 +952,22 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
                         if (lane == q) running += __popcll(msk);
                         left &= ~msk;
                     }
+                    if constexpr (SPLIT) {
+                        // `running` holds this chunk's counts alone: add those of the
+                        // earlier rounds (in `seen`) and of the earlier waves
+                        if (lane < 27) moves[27 * wave + lane] = running;
+                        __syncthreads();
+                        int before = seen;
+                        if (lane < 27)
+                            for (int w2 = 0; w2 < WPB; w2++) {
+                                const int m = moves[27 * w2 + lane];
+                                if (w2 < wave) before += m;
+                                seen += m;
+                            }
+                        running = 0;
+                        myrank += __shfl(before, e & 31);
+                        __syncthreads();
+                    }
                     if (act) {
                         a.rank[ip] = myrank;
                         a.mv[ip] = (unsigned char)(e >= 27 ? e - 27 : e);
@@ -1097,10 +1114,10 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     if constexpr (s == 1) {
-        if (inside_domain && lane < (inside1 ? 54 : 27)) a.mcount[(int64_t)cell * 27 + lane] = running;
+        if (owner && lane < (inside1 ? 54 : 27)) a.mcount[(int64_t)cell * 27 + lane] = SPLIT ? seen : running;
     }
     if (!deposits) return;
-    if constexpr (!MERGE) {
+    if constexpr (!PM) {
         // ---- flush this wave's (last) cell's deposit straight to the grid
         if constexpr (CPW == 2) {
             if (n1 > 0) flush_direct(1);

@@ -517,6 +517,7 @@ struct emu_state {
     // layout: np + ncell (align - 1).
     int align = 1;
     int64_t cap = 1;
+    bool split = false; // several waves per cell (k_stage's MODE 3)
     // persistent arrays, two copies for the sort
     void* block[2] = {nullptr, nullptr};
     // scratch
@@ -566,6 +567,26 @@ namespace {
 // Up to here the plan's two small launches cost less in line than the event
 // pairs and the second stream that hide them.
 constexpr int64_t kInlinePlanCells = 32768;
+
+// Whether four waves share a cell (k_stage's MODE 3): where the cells hold more
+// than one chunk of 64 particles each and are too few to fill the chip one (or,
+// in FP32-bulk, half) a wave.  By LDS the chip holds about 1024 such workgroups
+// in FP32-bulk and 768 in FP64 at once; up to twice that they still pay where a
+// wave alone would walk 3 chunks or more.  us per step, one wave / four waves per
+// cell, NF = 3:
+//   FP32-bulk  4^3 cells  x 92: 126 / 70    x 378: 367 / 103
+//              8^3        x 92: 141 / 94    x 378: 395 / 159
+//              1024 (1-D) x 92:  80 / 70    x 378: 196 / 143
+//              12^3       x 92: 201 / 216   x 200: 352 / 245
+//              16^3       x 92: 281 / 387   x 378: 819 / 822
+//   FP64       8^3        x 92: 132 / 113   x 378: 329 / 211
+//              1024 (1-D) x 92:  97 / 110   x 200: 164 / 140
+//              12^3       x 92: 204 / 309   x 378: 563 / 634
+bool split_cells(int64_t np, int64_t ncell, int precision)
+{
+    const int64_t at_once = precision == EMU_FP32_BULK ? 1024 : 768;
+    return (ncell <= at_once && np > 64 * ncell) || (ncell <= 2 * at_once && np > 160 * ncell);
+}
 
 template <typename T> Arrays<T> arrays_of(emu_state* st, int copy)
 {
@@ -617,21 +638,26 @@ int scan_counts(emu_state* st, const int* in, int* out, hipStream_t s = nullptr)
 }
 
 
-template <int NF, typename T, int WX, int WY, int WZ, int S, int AUX>
-void launch_stage_k(emu_state* st, StageArgs<T>& a)
+template <int NF, typename T, int WX, int WY, int WZ, int S, int AUX, int MODE>
+void launch_stage_mode(emu_state* st, StageArgs<T>& a)
 {
-    constexpr int MODE = stage_mode<T, S, AUX>();
-    constexpr bool PM = MODE >= 1;
     constexpr int WPB = stage_waves_per_block<MODE, AUX>(); // waves per workgroup
-    using PT = Patch<WX, WY, WZ, WPB, PM, stage_cells_per_wave<T, WX, MODE>()>;
+    using PT = StagePatch<T, WX, WY, WZ, WPB, MODE>;
     const Geom& g = st->ctx->g;
     const int64_t npatch = (int64_t)((g.n[0] + PT::PX - 1) / PT::PX) * ((g.n[1] + PT::PY - 1) / PT::PY) *
                            ((g.n[2] + PT::PZ - 1) / PT::PZ);
-    const int64_t nblk = PM ? npatch : (npatch + WPB - 1) / WPB;
+    const int64_t nblk = MODE >= 2 ? npatch : (npatch + WPB - 1) / WPB;
     a.blocks_per_xcd = (int)((nblk + 7) / 8);
     const size_t lds = (size_t)stage_lds_doubles_per_block<NF, T, WX, WY, WZ, WPB, S, AUX, MODE>() * sizeof(double);
     hipLaunchKernelGGL((k_stage<NF, T, WX, WY, WZ, WPB, S, AUX, MODE>), dim3((unsigned)(8 * a.blocks_per_xcd)),
                        dim3(64 * WPB), lds, st->ctx->stream, a);
+}
+
+template <int NF, typename T, int WX, int WY, int WZ, int S, int AUX>
+void launch_stage_k(emu_state* st, StageArgs<T>& a)
+{
+    if (st->split) launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, 3>(st, a);
+    else launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, stage_mode<T, S, AUX>()>(st, a);
 }
 
 template <int NF, typename T, int WX, int WY, int WZ>
@@ -824,6 +850,7 @@ extern "C" int emu_state_create(emu_ctx* ctx, int64_t np, int precision, emu_sta
     if (np == 0 || np + st->ncell * (a128 - 1) > (int64_t)INT32_MAX) aligned = false;
     st->align = aligned ? a128 : 1;
     st->cap = std::max<int64_t>(np + st->ncell * (st->align - 1), 1);
+    st->split = split_cells(np, st->ncell, precision);
     const int64_t npa = st->cap;
     const size_t pb = persistent_bytes(npa, st->nh, st->tsize);
     bool ok = hipMalloc(&st->block[0], pb) == hipSuccess && hipMalloc(&st->block[1], pb) == hipSuccess &&
