@@ -7,12 +7,9 @@
 //
 // Gather (MFMA): with s(p) = (1, -vx, -vy, -vz) and G_g(t, c) the four field
 // groups (M, Phix, Phiy, Phiz) of neighbour t,
-//   inside_c(p) = sum_t sum_g [w_t(p) s_g(p)] G_g(t, c),
-// a (16 particles x 4*27) x (4*27 x NH) product per tile of 16 particles: one
-// 16x16x4 step per neighbour t, its K = 4 slice being the four groups.  The
-// cell's 27 x 4 NH neighbour fields are staged in LDS once per cell with
-// coalesced loads and feed the B operand; A is the particle's weight times
-// s_g, read from the shape factors staged in LDS.
+//   inside_c(p) = sum_g s_g(p) sum_t w_t(p) G_g(t, c),
+// the sum over t a product of the cell's 27 x 4 NH neighbour fields, staged in
+// LDS once per cell with coalesced loads, and the particles' weights (WaveGather).
 // Deposit (MFMA): the contribution of the cell's particles p to target cell t
 // and field column q is D[t][q] = sum_p W[p][t] R[p][q], with W the shape
 // weights and R = (1, vx, vy, vz) x q_c(p), q = N f - conj(Nbar fbar).  Over a
@@ -32,6 +29,24 @@ typedef float mf_f4 __attribute__((ext_vector_type(4)));
 
 // Transpose of a 4 x 4 block of 16-lane rows: row i of register k <-> row k of
 // register i.
+__device__ __forceinline__ void transpose_rows(unsigned& a, unsigned& b, unsigned& c, unsigned& d)
+{
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    auto swap32 = [](unsigned& x, unsigned& y) __attribute__((always_inline)) { // upper half of x <-> lower half of y
+        const u2 r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        x = r[0];
+        y = r[1];
+    };
+    auto swap16 = [](unsigned& x, unsigned& y) __attribute__((always_inline)) { // odd rows of x <-> even rows of y
+        const u2 r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        x = r[0];
+        y = r[1];
+    };
+    swap32(a, c);
+    swap32(b, d);
+    swap16(a, b);
+    swap16(c, d);
+}
 __device__ __forceinline__ void transpose_rows(float& a, float& b, float& c, float& d)
 {
     typedef unsigned u2 __attribute__((ext_vector_type(2)));
@@ -50,6 +65,136 @@ __device__ __forceinline__ void transpose_rows(float& a, float& b, float& c, flo
     swap16(a, b);
     swap16(c, d);
 }
+__device__ __forceinline__ void transpose_rows(double& a, double& b, double& c, double& d)
+{
+    double* v[4] = {&a, &b, &c, &d};
+    unsigned lo[4], hi[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const unsigned long long u = (unsigned long long)__double_as_longlong(*v[i]);
+        lo[i] = (unsigned)u;
+        hi[i] = (unsigned)(u >> 32);
+    }
+    transpose_rows(lo[0], lo[1], lo[2], lo[3]);
+    transpose_rows(hi[0], hi[1], hi[2], hi[3]);
+#pragma unroll
+    for (int i = 0; i < 4; i++) *v[i] = __longlong_as_double((long long)(((unsigned long long)hi[i] << 32) | lo[i]));
+}
+
+template <typename T> struct Mfma16x16x4;
+template <> struct Mfma16x16x4<double> {
+    typedef mf_d4 acc_t;
+    static __device__ __forceinline__ acc_t step(double a, double b, acc_t c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    // the group and the component (of 4) of row i of A, such that element g of a
+    // lane of the result is group g: element r of lane l holds row 4r + l/16
+    static __device__ __forceinline__ int group(int i) { return i >> 2; }
+    static __device__ __forceinline__ int comp(int i) { return i & 3; }
+};
+template <> struct Mfma16x16x4<float> {
+    typedef mf_f4 acc_t;
+    static __device__ __forceinline__ acc_t step(float a, float b, acc_t c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    // element r of lane l holds row 4 (l/16) + r
+    static __device__ __forceinline__ int group(int i) { return i & 3; }
+    static __device__ __forceinline__ int comp(int i) { return i >> 2; }
+};
+
+// The gather of a wave's chunk of up to 64 particles on the matrix cores:
+//   out_c(p) = sum_t w_t(p) (G_0c(t) + s v_1(p) G_1c(t) + s v_2(p) G_2c(t) + s v_3(p) G_3c(t)),
+// s = SIGN, t the WX x WY x WZ neighbours, rows of 4 NH fields in LDS.  Per tile of 16
+// particles the product is G^T W: A's rows are 4 components x the 4 field groups,
+// K the neighbours (4 per step), B's columns the particles, so that a lane's four
+// results are the four groups of one component of one particle, and contracting
+// them with v is 3 FMAs in the lane: ceil(27 / 4) = 7 steps per 4 components.  (A
+// tile of 16 particles by NH of 16 columns with the groups as K takes 27 steps
+// for any NH.)  The particle's own lane forms its 27 weights once; a transpose of
+// 16-lane rows turns four of them into the operands of all four tiles, and
+// another returns the results, without LDS.
+template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false> struct WaveGather {
+    using MF = Mfma16x16x4<T>;
+    static constexpr int nh = NH<NF>, NT = WX * WY * WZ, KK = (NT + 3) / 4, MG = (nh + 3) / 4;
+    // this lane's entry of A at step k, row i = l%16, neighbour t = 4k + l/16 (past
+    // the last one: any in-range entry, its weight is zero; rows past NH feed
+    // results that are dropped)
+    unsigned goff[PACK ? (KK + 1) / 2 : KK]; // PACK: two 16-bit offsets each, taken apart once per chunk
+
+    // row(t): offset of neighbour t's row of fields
+    template <typename F> __device__ __forceinline__ void init(int lane, F&& row)
+    {
+#pragma unroll
+        for (int k = 0; k < KK; k++) {
+            const int t = 4 * k + (lane >> 4);
+            const unsigned o = row(t < NT ? t : NT - 1) + MF::group(lane & 15) * nh + MF::comp(lane & 15);
+            if (PACK) goff[k / 2] = k % 2 ? goff[k / 2] | o << 16 : o;
+            else goff[k] = o;
+        }
+    }
+
+    // wd: the particle's shape factors; rows(m): the fields of tile m's cell; vel(m):
+    // v of particle 16 m + l%16, by pointer; ntile: tiles with particles
+    template <int SIGN, typename F, typename V>
+    __device__ __forceinline__ void run(const double wd[3][3], int ntile, F&& rows, V&& vel, T* out)
+    {
+        int off[KK];
+#pragma unroll
+        for (int k = 0; k < KK; k++) {
+            if (PACK && k % 2 == 0) asm volatile("" : "+v"(goff[k / 2]));
+            off[k] = !PACK ? goff[k] : (k % 2 ? goff[k / 2] >> 16 : goff[k / 2] & 0xffffu);
+        }
+        T w[4 * KK];
+        {
+            T fx[3], fyz[3][3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) fx[i] = T(wd[0][i]);
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) fyz[k][j] = T(wd[1][j]) * T(wd[2][k]);
+#pragma unroll
+            for (int t = 0; t < 4 * KK; t++) {
+                const int i = WX == 1 ? 1 : t % WX, j = WY == 1 ? 1 : (t / WX) % WY, k = WZ == 1 ? 1 : (t / (WX * WY)) % 3;
+                w[t] = t < NT ? fx[i] * fyz[k][j] : T(0);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < KK; k++) transpose_rows(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+        // w[4 k + m] now holds tile m's operand of step k
+        T res[MG][4];
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+#pragma unroll
+            for (int c = 0; c < MG; c++) res[c][m] = T(0);
+            if (m < ntile) {
+                const T* G = rows(m);
+                T v0, v1, v2;
+                vel(m, v0, v1, v2);
+                typename MF::acc_t acc[MG];
+#pragma unroll
+                for (int c = 0; c < MG; c++) acc[c] = typename MF::acc_t{T(0), T(0), T(0), T(0)};
+#pragma unroll
+                for (int k = 0; k < KK; k++)
+#pragma unroll
+                    for (int c = 0; c < MG; c++) acc[c] = MF::step(G[off[k] + 4 * c], w[4 * k + m], acc[c]);
+#pragma unroll
+                for (int c = 0; c < MG; c++)
+                    res[c][m] = SIGN < 0 ? acc[c][0] - v0 * acc[c][1] - v1 * acc[c][2] - v2 * acc[c][3]
+                                         : acc[c][0] + v0 * acc[c][1] + v1 * acc[c][2] + v2 * acc[c][3];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < MG; c++) {
+            transpose_rows(res[c][0], res[c][1], res[c][2], res[c][3]);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (4 * c + j < nh) out[4 * c + j] = res[c][j];
+        }
+    }
+};
 
 template <typename T> struct PArrays {
     double* pos[3];
@@ -457,7 +602,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     };
     // box index of this wave's stencil target t (of its first cell; the second
     // cell's is one further along x)
-    auto box_of = [&](int t) -> int {
+    auto box_of = [&](int t) __attribute__((always_inline)) -> int {
         const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
         return ((oz + kk) * PT::NBY + (oy + jj)) * PT::NBX + (ox + ii);
     };
@@ -564,27 +709,29 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     // only on row t of A and column q only on column q of B, so the padding
     // rows (t >= NT) and columns (q >= QGA), which are never flushed, read any
     // in-range entries instead of being masked.
+    // PACK: in three registers, taken apart once per chunk.  It pays where the
+    // twelve crowd the commutators out into scratch memory (FP32-bulk's NF = 3
+    // launch with the auxiliaries, 3.33 -> 3.21 ms at 64^3 x 92) or cost a wave per
+    // SIMD (its stage 4; FP64's NF = 2 launch with the auxiliaries, 36 -> 33 us at
+    // 16^3 x 26); elsewhere the unpacking costs 2 to 4%.
+    constexpr bool PACK = sizeof(T) == 4 ? NF == 3 && (AUX != 0 || s == 4) : NF == 2 && AUX != 0 && s != 0;
+    unsigned ptdx = 0, pb1 = 0, pb2 = 0; // 4 bits a shape factor, 8 bits a source
     int tdx[MT][3];
+    static_assert(3 * MT <= 8, "eight packed factors");
 #pragma unroll
     for (int m = 0; m < MT; m++) {
         const int t = 16 * m + (lane & 15);
         const int tc = t < NT ? t : NT - 1;
         const int ii = tc % WX, jj = (tc / WX) % WY, kk = tc / (WX * WY);
-        tdx[m][0] = WX == 1 ? 1 : ii;
-        tdx[m][1] = 3 + (WY == 1 ? 1 : jj);
-        tdx[m][2] = 6 + (WZ == 1 ? 1 : kk);
-    }
-    // FP32-bulk's gather: this lane's entry of A at step k, row i = l%16 (group
-    // i%4, component i/4 of the step's four), neighbour t = 4k + l/16 (past the
-    // last one: any in-range entry, its weight is zero; rows past NH feed results
-    // that are dropped)
-    constexpr int KG = sizeof(T) == 4 && s != 0 ? (NT + 3) / 4 : 1;
-    int goff[KG];
+        const int f[3] = {WX == 1 ? 1 : ii, 3 + (WY == 1 ? 1 : jj), 6 + (WZ == 1 ? 1 : kk)};
 #pragma unroll
-    for (int k = 0; k < KG; k++) {
-        const int t = 4 * k + (lane >> 4);
-        goff[k] = box_of(t < NT ? t : NT - 1) * QG + (lane & 3) * nh + ((lane & 15) >> 2);
+        for (int d = 0; d < 3; d++) {
+            tdx[m][d] = f[d];
+            ptdx |= (unsigned)f[d] << (4 * (3 * m + d));
+        }
     }
+    WaveGather<NF, T, WX, WY, WZ, PACK> gather;
+    if constexpr (s != 0) gather.init(lane, [&](int t) __attribute__((always_inline)) { return box_of(t) * QG; });
     // The last columns, when at most 8 remain past the 16-column tiles (NF = 3:
     // 36 = 2 x 16 + 4 without the auxiliaries, 39 = 2 x 16 + 7 with the
     // diagonal ones), run as 4-column tiles on the 4-block 4x4x4 form instead:
@@ -598,22 +745,25 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     constexpr int NSM = SMALL ? (QREM + 3) / 4 : 0;               // 4-column tiles
     constexpr int NCG = NTF + NSM;                                // column groups of the B operand
     static_assert(NTL == NTF + (SMALL ? 1 : 0), "column tiles");
+    static_assert(NCG <= 4, "four packed columns");
     int bi1[NCG], bi2[NCG];
 #pragma unroll
     for (int n = 0; n < NCG; n++) {
+        int b1 = nh + 3, b2 = nh + 3;
         const int q = n >= NTF ? 16 * NTF + 4 * (n - NTF) + (lane & 3) : 16 * n + (lane & 15);
         if (q < QG) {
             const int f = q / nh, c = q % nh;
-            bi1[n] = c;
-            bi2[n] = f == 0 ? nh + 3 : nh + f - 1;
+            b1 = c;
+            b2 = f == 0 ? nh + 3 : nh + f - 1;
         } else if (aux && q < QGA) {
             const int x = q - QG;
-            bi1[n] = NSRC + (x < NF ? x : NF + (x - NF) / 3);
-            bi2[n] = x < NF ? nh + 3 : nh + (x - NF) % 3;
-        } else {
-            bi1[n] = nh + 3;
-            bi2[n] = nh + 3;
+            b1 = NSRC + (x < NF ? x : NF + (x - NF) / 3);
+            b2 = x < NF ? nh + 3 : nh + (x - NF) % 3;
         }
+        bi1[n] = b1;
+        bi2[n] = b2;
+        pb1 |= (unsigned)b1 << (8 * n);
+        pb2 |= (unsigned)b2 << (8 * n);
     }
     mf_d4 acc[MT][NTF];
     double accs[MT][NSM > 0 ? NSM : 1]; // the 4x4x4 tiles
@@ -733,129 +883,16 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
             // ---- gather on the matrix cores, 16 particles per tile
             T inside[nh];
             const int ntile = CPW == 1 ? (min(64, end - base) + 15) >> 4 : min(4, (NSL + 15 - sbase) >> 4);
-            if constexpr (sizeof(T) == 4) {
-                // FP32-bulk: per tile of 16 particles the product is G^T W.  A's rows
-                // are 4 components x the 4 field groups, K the neighbours (4 per
-                // step), B's columns the particles, so that a lane's four results are
-                // the four groups of one component of one particle, and contracting
-                // them with s is 3 FMAs in the lane: 7 steps per 4 components
-                // (ceil(27 / 4)) instead of 27 steps whose 16 columns hold NH.
-                // The particle's own lane forms its 27 weights once; a transpose of
-                // 16-lane rows turns four of them into the operands of all four
-                // tiles, and another returns the results, without LDS.
-                constexpr int KK = (NT + 3) / 4, MG = (nh + 3) / 4;
-                const int c16 = lane & 15;
-                T w[4 * KK];
-                {
-                    T fx[3], fyz[3][3];
-#pragma unroll
-                    for (int ii = 0; ii < 3; ii++) fx[ii] = T(wd[0][ii]);
-#pragma unroll
-                    for (int kk = 0; kk < 3; kk++)
-#pragma unroll
-                        for (int jj = 0; jj < 3; jj++) fyz[kk][jj] = T(wd[1][jj]) * T(wd[2][kk]);
-#pragma unroll
-                    for (int t = 0; t < 4 * KK; t++) {
-                        const int ii = WX == 1 ? 1 : t % WX, jj = WY == 1 ? 1 : (t / WX) % WY,
-                                  kk = WZ == 1 ? 1 : (t / (WX * WY)) % 3;
-                        w[t] = t < NT ? fx[ii] * fyz[kk][jj] : T(0);
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < KK; k++) transpose_rows(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
-                // w[4 k + m] now holds tile m's operand of step k
-                T res[4 * MG][4];
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-#pragma unroll
-                    for (int c = 0; c < MG; c++) res[c][m] = T(0);
-                    if (m < ntile) {
-                        // the tile's cell's neighbourhood: the second cell's box is one
-                        // column further along x (box rows of QG values)
-                        const T* Gt = Gs + (CPW == 2 && (sbase >> 4) + m >= T0 ? QG : 0);
-                        const T* vp = Src + (16 * m + c16) * NSR + nh;
-                        const T v0 = vp[0], v1 = vp[1], v2 = vp[2];
-                        mf_f4 acc_g[MG];
-#pragma unroll
-                        for (int c = 0; c < MG; c++) acc_g[c] = mf_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int k = 0; k < KK; k++)
-#pragma unroll
-                            for (int c = 0; c < MG; c++)
-                                acc_g[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(Gt[goff[k] + 4 * c], w[4 * k + m],
-                                                                                acc_g[c], 0, 0, 0);
-#pragma unroll
-                        for (int c = 0; c < MG; c++)
-                            res[c][m] = acc_g[c][0] - v0 * acc_g[c][1] - v1 * acc_g[c][2] - v2 * acc_g[c][3];
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < MG; c++) {
-                    transpose_rows(res[c][0], res[c][1], res[c][2], res[c][3]);
-#pragma unroll
-                    for (int j = 0; j < 4; j++)
-                        if (4 * c + j < nh) inside[4 * c + j] = res[c][j];
-                }
-            } else {
-                const int g4 = lane >> 4, c16 = lane & 15;
-                // B columns past NH only feed result columns that are dropped, so
-                // every lane reads an in-range entry, unmasked
-                const int cq = g4 * nh + (c16 < nh ? c16 : nh - 1);
-                constexpr int NCB = (nh + 3) / 4; // 4-column blocks (FP64 form)
-                int cqb[NCB];
-#pragma unroll
-                for (int cb = 0; cb < NCB; cb++) {
-                    const int c = 4 * cb + (lane & 3);
-                    cqb[cb] = g4 * nh + (c < nh ? c : nh - 1);
-                }
-#pragma unroll 1
-                for (int m = 0; m < ntile; m++) {
-                    const int p = 16 * m + c16; // the particle of this lane's A rows
-                    double w3[9];
-#pragma unroll
-                    for (int e = 0; e < 9; e++) w3[e] = Wf[p * 9 + e];
-                    const T* vp = Src + p * NSR + nh;
-                    const T v0 = vp[0], v1 = vp[1], v2 = vp[2];
-                    const T sg = g4 == 0 ? T(1) : (g4 == 1 ? -v0 : (g4 == 2 ? -v1 : -v2));
-                    // A = (w_x s_g) (w_y w_z): 3 + WY WZ products, then one per target
-                    T ax[WX], ayz[WY * WZ];
-#pragma unroll
-                    for (int ii = 0; ii < WX; ii++) ax[ii] = T(w3[WX == 1 ? 1 : ii]) * sg;
-#pragma unroll
-                    for (int kk = 0; kk < WZ; kk++)
-#pragma unroll
-                        for (int jj = 0; jj < WY; jj++)
-                            ayz[kk * WY + jj] = T(w3[3 + (WY == 1 ? 1 : jj)] * w3[6 + (WZ == 1 ? 1 : kk)]);
-                    // FP64: the NH result columns in blocks of 4 on the 4-block
-                    // 4x4x4 form (16 cycles each): 3 blocks instead of one 16-column
-                    // 16x16x4 (64 cycles) at NF = 3.  Block b is particles
-                    // 16m + 4b .. +3; A[b][i][k] sits in lane 16k + 4b + i, which is
-                    // the same particle and group as the 16x16x4 operand above;
-                    // B[b][k][j] in lane 16k + 4b + j; D[b][i][j] in lane 16i + 4b + j.
-                    double accb[NCB];
-#pragma unroll
-                    for (int cb = 0; cb < NCB; cb++) accb[cb] = 0.0;
-#pragma unroll
-                    for (int t = 0; t < NT; t++) {
-                        const int ii = t % WX, jj = (t / WX) % WY, kk = t / (WX * WY);
-                        const T A = ax[ii] * ayz[kk * WY + jj];
-#pragma unroll
-                        for (int cb = 0; cb < NCB; cb++)
-                            accb[cb] = __builtin_amdgcn_mfma_f64_4x4x4f64(A, Gs[box_of(t) * QG + cqb[cb]], accb[cb], 0, 0, 0);
-                    }
-                    const int pr = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4);
-#pragma unroll
-                    for (int cb = 0; cb < NCB; cb++) {
-                        const int c = 4 * cb + (lane & 3);
-                        if (c < nh) Src[pr * NSR + c] = T(accb[cb]);
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-                for (int c = 0; c < nh; c++) inside[c] = Src[lane * NSR + c];
-            }
+            gather.template run<-1>(
+                wd, ntile,
+                // the tile's cell's neighbourhood: the second cell's box is one column
+                // further along x (box rows of QG values)
+                [&](int m) __attribute__((always_inline)) { return Gs + (CPW == 2 && (sbase >> 4) + m >= T0 ? QG : 0); },
+                [&](int m, T& v0, T& v1, T& v2) __attribute__((always_inline)) {
+                    const T* vp = Src + (16 * m + (lane & 15)) * NSR + nh;
+                    v0 = vp[0], v1 = vp[1], v2 = vp[2];
+                },
+                inside);
             // ---- the RK registers this stage reads, as one batch of loads whose
             // latency the Hamiltonian and commutator arithmetic covers
             T yn[2 * nh], ao[2 * nh];
@@ -1056,17 +1093,18 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
         const int kb = CPW == 2 && n0 > 0 && sbase < n0 && n0 <= sbase + 64 ? (16 * T0 - sbase) / (4 * KU) : -1;
         lds_d wa[MT][3];
         lds_t sb[NCG][2];
+        if (PACK) asm volatile("" : "+v"(ptdx), "+v"(pb1), "+v"(pb2)); // taken apart here, not before the loop
 #pragma unroll
         for (int m = 0; m < MT; m++)
 #pragma unroll
             for (int d = 0; d < 3; d++) {
-                wa[m][d] = (lds_d)(Wf + (lane >> 4) * 9 + tdx[m][d]);
+                wa[m][d] = (lds_d)(Wf + (lane >> 4) * 9 + (PACK ? (int)((ptdx >> (4 * (3 * m + d))) & 15u) : tdx[m][d]));
                 asm volatile("" : "+v"(wa[m][d]));
             }
 #pragma unroll
         for (int n = 0; n < NCG; n++) {
-            sb[n][0] = (lds_t)(Src + (lane >> 4) * NSR + bi1[n]);
-            sb[n][1] = (lds_t)(Src + (lane >> 4) * NSR + bi2[n]);
+            sb[n][0] = (lds_t)(Src + (lane >> 4) * NSR + (PACK ? (int)((pb1 >> (8 * n)) & 255u) : bi1[n]));
+            sb[n][1] = (lds_t)(Src + (lane >> 4) * NSR + (PACK ? (int)((pb2 >> (8 * n)) & 255u) : bi2[n]));
             asm volatile("" : "+v"(sb[n][0]));
             asm volatile("" : "+v"(sb[n][1]));
         }
