@@ -5,7 +5,8 @@
 // take one particle per thread with its own stencil; the deposits sum over
 // the particles that share a stencil on the matrix cores first
 // (k_cell_deposit), then add to the grid with FP64 atomics.  All arrays are
-// SoA: [component][np].
+// SoA: [component][np].  The step calls run one wave per cell instead, gather
+// and deposit both on the matrix cores.
 //
 // Forward RHS for stage state Y (positions frozen within the step):
 //   q_p  = N_p f_p - conj(Nbar_p fbar_p)                    (per particle)
@@ -406,23 +407,66 @@ __global__ void k_renorm_soa(int64_t np, double* Y, const double* Ll, double max
 // ---------------------------------------------------------------------------
 // Step-level kernels: one launch per RK4 stage after that stage's deposit.
 // The stage algebra is step()'s (AMReX RK4 with the reference's saxpys,
-// FlavoredNeutrinoContainer.H:39-46), each a x + y rounded as written.
+// FlavoredNeutrinoContainer.H:39-46), each a x + y rounded as written but for
+// the accumulator's first two sums (k_fwd_stage).
 //
 // They take one cell per wave (the cell list's runs): every particle of the
-// wave has its stencil in the cell's 27-cell neighbourhood, so the grid rows
-// are the same for all lanes and are read as scalar loads, one neighbour at
-// a time, while each lane forms its own weights.
+// wave has its stencil in the cell's 27-cell neighbourhood, whose rows of
+// fields the wave stages in LDS once (CellBox) and gathers from on the matrix
+// cores (WaveGather).
 // ---------------------------------------------------------------------------
 constexpr int kCellWaves = 4; // waves (cells) per workgroup
 
 // The wave's cell, in an XCD-aware order (consecutive cells share an XCD's
 // L2); -1 past the last cell.
-__device__ __forceinline__ int wave_cell(int64_t ncell, int blocks_per_xcd)
+template <int WAVES = kCellWaves> __device__ __forceinline__ int wave_cell(int64_t ncell, int blocks_per_xcd)
 {
     const int b = blockIdx.x;
-    const int64_t c = ((int64_t)(b & 7) * blocks_per_xcd + (b >> 3)) * kCellWaves + (threadIdx.x >> 6);
+    const int64_t c = ((int64_t)(b & 7) * blocks_per_xcd + (b >> 3)) * WAVES + (threadIdx.x >> 6);
     return c < ncell ? __builtin_amdgcn_readfirstlane((int)c) : -1;
 }
+
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A wave's copy of its cell's neighbourhood in LDS: 27 rows of 4 NH fields in T
+// (the FP32 form rounds the FP64 grid here), then a row of zeros that the gather's
+// last step reads with zero weights.  In a dimension of shape order 0 the weights
+// are (0, 1, 0), so the other rows do not count.
+// The gather read the grid through scalar loads before (one neighbour's fields at a
+// time, every lane the same ones), a chain of 27 loads per chunk with nothing else
+// for the wave to do: on 32^3 cells x 92 particles, 2 flavours in FP64, a stage took
+// 398 us and a reverse boundary 715 us, now 284 and 590.
+template <int NF, typename T> struct CellBox {
+    static constexpr int QG = 4 * NH<NF>, N = 28 * QG;
+    using Gather = WaveGather<NF, T, 3, 3, 3, false, QG>;
+
+    // index of the neighbours' cells, for lanes 0..26 of the wave
+    static __device__ __forceinline__ void table(const Geom& g, int cell, int lane, int* ctab)
+    {
+        if (lane < 27) {
+            auto wrap = [](int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); };
+            const int x = wrap(cell % g.n[0] + lane % 3 - 1, g.n[0]);
+            const int y = wrap((cell / g.n[0]) % g.n[1] + (lane / 3) % 3 - 1, g.n[1]);
+            const int z = wrap(cell / (g.n[0] * g.n[1]) + lane / 9 - 1, g.n[2]);
+            ctab[lane] = (z * g.n[1] + y) * g.n[0] + x;
+        }
+    }
+    // (after table and a wave_sync; followed by a wave_sync)
+    static __device__ __forceinline__ void stage(const double* grid, const int* ctab, int lane, T* box)
+    {
+#pragma unroll
+        for (int e0 = 0; e0 < N; e0 += 64) {
+            const int e = e0 + lane;
+            if (e < 27 * QG) box[e] = T(grid[(int64_t)ctab[e / QG] * QG + e % QG]);
+            else if (e < N) box[e] = T(0);
+        }
+    }
+};
 
 // The deposit of both directions with the sum over particles on the matrix
 // cores.  KIND 0: the forward q_c = N f_c - conj(Nbar fbar_c) with (1, v);
@@ -595,95 +639,6 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_cell_deposit(AdjInT<T> in, 
 }
 
 
-// out[c] += sum over the neighbourhood of `cell` (wave-uniform) of
-// w_t (G_t[0][c] + s0 G_t[1][c] + s1 G_t[2][c] + s2 G_t[3][c]), with the
-// particle's shape factors w (shape3's windows) and multipliers s.
-template <int NF, typename T>
-__device__ __forceinline__ void gather_cell_box(const Geom& g, int cell, const T* grid_, const T w[3][3], const T s[3],
-                                                T* out)
-{
-    constexpr int nh = NH<NF>, QG = 4 * nh;
-    typedef __attribute__((address_space(4))) const T* cdp;
-    const cdp grid = (cdp)grid_;
-    // the neighbourhood's indices are wave-uniform: kept in scalar registers so
-    // that the grid rows below are scalar loads (vector loads of one address
-    // would return 64 copies of each row through the vector memory path)
-    const int cx = __builtin_amdgcn_readfirstlane(cell % g.n[0]);
-    const int cy = __builtin_amdgcn_readfirstlane((cell / g.n[0]) % g.n[1]);
-    const int cz = __builtin_amdgcn_readfirstlane(cell / (g.n[0] * g.n[1]));
-    auto wrap = [](int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); };
-    int lo[3], hi[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        lo[d] = g.order[d] > 0 ? 0 : 1;
-        hi[d] = g.order[d] > 0 ? 3 : 2;
-    }
-    auto pick = [](const T* x, int i) { return i == 0 ? x[0] : (i == 1 ? x[1] : x[2]); };
-#pragma unroll 1
-    for (int kk = lo[2]; kk < hi[2]; kk++) {
-        const int nz = wrap(cz + kk - 1, g.n[2]);
-#pragma unroll 1
-        for (int jj = lo[1]; jj < hi[1]; jj++) {
-            const int ny = wrap(cy + jj - 1, g.n[1]);
-            const T wyz = pick(w[1], jj) * pick(w[2], kk);
-#pragma unroll 1
-            for (int ii = lo[0]; ii < hi[0]; ii++) {
-                const int64_t nb = __builtin_amdgcn_readfirstlane((nz * g.n[1] + ny) * g.n[0] + wrap(cx + ii - 1, g.n[0]));
-                const T wt = pick(w[0], ii) * wyz;
-                const T a[4] = {wt, wt * s[0], wt * s[1], wt * s[2]};
-                const cdp G = grid + nb * QG;
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-#pragma unroll
-                    for (int c = 0; c < nh; c++) out[c] += a[v] * G[v * nh + c];
-            }
-        }
-    }
-}
-
-// The particle's shape factors (from the FP64 positions, rounded to T) and
-// direction (positions frozen within a step).
-template <typename T>
-__device__ __forceinline__ void particle_shape(const AdjInT<T>& in, int64_t p, const Geom& g, T w[3][3], T v[3])
-{
-    const int64_t np = in.np;
-    const double x[3] = {in.pos[p], in.pos[np + p], in.pos[2 * np + p]};
-    const T pt = in.pup[3 * np + p];
-    v[0] = in.pup[p] / pt;
-    v[1] = in.pup[np + p] / pt;
-    v[2] = in.pup[2 * np + p] / pt;
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        int idx;
-        double wd[3];
-        shape3((x[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, wd);
-#pragma unroll
-        for (int e = 0; e < 3; e++) w[d][e] = T(wd[e]);
-    }
-}
-
-// H/hbar and Hbar/hbar of a particle of the wave's cell (as hamiltonians()).
-template <int NF, typename T>
-__device__ __forceinline__ void cell_hamiltonians(const AdjInT<T>& in, int64_t p, const Geom& g, int cell,
-                                                  const T* grid, const HamParams& hp, T* H, T* Hb)
-{
-    constexpr int nh = NH<NF>;
-    T w[3][3], v[3];
-    particle_shape(in, p, g, w, v);
-    const T s[3] = {-v[0], -v[1], -v[2]};
-    T inside[nh];
-#pragma unroll
-    for (int c = 0; c < nh; c++) inside[c] = T(0);
-    gather_cell_box<NF, T>(g, cell, grid, w, s, inside);
-    const T pt = in.pup[3 * in.np + p];
-#pragma unroll
-    for (int c = 0; c < nh; c++) {
-        const T hv = T(hp.vac[c]) / pt, hs = T(hp.coef) * inside[c];
-        H[c] = hv + hs;
-        Hb[c] = is_im_comp<NF>(c) ? hs - hv : hv - hs;
-    }
-}
-
 // A wave's deposit of its cell's particles on the f64 matrix cores, a chunk
 // of up to 64 at a time: lane l's particle adds its source row (NH values,
 // zero on inactive lanes) times (1, s_x, s_y, s_z) with its shape factors to
@@ -814,38 +769,64 @@ template <int NF> struct WaveDeposit {
     }
 };
 
-// Stage S of one step, in.Y = Y_S, grid = its deposit (rounded to T).
-//  STORE 0 (the forward step): S = 1..3 write Y_{S+1} into ynext and the
-//  accumulator into acc; S = 4 finishes acc = y_{n+1}, renormalizes it
-//  (status deferred into err) and advances the particle's position.
+// Waves per workgroup of a kernel that holds `boxes` neighbourhoods and, with dep,
+// a deposit's region per wave: 4, or 2 where 4 would pass 64 KB of static LDS.
+template <int NF, typename T> constexpr int step_lds_bytes(int boxes, bool dep)
+{
+    return boxes * CellBox<NF, T>::N * (int)sizeof(T) + (dep ? WaveDeposit<NF>::REG * 8 : 0) + 28 * 4;
+}
+template <int NF, typename T> constexpr int step_waves(int boxes, bool dep)
+{
+    return 4 * step_lds_bytes<NF, T>(boxes, dep) <= 65536 ? 4 : 2;
+}
+
+// Stage S of one step, in.Y = Y_S, grid = its deposit.
+//  STORE 0 (the forward step): S = 1..3 write Y_{S+1} into ynext, S = 3 also the
+//  accumulator acc; S = 4 finishes acc = y_{n+1}, renormalizes it (status
+//  deferred into err) and advances the particle's position.  The accumulators
+//  after stages 1 and 2 are not stored: with Y2 = y + dt/2 k1 and Y3 = y + dt/2 k2
+//  the second is Y3 + (Y2 - Y3)/3, which stage 3 forms from y2 = Y2 and in.Y = Y3
+//  (24 NF^2 fewer values moved per particle and step; the change is at
+//  rounding level, as in the fused step).
 //  STORE 1 (the VJP's recompute): S = 1..3 write Y_{S+1} into ynext only.
-//  With DEP (S = 1..3), the stage also deposits Y_{S+1} onto gnext (its base
-//  already there), the wave's particles on the matrix cores as the deposit
-//  kernel does: positions are frozen within the step, so the cell's particles
-//  are the ones whose stencils the deposit needs, and the stage state goes
-//  from registers to the grid without a second pass over the particles.  That
-//  pays at NF = 2; at NF = 3 the deposit's 36 columns and the gather's 36-value
-//  rows in one kernel ran slower than the two kernels, which NF = 3 keeps.
-template <int NF, int S, int STORE, typename T, bool DEP>
-__global__ __launch_bounds__(64 * kCellWaves) void k_fwd_stage(AdjInT<T> in, Geom g, const int* start, const int* perm,
-                                                               int64_t ncell, int bpx, const T* grid, HamParams hp,
-                                                               const T* y0, T* ynext, T* acc, const T* Ll,
-                                                               double maxError, double dt, double* pos_out,
-                                                               unsigned long long* err, double* gnext)
+//  S = 1..3 also deposit Y_{S+1} onto gnext (its base already there), the wave's
+//  particles on the matrix cores: positions are frozen within the step, so the
+//  cell's particles are the ones whose stencils the deposit needs, and the stage
+//  state goes from registers to the grid without a second pass over the
+//  particles (3 flavours too: 706k particles in FP32, stage 1 at 124 us with the
+//  deposit inside against 88 us and 80 us for a deposit of its own).
+// Bounded by latency and memory together: stage 3 moves 1.26 GB in 483 us at 3.0 M
+// particles, 2 flavours, FP64 (50 % of the rate of a large copy).
+template <int NF, int S, int STORE, typename T>
+__global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stage(
+    AdjInT<T> in, Geom g, const int* start, const int* perm, int64_t ncell, int bpx, const double* grid, HamParams hp,
+    const T* y0, const T* y2, T* ynext, T* acc, const T* Ll, double maxError, double dt, double* pos_out,
+    unsigned long long* err, double* gnext)
 {
     using WD = WaveDeposit<NF>;
-    static_assert(!DEP || S < 4, "stage 4 deposits nothing");
+    using Box = CellBox<NF, T>;
+    constexpr bool DEP = S < 4;
+    constexpr int WAVES = step_waves<NF, T>(1, DEP);
     constexpr int nh = NH<NF>, S2 = 2 * nh;
-    __shared__ double lds[DEP ? kCellWaves * WD::REG : 1];
+    __shared__ T boxes[WAVES * Box::N];
+    __shared__ double lds[DEP ? WAVES * WD::REG : 1];
+    __shared__ int tables[WAVES * 28];
     const int wave = threadIdx.x >> 6;
-    double* Wf = lds + wave * WD::REG;
+    T* box = boxes + wave * Box::N;
+    double* Wf = lds + (DEP ? wave * WD::REG : 0);
     double* Sr = Wf + 64 * 9;
     const int64_t np = in.np;
-    const int cell = wave_cell(ncell, bpx);
+    const int cell = wave_cell<WAVES>(ncell, bpx);
     if (cell < 0) return;
     const int beg = __builtin_amdgcn_readfirstlane(start[cell]), end = __builtin_amdgcn_readfirstlane(start[cell + 1]);
     if (beg == end) return;
     const int lane = threadIdx.x & 63;
+    Box::table(g, cell, lane, tables + 28 * wave);
+    wave_sync();
+    Box::stage(grid, tables + 28 * wave, lane, box);
+    wave_sync();
+    typename Box::Gather gather;
+    gather.init(lane);
     const T a_next = T(S == 3 ? dt * 1.0 : dt * 0.5);
     const T a_acc = T(S == 1 || S == 4 ? dt * (1. / 6.) : dt * (1. / 3.));
     WD dep;
@@ -855,23 +836,23 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_fwd_stage(AdjInT<T> in, Geo
         const int64_t p = perm[act ? base + lane : beg];
         const double x[3] = {in.pos[p], in.pos[np + p], in.pos[2 * np + p]};
         double wd[3][3];
-        T w[3][3];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             int idx;
             shape3((x[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, wd[d]);
-#pragma unroll
-            for (int e = 0; e < 3; e++) w[d][e] = T(wd[d][e]);
         }
         const T pt = in.pup[3 * np + p];
         const T v[3] = {in.pup[p] / pt, in.pup[np + p] / pt, in.pup[2 * np + p] / pt};
         T H[nh], Hb[nh];
         {
-            const T sv[3] = {-v[0], -v[1], -v[2]};
             T inside[nh];
-#pragma unroll
-            for (int c = 0; c < nh; c++) inside[c] = T(0);
-            gather_cell_box<NF, T>(g, cell, grid, w, sv, inside);
+            gather.template run<-1>(
+                wd, (min(64, end - base) + 15) >> 4, [&](int) { return box; },
+                [&](int m, T& v0, T& v1, T& v2) {
+                    const int from = 16 * m + (lane & 15);
+                    v0 = __shfl(v[0], from), v1 = __shfl(v[1], from), v2 = __shfl(v[2], from);
+                },
+                inside);
 #pragma unroll
             for (int c = 0; c < nh; c++) {
                 const T hv = T(hp.vac[c]) / pt, hs = T(hp.coef) * inside[c];
@@ -879,27 +860,27 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_fwd_stage(AdjInT<T> in, Geo
                 Hb[c] = is_im_comp<NF>(c) ? hs - hv : hv - hs;
             }
         }
-        T q[nh]; // the sources of Y_{S+1} for the fused deposit (zero on inactive lanes)
+        T q[nh]; // the sources of Y_{S+1} for the deposit (zero on inactive lanes)
 #pragma unroll
         for (int c = 0; c < nh; c++) q[c] = T(0);
         if (act) {
-            T f[nh], k[S2];
+            T f[S2], k[S2];
 #pragma unroll
-            for (int c = 0; c < nh; c++) f[c] = in.Y[(int64_t)c * np + p];
+            for (int c = 0; c < S2; c++) f[c] = in.Y[(int64_t)c * np + p];
             commutator_rhs<NF, T>(H, f, k, T(1));
-#pragma unroll
-            for (int c = 0; c < nh; c++) f[c] = in.Y[(int64_t)(nh + c) * np + p];
-            commutator_rhs<NF, T>(Hb, f, k + nh, T(1));
+            commutator_rhs<NF, T>(Hb, f + nh, k + nh, T(1));
             if constexpr (S < 4) {
 #pragma clang fp contract(off)
                 T yv[S2];
 #pragma unroll
                 for (int c = 0; c < S2; c++) {
-                    const T y = y0[(int64_t)c * np + p];
+                    const T y = S == 1 ? f[c] : y0[(int64_t)c * np + p];
                     yv[c] = a_next * k[c] + y;
                     ynext[(int64_t)c * np + p] = yv[c];
-                    if constexpr (STORE == 0)
-                        acc[(int64_t)c * np + p] = a_acc * k[c] + (S == 1 ? y : acc[(int64_t)c * np + p]);
+                    if constexpr (STORE == 0 && S == 3) {
+                        const T a2 = (y2[(int64_t)c * np + p] - f[c]) * T(1.0 / 3.0) + f[c];
+                        acc[(int64_t)c * np + p] = a_acc * k[c] + a2;
+                    }
                 }
                 const T N = in.Nn[p], Nb = in.Nn[np + p];
 #pragma unroll
@@ -943,27 +924,41 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_fwd_stage(AdjInT<T> in, Geo
 //    k_cell_deposit with KIND 1) without writing mu out.
 // Against separate commutator, deposit and gather launches per stage, this
 // form reads each particle once per boundary and holds one stage adjoint
-// array instead of two and no mu array.  Every
+// array instead of two and no mu array.  Its floor is the 1.2 GB that a boundary
+// moves at 3.0 M particles, 2 flavours, FP64: 235 us of the 590 us it takes; two
+// gathers' and a deposit's matrix instructions do not overlap with the rest at the
+// two waves per SIMD that its registers allow.  Every
 // stencil width runs the 3 x 3 x 3 target set (the weights of an order-0
 // dimension are (0, 1, 0), so its other targets receive zeros).
 template <int NF, typename T, bool G, bool C>
-__global__ __launch_bounds__(64 * kCellWaves) void k_vjp_fused(AdjInT<T> in, Geom g, const int* start,
-                                                               const int* perm, int64_t ncell, int bpx,
-                                                               const T* Ynext, const T* Ycur, const T* gadj_in,
-                                                               const T* grid, double* gadj_out, HamParams hp,
-                                                               const T* lam, T* lY, T* lam_out, double* lamNbar,
-                                                               int first, double alpha, double beta)
+__global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void k_vjp_fused(
+    AdjInT<T> in, Geom g, const int* start, const int* perm, int64_t ncell, int bpx, const T* Ynext, const T* Ycur,
+    const double* gadj_in, const double* grid, double* gadj_out, HamParams hp, const T* lam, T* lY, T* lam_out,
+    double* lamNbar, int first, double alpha, double beta)
 {
     using WD = WaveDeposit<NF>;
+    using Box = CellBox<NF, T>;
+    constexpr int WAVES = step_waves<NF, T>(int(G) + int(C), C);
     constexpr int nh = NH<NF>;
-    __shared__ double lds[C ? kCellWaves * WD::REG : 1];
+    __shared__ T boxes[WAVES * (int(G) + int(C)) * Box::N];
+    __shared__ double lds[C ? WAVES * WD::REG : 1];
+    __shared__ int tables[WAVES * 28];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    double* Wf = lds + wave * WD::REG;
+    T* boxC = boxes + wave * (int(G) + int(C)) * Box::N;
+    T* boxG = boxC + int(C) * Box::N;
+    double* Wf = lds + (C ? wave * WD::REG : 0);
     double* Sr = Wf + 64 * 9;
-    const int cell = wave_cell(ncell, bpx);
+    const int cell = wave_cell<WAVES>(ncell, bpx);
     if (cell < 0) return;
     const int beg = __builtin_amdgcn_readfirstlane(start[cell]), end = __builtin_amdgcn_readfirstlane(start[cell + 1]);
     if (beg == end) return;
+    Box::table(g, cell, lane, tables + 28 * wave);
+    wave_sync();
+    if constexpr (C) Box::stage(grid, tables + 28 * wave, lane, boxC);
+    if constexpr (G) Box::stage(gadj_in, tables + 28 * wave, lane, boxG);
+    wave_sync();
+    typename Box::Gather gather;
+    gather.init(lane);
     const int64_t np = in.np;
     const T al = T(alpha), be = T(beta);
     WD dep;
@@ -971,25 +966,25 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_vjp_fused(AdjInT<T> in, Geo
     for (int base = beg; base < end; base += 64) {
         const bool act = base + lane < end;
         const int64_t p = perm[act ? base + lane : beg];
-        // shape factors (FP64 for the deposit, T for the gathers) and direction
+        const int ntile = (min(64, end - base) + 15) >> 4;
+        // shape factors and direction
         const double x[3] = {in.pos[p], in.pos[np + p], in.pos[2 * np + p]};
         double wd[3][3];
-        T w[3][3];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             int idx;
             shape3((x[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, wd[d]);
-#pragma unroll
-            for (int e = 0; e < 3; e++) w[d][e] = T(wd[d][e]);
         }
         const T pt = in.pup[3 * np + p];
         const T v[3] = {in.pup[p] / pt, in.pup[np + p] / pt, in.pup[2 * np + p] / pt};
+        auto vel = [&](int m, T& v0, T& v1, T& v2) {
+            const int from = 16 * m + (lane & 15);
+            v0 = __shfl(v[0], from), v1 = __shfl(v[1], from), v2 = __shfl(v[2], from);
+        };
         T lYn[2 * nh];
         if constexpr (G) {
             T lq[nh];
-#pragma unroll
-            for (int c = 0; c < nh; c++) lq[c] = T(0);
-            gather_cell_box<NF, T>(g, cell, gadj_in, w, v, lq);
+            gather.template run<1>(wd, ntile, [&](int) { return boxG; }, vel, lq);
             if (act) {
                 const T N = in.Nn[p], Nb = in.Nn[np + p];
                 T ln = T(0);
@@ -1012,9 +1007,7 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_vjp_fused(AdjInT<T> in, Geo
             T H[nh], Hb[nh];
             {
                 T inside[nh];
-#pragma unroll
-                for (int c = 0; c < nh; c++) inside[c] = T(0);
-                gather_cell_box<NF, T>(g, cell, grid, w, sv, inside);
+                gather.template run<-1>(wd, ntile, [&](int) { return boxC; }, vel, inside);
 #pragma unroll
                 for (int c = 0; c < nh; c++) {
                     const T hv = T(hp.vac[c]) / pt, hs = T(hp.coef) * inside[c];
@@ -1176,9 +1169,9 @@ static double m00_of(const emu_ctx* ctx)
 }
 
 // blocks per XCD of a one-wave-per-cell launch
-static int cell_blocks_per_xcd(int64_t ncell)
+static int cell_blocks_per_xcd(int64_t ncell, int waves = kCellWaves)
 {
-    const int64_t nb = (ncell + kCellWaves - 1) / kCellWaves;
+    const int64_t nb = (ncell + waves - 1) / waves;
     return (int)((nb + 7) / 8);
 }
 
@@ -1358,9 +1351,8 @@ extern "C" int emu_adj_axpy(emu_ctx* ctx, int64_t n, double a, const double* x, 
 // the gathers, commutators and stage algebra in FP32; the deposits sum in
 // FP64 and Renormalize runs in FP64, as in the fused FP32-bulk step).
 // Work layout, in doubles: the four stage grids [4][ncell][4 NH] and two
-// grid adjoints (FP64); for T = float two T copies of grids, which the
-// gathers read; then, in T, the stage states [3][2 NH][np] (Y2, Y3, Y4) and
-// one stage adjoint [2 NH][np]; then the cell sort.
+// grid adjoints (FP64); then, in T, the stage states [3][2 NH][np] (Y2, Y3, Y4)
+// and one stage adjoint [2 NH][np]; then the cell sort.
 // ---------------------------------------------------------------------------
 namespace {
 template <typename T> int64_t t_doubles(int64_t n) { return (n * (int64_t)sizeof(T) + 7) / 8; }
@@ -1368,7 +1360,6 @@ template <typename T> int64_t t_doubles(int64_t n) { return (n * (int64_t)sizeof
 template <typename T> struct StepWork {
     double* G[4];
     double* gadj[2];
-    T* gT[2]; // the grids a float gather reads (the double gathers read the grids themselves)
     T* Ys[3];
     T* lY;
     CellSort cs;
@@ -1382,10 +1373,6 @@ template <typename T> StepWork<T> step_work(const emu_ctx* ctx, int64_t np, doub
     double* b = work;
     for (int s = 0; s < 4; s++, b += ng) w.G[s] = b;
     for (int s = 0; s < 2; s++, b += ng) w.gadj[s] = b;
-    w.gT[0] = w.gT[1] = nullptr;
-    if constexpr (sizeof(T) != sizeof(double)) {
-        for (int s = 0; s < 2; s++, b += t_doubles<T>(ng)) w.gT[s] = (T*)b;
-    }
     for (int s = 0; s < 3; s++, b += t_doubles<T>(ns)) w.Ys[s] = (T*)b;
     w.lY = (T*)b;
     b += t_doubles<T>(ns);
@@ -1397,28 +1384,7 @@ template <typename T> int64_t step_work_doubles(const emu_ctx* ctx, int64_t np)
 {
     const int nh = ctx->p.nf * ctx->p.nf;
     const int64_t ng = ncell_of(ctx) * 4 * nh, ns = 2 * nh * np;
-    return 6 * ng + (sizeof(T) != sizeof(double) ? 2 * t_doubles<T>(ng) : 0) + 4 * t_doubles<T>(ns) +
-           cell_sort_doubles(ctx, np);
-}
-
-__global__ void k_to_float(const double* in, float* out, int64_t n)
-{
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
-        out[t] = (float)in[t];
-}
-
-// The grid a gather reads: the FP64 grid, or its FP32 rounding in buffer
-// `slot` (the FP32-bulk gather's input, as the fused step rounds its grid
-// when staging it).
-template <typename T> const T* gather_grid(emu_ctx* ctx, const StepWork<T>& w, const double* g, int slot = 0)
-{
-    if constexpr (sizeof(T) == sizeof(double)) {
-        return g;
-    } else {
-        const int64_t ng = ncell_of(ctx) * 4 * ctx->p.nf * ctx->p.nf;
-        hipLaunchKernelGGL(k_to_float, dim3(nblk(ng)), dim3(kB), 0, ctx->stream, g, w.gT[slot], ng);
-        return w.gT[slot];
-    }
+    return 6 * ng + 4 * t_doubles<T>(ns) + cell_sort_doubles(ctx, np);
 }
 
 int arm_status(emu_ctx* ctx)
@@ -1431,25 +1397,18 @@ int arm_status(emu_ctx* ctx)
 }
 
 // Stage S reads the deposit of Y_S (grid) and, for S < 4, leaves the deposit
-// of Y_{S+1} on gnext: within the stage kernel at NF = 2, as a kernel of its
-// own after it at NF = 3.
+// of Y_{S+1} on gnext.
 template <int NF, int S, int STORE, typename T>
 void fwd_stage(emu_ctx* ctx, const AdjInT<T>& in, const StepWork<T>& w, const double* grid, const T* y0, T* ynext,
                T* acc, const T* Ll, double dt, double* pos, double wscale, double* gnext)
 {
-    constexpr bool DEP = S < 4 && NF == 2;
+    constexpr int WAVES = step_waves<NF, T>(1, S < 4);
     const int64_t nc = ncell_of(ctx);
-    const int bpx = cell_blocks_per_xcd(nc);
-    if (DEP) fill_base(ctx, gnext, wscale);
-    const T* gg = gather_grid<T>(ctx, w, grid);
-    hipLaunchKernelGGL((k_fwd_stage<NF, S, STORE, T, DEP>), dim3(8 * bpx), dim3(64 * kCellWaves), 0, ctx->stream, in,
-                       ctx->g, w.cs.start, w.cs.perm, nc, bpx, gg, ham_params(ctx, wscale), y0, ynext, acc, Ll,
-                       ctx->p.maxError, dt, pos, ctx->d_red + 5, gnext);
-    if (S < 4 && !DEP) {
-        AdjInT<T> next = in;
-        next.Y = ynext;
-        deposit(ctx, next, w.cs, gnext, wscale);
-    }
+    const int bpx = cell_blocks_per_xcd(nc, WAVES);
+    if (S < 4) fill_base(ctx, gnext, wscale);
+    hipLaunchKernelGGL((k_fwd_stage<NF, S, STORE, T>), dim3(8 * bpx), dim3(64 * WAVES), 0, ctx->stream, in, ctx->g,
+                       w.cs.start, w.cs.perm, nc, bpx, grid, ham_params(ctx, wscale), y0, (const T*)w.Ys[0], ynext, acc,
+                       Ll, ctx->p.maxError, dt, pos, ctx->d_red + 5, gnext);
 }
 
 // A step's kept data (emu_adj_step_keep): the stage states Y2, Y3, Y4
@@ -1532,34 +1491,33 @@ int adj_step_vjp_nf(emu_ctx* ctx, int64_t np, const double* pos, const T* pup, c
     // lam_out = lam + lY4 + lY3 + lY2 + lY1.  Launch s (3 .. -1) finishes
     // stage s+1's lY (the gather back of its grid adjoint) and runs stage s's
     // commutator adjoints, depositing mu_s onto the other grid adjoint.
-    const int bpx = cell_blocks_per_xcd(ncell_of(ctx));
     const double alpha[4] = {dt * (1. / 6.), dt * (1. / 3.), dt * (1. / 3.), dt * (1. / 6.)};
     const double beta[4] = {dt * 0.5, dt * 0.5, dt * 1.0, 0.0};
     const HamParams hp = ham_params(ctx, wscale);
-    const dim3 grid_dim(8 * bpx), block_dim(64 * kCellWaves);
+    const int64_t nc = ncell_of(ctx);
+#define VJP_LAUNCH(G, C)                                                                                             \
+    do {                                                                                                             \
+        constexpr int WAVES = step_waves<NF, T>(int(G) + int(C), C);                                                  \
+        const int bpx = cell_blocks_per_xcd(nc, WAVES);                                                               \
+        hipLaunchKernelGGL((k_vjp_fused<NF, T, G, C>), dim3(8 * bpx), dim3(64 * WAVES), 0, ctx->stream, in, ctx->g,    \
+                           w.cs.start, w.cs.perm, nc, bpx, ynext, ycur, gin, gs, gout, hp, lam_in, w.lY, lam_out,     \
+                           lam_Nbar, first, a, b);                                                                    \
+    } while (0)
     for (int s = 3; s >= -1; s--) {
         const bool g_half = s < 3, c_half = s >= 0;
         double* gout = c_half ? w.gadj[s & 1] : nullptr;
         if (c_half) hipLaunchKernelGGL(k_zero, dim3(nblk(ng)), dim3(kB), 0, ctx->stream, gout, ng);
-        const T* gin = g_half ? gather_grid<T>(ctx, w, w.gadj[(s + 1) & 1], 1) : nullptr;
-        const T* gs = c_half ? gather_grid<T>(ctx, w, w.G[s], 0) : nullptr;
+        const double* gin = g_half ? w.gadj[(s + 1) & 1] : nullptr;
+        const double* gs = c_half ? w.G[s] : nullptr;
         const T* ynext = g_half ? Yst[s + 1] : nullptr;
         const T* ycur = c_half ? Yst[s] : nullptr;
         const double a = c_half ? alpha[s] : 0.0, b = c_half ? beta[s] : 0.0;
         const int first = s == 2 ? 1 : 0;
-        if (!g_half)
-            hipLaunchKernelGGL((k_vjp_fused<NF, T, false, true>), grid_dim, block_dim, 0, ctx->stream, in, ctx->g,
-                               w.cs.start, w.cs.perm, ncell_of(ctx), bpx, ynext, ycur, gin, gs, gout, hp, lam_in, w.lY,
-                               lam_out, lam_Nbar, first, a, b);
-        else if (c_half)
-            hipLaunchKernelGGL((k_vjp_fused<NF, T, true, true>), grid_dim, block_dim, 0, ctx->stream, in, ctx->g,
-                               w.cs.start, w.cs.perm, ncell_of(ctx), bpx, ynext, ycur, gin, gs, gout, hp, lam_in, w.lY,
-                               lam_out, lam_Nbar, first, a, b);
-        else
-            hipLaunchKernelGGL((k_vjp_fused<NF, T, true, false>), grid_dim, block_dim, 0, ctx->stream, in, ctx->g,
-                               w.cs.start, w.cs.perm, ncell_of(ctx), bpx, ynext, ycur, gin, gs, gout, hp, lam_in, w.lY,
-                               lam_out, lam_Nbar, first, a, b);
+        if (!g_half) VJP_LAUNCH(false, true);
+        else if (c_half) VJP_LAUNCH(true, true);
+        else VJP_LAUNCH(true, false);
     }
+#undef VJP_LAUNCH
     return EMU_OK;
 }
 

@@ -115,22 +115,31 @@ template <> struct Mfma16x16x4<float> {
 // for any NH.)  The particle's own lane forms its 27 weights once; a transpose of
 // 16-lane rows turns four of them into the operands of all four tiles, and
 // another returns the results, without LDS.
-template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false> struct WaveGather {
+// LIN: the neighbours' rows follow each other in t, LIN values apart, and a row of
+// zeros (or any finite values) follows the last one.
+template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false, int LIN = 0> struct WaveGather {
     using MF = Mfma16x16x4<T>;
     static constexpr int nh = NH<NF>, NT = WX * WY * WZ, KK = (NT + 3) / 4, MG = (nh + 3) / 4;
     // this lane's entry of A at step k, row i = l%16, neighbour t = 4k + l/16 (past
     // the last one: any in-range entry, its weight is zero; rows past NH feed
     // results that are dropped)
-    unsigned goff[PACK ? (KK + 1) / 2 : KK]; // PACK: two 16-bit offsets each, taken apart once per chunk
+    // (LIN: step 0 only; PACK: two 16-bit offsets each, taken apart once per chunk)
+    unsigned goff[LIN ? 1 : (PACK ? (KK + 1) / 2 : KK)];
 
     // row(t): offset of neighbour t's row of fields
+    __device__ __forceinline__ void init(int lane)
+    {
+        static_assert(LIN > 0, "rows at a constant distance");
+        goff[0] = (lane >> 4) * LIN + MF::group(lane & 15) * nh + MF::comp(lane & 15);
+    }
     template <typename F> __device__ __forceinline__ void init(int lane, F&& row)
     {
+        static_assert(LIN == 0, "rows anywhere");
 #pragma unroll
         for (int k = 0; k < KK; k++) {
             const int t = 4 * k + (lane >> 4);
             const unsigned o = row(t < NT ? t : NT - 1) + MF::group(lane & 15) * nh + MF::comp(lane & 15);
-            if (PACK) goff[k / 2] = k % 2 ? goff[k / 2] | o << 16 : o;
+            if constexpr (PACK) goff[k / 2] = k % 2 ? goff[k / 2] | o << 16 : o;
             else goff[k] = o;
         }
     }
@@ -143,8 +152,14 @@ template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false> struct 
         int off[KK];
 #pragma unroll
         for (int k = 0; k < KK; k++) {
-            if (PACK && k % 2 == 0) asm volatile("" : "+v"(goff[k / 2]));
-            off[k] = !PACK ? goff[k] : (k % 2 ? goff[k / 2] >> 16 : goff[k / 2] & 0xffffu);
+            if constexpr (LIN > 0) {
+                off[k] = goff[0] + 4 * k * LIN;
+            } else if constexpr (PACK) {
+                if (k % 2 == 0) asm volatile("" : "+v"(goff[k / 2]));
+                off[k] = k % 2 ? goff[k / 2] >> 16 : goff[k / 2] & 0xffffu;
+            } else {
+                off[k] = goff[k];
+            }
         }
         T w[4 * KK];
         {

@@ -51,8 +51,9 @@ int emu_adj_axpy(emu_ctx* ctx, int64_t n, double a, const double* x, const doubl
 int64_t emu_adj_step_work_doubles(const emu_ctx* ctx, int64_t np);
 
 /* One RK4 step of length dt at the step's positions (main.cpp:129-213 with
- * the RK hook of FlavoredNeutrinoContainer.H:33-47; the stage states and
- * accumulator rounded as the AMReX RK4 saxpys): y_out = y_{n+1} from
+ * the RK hook of FlavoredNeutrinoContainer.H:33-47; the stage states rounded
+ * as the AMReX RK4 saxpys, the accumulator of the first two stages formed
+ * again from the stage states to rounding): y_out = y_{n+1} from
  * y_in = y_n, Renormalize on y_out (FlavoredNeutrinoContainer.cpp:89-113)
  * with its status deferred to emu_adj_status, then pos advanced in place.
  * y_out must not alias y_in.  Asynchronous. */
