@@ -61,3 +61,60 @@ def test_step_kernels_at_the_edges(oracle, nf, form):
     fd = float((lam * (step(p64.f0 + h * dy) - step(p64.f0 - h * dy))).sum() / (2 * h))
     assert float((g * dy).sum()) == pytest.approx(fd, rel=1e-8)
     assert close(p32.step_adjoint(pos, p32.Nn_base, p32.f0, lam.float()), g, 1e-5)
+
+
+def shape_weights(x, n, order):
+    """Cell indexes and weights of a shape of the given order, 3 targets a dimension."""
+    if order == 0:
+        i = np.floor(x).astype(int)
+        return [(i % n, np.ones_like(x))]
+    if order == 1:
+        i = np.floor(x - 0.5).astype(int)
+        t = x - 0.5 - i
+        return [(i % n, 1 - t), ((i + 1) % n, t)]
+    i = np.floor(x).astype(int)
+    t = x - i - 0.5
+    return [((i - 1) % n, 0.5 * (0.5 - t) ** 2), (i % n, 0.75 - t * t), ((i + 1) % n, 0.5 * (0.5 + t) ** 2)]
+
+
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nf", [2, 3])
+def test_objective_at_the_edges(oracle, nf, prec, form):
+    """J and dJ/dY against sums in numpy.  A cell's sum over n <= 4608 particles is off
+    by at most n eps = 1e-12 of the sum of magnitudes, J by twice that of the sum of
+    their squares; the float form writes dJ/dY in float (6e-8)."""
+    import torch
+    from emu_amd import adjoint, core
+    ncell, nphi, order, crowd = form
+    d = cases.fast_flavor_dict(nf=nf, ncell=ncell, nphi=nphi, st4_amplitude=1e-3, maxError=1e-2, shape_order=order)
+    emu = core.Emu(cases.product_params(d))
+    c = core.FlavoredNeutrinoContainer.from_aos(emu, oracle.init_particles(cases.oracle_deck(oracle, d)))
+    prob = adjoint.AdjointProblem(emu, c, dt=1e-13, nsteps=1, precision=prec)
+    rng = np.random.default_rng(23)
+    n = prob.pos0.shape[1]
+    at = rng.random((3, n)) * 0.5 * np.array(ncell)[:, None]
+    at[:, rng.random(n) < crowd] = 0.25
+    Y = prob.f0 + torch.from_numpy(rng.standard_normal(prob.f0.shape)).to(prob.f0) * 0.1
+    J, dJ = prob.objective(torch.from_numpy(at).to(prob.pos0), prob.Nn_base, Y)
+    N = prob.Nn_base.cpu().numpy().astype(np.float64)[0]
+    f = Y.cpu().numpy().astype(np.float64)
+    re, im = emu.K["f01_Re"] - emu.K["f00_Re"], emu.K["f01_Im"] - emu.K["f00_Re"]
+    grid, mags = np.zeros(ncell, dtype=complex), np.zeros(ncell)
+    targets = []
+    for ix, wx in shape_weights(at[0] / 0.5, ncell[0], order):
+        for iy, wy in shape_weights(at[1] / 0.5, ncell[1], order):
+            for iz, wz in shape_weights(at[2] / 0.5, ncell[2], order):
+                w = wx * wy * wz
+                targets.append((ix, iy, iz, w))
+                np.add.at(grid, (ix, iy, iz), w * N * (f[re] + 1j * f[im]))
+                np.add.at(mags, (ix, iy, iz), w * N * (abs(f[re]) + abs(f[im])))
+    assert abs(J - (abs(grid) ** 2).sum()) <= 2e-12 * (mags ** 2).sum()
+    got = dJ.cpu().numpy().astype(np.float64)
+    back = sum(w * grid[ix, iy, iz] for ix, iy, iz, w in targets)
+    most = sum(w * mags[ix, iy, iz] for ix, iy, iz, w in targets)
+    eps = 2e-12 if prec == "fp64" else 2e-12 + 6e-8
+    assert (abs(got[re] - 2 * N * back.real) <= eps * 2 * N * most).all()
+    assert (abs(got[im] - 2 * N * back.imag) <= eps * 2 * N * most).all()
+    got[[re, im]] = 0
+    assert not got.any()
