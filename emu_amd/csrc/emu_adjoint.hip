@@ -376,7 +376,7 @@ __device__ __forceinline__ void wave_sync()
 // The gather read the grid through scalar loads before (one neighbour's fields at a
 // time, every lane the same ones), a chain of 27 loads per chunk with nothing else
 // for the wave to do: on 32^3 cells x 92 particles, 2 flavours in FP64, a stage took
-// 398 us and a reverse boundary 715 us, now 284 and 590.
+// 398 us and a reverse boundary 715 us, then 284 and 590.
 template <int NF, typename T> struct CellBox {
     static constexpr int QG = 4 * NH<NF>, N = 28 * QG;
     using Gather = WaveGather<NF, T, 3, 3, 3, false, QG>;
@@ -792,8 +792,9 @@ template <int NF, typename T> constexpr int step_waves(int boxes, bool dep)
 //  state goes from registers to the grid without a second pass over the
 //  particles (3 flavours too: 706k particles in FP32, stage 1 at 124 us with the
 //  deposit inside against 88 us and 80 us for a deposit of its own).
-// Bounded by latency and memory together: stage 3 moves 1.26 GB in 483 us at 3.0 M
-// particles, 2 flavours, FP64 (50 % of the rate of a large copy).
+// Bounded by latency and memory together: stage 3 moves 1.2 GB in 392 us at 3.0 M
+// particles, 2 flavours, FP64 (60 % of the rate of a large copy); with a load after
+// each store it took 482 us, with the loads ahead of the gather 409 (registers).
 template <int NF, int S, int STORE, typename T>
 __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stage(
     AdjInT<T> in, Geom g, const int* start, const int* perm, int64_t ncell, int bpx, const double* grid, HamParams hp,
@@ -832,14 +833,15 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
         const bool act = base + lane < end;
         const int64_t p = perm[act ? base + lane : beg];
         const double x[3] = {in.pos[p], in.pos[np + p], in.pos[2 * np + p]};
+        const T pt = in.pup[3 * np + p];
+        const T u[3] = {in.pup[p], in.pup[np + p], in.pup[2 * np + p]};
         double wd[3][3];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             int idx;
             shape3((x[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, wd[d]);
         }
-        const T pt = in.pup[3 * np + p];
-        const T v[3] = {in.pup[p] / pt, in.pup[np + p] / pt, in.pup[2 * np + p] / pt};
+        const T v[3] = {u[0] / pt, u[1] / pt, u[2] / pt};
         T H[nh], Hb[nh];
         {
             T inside[nh];
@@ -861,9 +863,19 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
 #pragma unroll
         for (int c = 0; c < nh; c++) q[c] = T(0);
         if (act) {
-            T f[S2], k[S2];
+            // (all of the particle's loads before the first store: the compiler cannot
+            // tell that the arrays do not overlap, and would wait for each load in turn)
+            T f[S2], r0[S2], r2[S2], w0[2];
 #pragma unroll
-            for (int c = 0; c < S2; c++) f[c] = in.Y[(int64_t)c * np + p];
+            for (int c = 0; c < S2; c++) {
+                const int64_t o = (int64_t)c * np + p;
+                f[c] = in.Y[o];
+                if (S == 2 || S == 3) r0[c] = y0[o];
+                if (S == 4) r0[c] = acc[o];
+                if (S == 3 && STORE == 0) r2[c] = y2[o];
+            }
+            if (S < 4) w0[0] = in.Nn[p], w0[1] = in.Nn[np + p];
+            T k[S2];
             commutator_rhs<NF, T>(H, f, k, T(1));
             commutator_rhs<NF, T>(Hb, f + nh, k + nh, T(1));
             if constexpr (S < 4) {
@@ -871,15 +883,15 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
                 T yv[S2];
 #pragma unroll
                 for (int c = 0; c < S2; c++) {
-                    const T y = S == 1 ? f[c] : y0[(int64_t)c * np + p];
+                    const T y = S == 1 ? f[c] : r0[c];
                     yv[c] = a_next * k[c] + y;
                     ynext[(int64_t)c * np + p] = yv[c];
                     if constexpr (STORE == 0 && S == 3) {
-                        const T a2 = (y2[(int64_t)c * np + p] - f[c]) * T(1.0 / 3.0) + f[c];
+                        const T a2 = (r2[c] - f[c]) * T(1.0 / 3.0) + f[c];
                         acc[(int64_t)c * np + p] = a_acc * k[c] + a2;
                     }
                 }
-                const T N = in.Nn[p], Nb = in.Nn[np + p];
+                const T N = w0[0], Nb = w0[1];
 #pragma unroll
                 for (int c = 0; c < nh; c++)
                     q[c] = is_im_comp<NF>(c) ? N * yv[c] + Nb * yv[nh + c] : N * yv[c] - Nb * yv[nh + c];
@@ -889,7 +901,7 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
                 // nu, then nubar unless nu failed; a failing half is left as it is
                 double y[S2];
 #pragma unroll
-                for (int c = 0; c < S2; c++) y[c] = double(a_acc * k[c] + acc[(int64_t)c * np + p]);
+                for (int c = 0; c < S2; c++) y[c] = double(a_acc * k[c] + r0[c]);
                 int e = renorm_fp64<NF>(y, double(Ll[p]), maxError);
                 if (e == EMU_OK) e = renorm_fp64<NF>(y + nh, double(Ll[np + p]), maxError);
                 if (e != EMU_OK) atomicMin(err, status_word(p, e));
@@ -898,7 +910,7 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
                 double vv[3], nx[3];
 #pragma unroll
                 for (int d = 0; d < 3; d++)
-                    vv[d] = double(in.pup[(int64_t)d * np + p]) / double(in.pup[3 * np + p]) * phys::c;
+                    vv[d] = double(u[d]) / double(pt) * phys::c;
                 end_position(x, vv, dt, g, nx);
 #pragma unroll
                 for (int d = 0; d < 3; d++) pos_out[(int64_t)d * np + p] = nx[d];
@@ -922,7 +934,7 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
 // Against separate commutator, deposit and gather launches per stage, this
 // form reads each particle once per boundary and holds one stage adjoint
 // array instead of two and no mu array.  Its floor is the 1.2 GB that a boundary
-// moves at 3.0 M particles, 2 flavours, FP64: 235 us of the 590 us it takes; two
+// moves at 3.0 M particles, 2 flavours, FP64: 235 us of the 501 us it takes; two
 // gathers' and a deposit's matrix instructions do not overlap with the rest at the
 // two waves per SIMD that its registers allow.  Every
 // stencil width runs the 3 x 3 x 3 target set (the weights of an order-0
@@ -964,16 +976,17 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void 
         const bool act = base + lane < end;
         const int64_t p = perm[act ? base + lane : beg];
         const int ntile = (min(64, end - base) + 15) >> 4;
-        // shape factors and direction
         const double x[3] = {in.pos[p], in.pos[np + p], in.pos[2 * np + p]};
+        const T pt = in.pup[3 * np + p];
+        const T u[3] = {in.pup[p], in.pup[np + p], in.pup[2 * np + p]};
+        // shape factors and direction
         double wd[3][3];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             int idx;
             shape3((x[d] - g.plo[d]) * g.dxi[d], g.order[d], idx, wd[d]);
         }
-        const T pt = in.pup[3 * np + p];
-        const T v[3] = {in.pup[p] / pt, in.pup[np + p] / pt, in.pup[2 * np + p] / pt};
+        const T v[3] = {u[0] / pt, u[1] / pt, u[2] / pt};
         auto vel = [&](int m, T& v0, T& v1, T& v2) {
             const int from = 16 * m + (lane & 15);
             v0 = __shfl(v[0], from), v1 = __shfl(v[1], from), v2 = __shfl(v[2], from);
@@ -984,17 +997,24 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void 
             gather.template run<1>(wd, ntile, [&](int) { return boxG; }, vel, lq);
             if (act) {
                 const T N = in.Nn[p], Nb = in.Nn[np + p];
+                T l0[2 * nh], o0[2 * nh], yn[nh]; // loads before stores, as in k_fwd_stage
+#pragma unroll
+                for (int c = 0; c < 2 * nh; c++) {
+                    const int64_t o = (int64_t)c * np + p;
+                    l0[c] = lY[o];
+                    o0[c] = first ? lam[o] : lam_out[o];
+                    if (c >= nh) yn[c - nh] = Ynext[o];
+                }
                 T ln = T(0);
 #pragma unroll
                 for (int c = 0; c < nh; c++) {
 #pragma clang fp contract(off)
                     const T sg = is_im_comp<NF>(c) ? T(1) : T(-1);
-                    const int64_t o0 = (int64_t)c * np + p, o1 = (int64_t)(nh + c) * np + p;
-                    lYn[c] = lY[o0] + N * lq[c];
-                    lYn[nh + c] = lY[o1] + sg * Nb * lq[c];
-                    lam_out[o0] = T(1) * lYn[c] + (first ? lam[o0] : lam_out[o0]);
-                    lam_out[o1] = T(1) * lYn[nh + c] + (first ? lam[o1] : lam_out[o1]);
-                    ln += sg * Ynext[o1] * lq[c];
+                    lYn[c] = l0[c] + N * lq[c];
+                    lYn[nh + c] = l0[nh + c] + sg * Nb * lq[c];
+                    lam_out[(int64_t)c * np + p] = T(1) * lYn[c] + o0[c];
+                    lam_out[(int64_t)(nh + c) * np + p] = T(1) * lYn[nh + c] + o0[nh + c];
+                    ln += sg * yn[c] * lq[c];
                 }
                 if (lamNbar) lamNbar[p] += double(ln);
             }
@@ -1016,25 +1036,29 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void 
 #pragma unroll
             for (int c = 0; c < nh; c++) mu[c] = T(0);
             if (act) {
-                T gH[2][nh];
+                T lm[2 * nh], f[2 * nh], gH[2][nh];
+#pragma unroll
+                for (int c = 0; c < 2 * nh; c++) {
+                    const int64_t o = (int64_t)c * np + p;
+                    lm[c] = lam[o];
+                    f[c] = Ycur[o];
+                }
 #pragma unroll
                 for (int bar = 0; bar < 2; bar++) {
-                    T lk[nh], L[nh], f[nh], gy[nh];
+                    T lk[nh], L[nh], gy[nh];
 #pragma unroll
                     for (int c = 0; c < nh; c++) {
 #pragma clang fp contract(off)
-                        const int64_t o = (int64_t)(bar * nh + c) * np + p;
-                        const T t = al * lam[o];
+                        const T t = al * lm[bar * nh + c];
                         if constexpr (G) lk[c] = be * lYn[bar * nh + c] + t;
                         else lk[c] = t;
-                        f[c] = Ycur[o];
                     }
                     lam_matrix<NF, T>(lk, L);
                     commutator_rhs<NF, T>(L, bar ? Hb : H, gy, T(1)); // -i[Lam, A]
                     double_offdiag<NF, T>(gy);
 #pragma unroll
                     for (int c = 0; c < nh; c++) lY[(int64_t)(bar * nh + c) * np + p] = gy[c];
-                    commutator_rhs<NF, T>(f, L, gH[bar], T(1));       // -i[B, Lam]
+                    commutator_rhs<NF, T>(f + bar * nh, L, gH[bar], T(1)); // -i[B, Lam]
                     double_offdiag<NF, T>(gH[bar]);
                 }
 #pragma unroll
