@@ -63,6 +63,8 @@ _SIGS = [
     ("emu_deposit_to_mesh_static", ctypes.c_int, [_P, ctypes.POINTER(EmuParticles), ctypes.POINTER(EmuGrid)]),
     ("emu_fill_boundary", ctypes.c_int, [_P, ctypes.POINTER(EmuGrid)]),
     ("emu_interpolate_rhs_from_mesh", ctypes.c_int, [_P, ctypes.POINTER(EmuParticles), ctypes.POINTER(EmuGrid)]),
+    ("emu_rhs_from_mesh", ctypes.c_int, [_P, ctypes.POINTER(EmuParticles), ctypes.POINTER(EmuParticles),
+                                          ctypes.POINTER(EmuGrid)]),
     ("emu_compute_dt", ctypes.c_int, [_P, ctypes.POINTER(EmuGrid), ctypes.c_double, ctypes.POINTER(ctypes.c_double)]),
     ("emu_vvac_max", ctypes.c_int, [_P, ctypes.POINTER(EmuParticles), ctypes.POINTER(ctypes.c_double)]),
     ("emu_renormalize", ctypes.c_int, [_P, ctypes.POINTER(EmuParticles), ctypes.POINTER(ctypes.c_int64)]),

@@ -81,6 +81,17 @@ class Emu:
         return tuple(g)
 
 
+def _row_pointers(t, n: int) -> list:
+    """Device addresses of rows 0 .. n-1 (a tensor's from its stride: one call
+    into torch, where a view per row costs 1 us each)."""
+    if not isinstance(t, torch.Tensor):
+        return [t[k].data_ptr() for k in range(n)]
+    if t.shape[0] < n:
+        raise IndexError(f"{n} rows wanted, the array has {t.shape[0]}")
+    base, pitch = t.data_ptr(), t.stride(0) * t.element_size()
+    return [base + k * pitch for k in range(n)]
+
+
 class FlavoredNeutrinoContainer:
     """SoA particle container on the device: pos (3, np) and rdata
     (nattribs, np), float64, PIdx order; ids (np,) int64."""
@@ -96,10 +107,10 @@ class FlavoredNeutrinoContainer:
     def view(self) -> capi.EmuParticles:
         v = capi.EmuParticles()
         v.np = self.np
-        for d in range(3):
-            v.pos[d] = self.pos[d].data_ptr() if self.np else None
-        for k in range(self.emu.nattribs):
-            v.rdata[k] = self.rdata[k].data_ptr() if self.np else None
+        if self.np:
+            n = self.emu.nattribs
+            v.pos[:] = _row_pointers(self.pos, 3)
+            v.rdata[:n] = _row_pointers(self.rdata, n)
         return v
 
     @classmethod
@@ -224,6 +235,17 @@ def interpolate_rhs_from_mesh(neutrinos_rhs: FlavoredNeutrinoContainer, state: M
           "interpolate_rhs_from_mesh", state.emu.ctx)
 
 
+def rhs_from_mesh(neutrinos_rhs: FlavoredNeutrinoContainer, neutrinos: FlavoredNeutrinoContainer, state: MultiFab):
+    """copyParticles(neutrinos) (main.cpp:148) and interpolate_rhs_from_mesh
+    (Evolve.cpp:128-176) in one call: the gather writes the rhs container."""
+    if neutrinos.np != neutrinos_rhs.np:
+        raise ValueError("size mismatch")
+    d, p, g = neutrinos_rhs.view(), neutrinos.view(), state.view()
+    check(lib().emu_rhs_from_mesh(state.emu.ctx, ctypes.byref(d), ctypes.byref(p), ctypes.byref(g)), "rhs_from_mesh",
+          state.emu.ctx)
+    neutrinos_rhs.ids.copy_(neutrinos.ids)
+
+
 def compute_dt(state: MultiFab, Vvac_max: float) -> float:
     """Evolve.cpp:22-89 (cfl factors from the context's parameters)."""
     g = state.view()
@@ -257,17 +279,22 @@ class Integrator:
     def rhs(self, F: FlavoredNeutrinoContainer, S: FlavoredNeutrinoContainer):
         deposit_to_mesh(S, self.state)                     # main.cpp:136
         self.state.FillBoundary()                          # main.cpp:137
-        F.copyParticles(S)                                 # main.cpp:148
-        interpolate_rhs_from_mesh(F, self.state)           # main.cpp:151
+        rhs_from_mesh(F, S, self.state)                    # main.cpp:148,151
 
     def advance(self):
         # each stage state and the result: copyParticles(old), then one
-        # ApplyFlavoredNeutrinoRHS per earlier stage -- one pass (rk_combine)
+        # ApplyFlavoredNeutrinoRHS per earlier stage -- one pass (rk_combine),
+        # which leaves out the stages whose coefficient is 0 (RK4's stage states
+        # have one other each: 7 right-hand sides read per step, not 10)
         dt = self.dt
+
+        def combine(row):
+            used = [j for j, a in enumerate(row) if a != 0.0]
+            self.new.rk_combine(self.old, [dt * row[j] for j in used], [self.F[j] for j in used])
         for i in range(len(self.B)):
-            self.new.rk_combine(self.old, [dt * a for a in self.A[i]], self.F[:len(self.A[i])])
+            combine(self.A[i])
             self.rhs(self.F[i], self.new)
-        self.new.rk_combine(self.old, [dt * b for b in self.B], self.F[:len(self.B)])
+        combine(self.B)
         self.time += dt
         self.step_number += 1
         # post_timestep_fun, main.cpp:155-199

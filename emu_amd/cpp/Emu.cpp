@@ -422,6 +422,15 @@ void FlavoredNeutrinoContainer::rk_combine(const FlavoredNeutrinoContainer& src,
               "copy ids");
 }
 
+void FlavoredNeutrinoContainer::rhs_of(const FlavoredNeutrinoContainer& src, const MultiFab& state)
+{
+    resize(src.np_);
+    if (np_ == 0) return;
+    emu_check(emu_rhs_from_mesh(geom_.ctx(), &view_, &src.view_, state.fab()), "interpolate_rhs_from_mesh", geom_.ctx());
+    hip_check(hipMemcpyAsync(ids_, src.ids_, (size_t)np_ * sizeof(int64_t), hipMemcpyDeviceToDevice, nullptr),
+              "copy ids");
+}
+
 void FlavoredNeutrinoContainer::SyncLocation(int type)
 {
     if (type != Sync::CoordinateToPosition && type != Sync::PositionToCoordinate) Abort("SyncLocation: bad type");
@@ -578,15 +587,24 @@ TimeIntegrator::~TimeIntegrator()
 void TimeIntegrator::advance(double dt)
 {
     // each stage state and the result: copyParticles(old) followed by one
-    // ApplyFlavoredNeutrinoRHS per earlier stage, as one pass (rk_combine)
-    double a[4];
+    // ApplyFlavoredNeutrinoRHS per earlier stage, as one pass (rk_combine), which
+    // leaves out the stages whose coefficient is 0
+    auto combine = [&](const double* row, int nrow) {
+        double a[4];
+        FlavoredNeutrinoContainer* used[4];
+        int n = 0;
+        for (int j = 0; j < nrow; j++)
+            if (row[j] != 0.0) {
+                a[n] = dt * row[j];
+                used[n++] = F_[j];
+            }
+        new_->rk_combine(*old_, n, a, used);
+    };
     for (int i = 0; i < tab_.nstages; i++) {
-        for (int j = 0; j < i; j++) a[j] = dt * tab_.A[i][j];
-        new_->rk_combine(*old_, i, a, F_.data());
+        combine(tab_.A[i], i);
         rhs_(*F_[i], *new_, time_ + tab_.c[i] * dt);
     }
-    for (int i = 0; i < tab_.nstages; i++) a[i] = dt * tab_.b[i];
-    new_->rk_combine(*old_, tab_.nstages, a, F_.data());
+    combine(tab_.b, tab_.nstages);
     time_ += dt;
 }
 
@@ -683,8 +701,7 @@ EvolveResult evolve_flavor(const TestParams* parms, const EvolveOptions& opt)
                               double /*time*/) {
             deposit_to_mesh(neutrinos, state, geom);
             state.FillBoundary(geom);
-            neutrinos_rhs.copyParticles(neutrinos, true);
-            interpolate_rhs_from_mesh(neutrinos_rhs, state, geom, parms);
+            neutrinos_rhs.rhs_of(neutrinos, state);
         };
         auto post_timestep_fun = [&]() {
             auto& neutrinos = integrator.get_new_data();

@@ -180,6 +180,8 @@ public:
     // copyParticles(src) followed by apply_rhs(a[j], *F[j]) for j < n, in one pass
     void rk_combine(const FlavoredNeutrinoContainer& src, int n, const double* a,
                     const FlavoredNeutrinoContainer* const* F);
+    // copyParticles(src) followed by interpolate_rhs_from_mesh on this container, in one call
+    void rhs_of(const FlavoredNeutrinoContainer& src, const MultiFab& state);
     // host copies (SoA, particle order), for output and restart
     void to_host(std::vector<double>& pos, std::vector<double>& rdata, std::vector<int64_t>& ids) const;
     void from_host(int64_t np, const std::vector<double>& pos, const std::vector<double>& rdata,

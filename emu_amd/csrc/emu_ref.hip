@@ -517,6 +517,17 @@ extern "C" int emu_interpolate_rhs_from_mesh(emu_ctx* ctx, emu_particles* rhs, c
     return box_run_batched(ctx, P, &P, fab, BoxCall::gather);
 }
 
+extern "C" int emu_rhs_from_mesh(emu_ctx* ctx, emu_particles* rhs, const emu_particles* src, const emu_grid* state)
+{
+    if (!ctx) return EMU_ERR_ARG;
+    Fab fab;
+    PView D, P;
+    if (!make_fab(ctx, state, fab) || !make_pview(ctx, rhs, D) || !make_pview(ctx, src, P) || D.np != P.np)
+        return set_error(ctx, EMU_ERR_ARG, "bad grid or particles");
+    if (P.np == 0) return EMU_OK;
+    return box_run_batched(ctx, P, &D, fab, BoxCall::gather);
+}
+
 extern "C" int emu_compute_dt(emu_ctx* ctx, const emu_grid* state, double Vvac_max, double* dt_out)
 {
     if (!ctx || !dt_out) return EMU_ERR_ARG;

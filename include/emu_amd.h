@@ -123,6 +123,12 @@ int emu_fill_boundary(emu_ctx* ctx, emu_grid* state);
  * attribute.  The grid's ghost cells must be filled. */
 int emu_interpolate_rhs_from_mesh(emu_ctx* ctx, emu_particles* rhs, const emu_grid* state);
 
+/* copyParticles(src) into rhs, then interpolate_rhs_from_mesh on it, in one
+ * call and bit for bit that sequence: the gather reads src and writes rhs, so
+ * the copy's pass over every attribute is spared.  rhs and src are distinct
+ * containers of as many particles (or the same one: the call above). */
+int emu_rhs_from_mesh(emu_ctx* ctx, emu_particles* rhs, const emu_particles* src, const emu_grid* state);
+
 /* compute_dt (Evolve.cpp:22-89) over the whole fab box, ghosts included.
  * Synchronous: writes *dt on the host. */
 int emu_compute_dt(emu_ctx* ctx, const emu_grid* state, double Vvac_max, double* dt);
