@@ -92,6 +92,20 @@ template <> struct Mfma16x16x4<double> {
     // lane of the result is group g: element r of lane l holds row 4r + l/16
     static __device__ __forceinline__ int group(int i) { return i >> 2; }
     static __device__ __forceinline__ int comp(int i) { return i & 3; }
+    // One component's four groups on the four-block form (16 cycles against 64): A's
+    // row l%4 is the group, B as above, the four blocks the quarters of the
+    // particles.  Lane l holds group l/16 of particle l%16: its term of the contraction.
+    typedef double tail_t;
+    static __device__ __forceinline__ tail_t tail_zero() { return 0.0; }
+    static __device__ __forceinline__ tail_t tail_step(double a, double b, tail_t c)
+    {
+        return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ double tail_term(tail_t d, int lane, double v0, double v1, double v2)
+    {
+        const int g = lane >> 4;
+        return (g == 0 ? 1.0 : (g == 1 ? v0 : (g == 2 ? v1 : v2))) * d;
+    }
 };
 template <> struct Mfma16x16x4<float> {
     typedef mf_f4 acc_t;
@@ -102,6 +116,20 @@ template <> struct Mfma16x16x4<float> {
     // element r of lane l holds row 4 (l/16) + r
     static __device__ __forceinline__ int group(int i) { return i & 3; }
     static __device__ __forceinline__ int comp(int i) { return i >> 2; }
+    // One component's four groups on the sixteen-block form (8 cycles against 32): A's
+    // row l%4 is the group, B as above, a block a neighbour (l/16) and a quarter of
+    // the particles.  Element g of lane l is group g of particle l%16 over the
+    // neighbours l/16, l/16 + 4, ..: a part of the sum.
+    typedef mf_f4 tail_t;
+    static __device__ __forceinline__ tail_t tail_zero() { return mf_f4{0.0f, 0.0f, 0.0f, 0.0f}; }
+    static __device__ __forceinline__ tail_t tail_step(float a, float b, tail_t c)
+    {
+        return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ float tail_term(tail_t d, int, float v0, float v1, float v2)
+    {
+        return d[0] + v0 * d[1] + v1 * d[2] + v2 * d[3];
+    }
 };
 
 // The gather of a wave's chunk of up to 64 particles on the matrix cores:
@@ -117,24 +145,39 @@ template <> struct Mfma16x16x4<float> {
 // another returns the results, without LDS.
 // LIN: the neighbours' rows follow each other in t, LIN values apart, and a row of
 // zeros (or any finite values) follows the last one.
-template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false, int LIN = 0> struct WaveGather {
+// BYITSELF: NF = 3's ninth component runs on the small blocks instead of a third tile
+// that is three quarters padding (per 16 particles 7 x 48 cycles less in FP64, 7 x 24
+// in FP32).  At 64^3 x 92, ms of stages 1 to 4: FP64 3.94 4.18 5.55 4.95 -> 3.87 4.04
+// 5.46 4.91.  FP32-bulk 2.70 2.61 3.24 3.12 -> 2.76 2.55 3.17 3.21: its offsets
+// cost stage 1 registers that it has not got (scratch memory) and stage 4 its fourth
+// wave per SIMD (134 registers, 125 without), so those two keep the third tile.
+template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false, int LIN = 0, bool BYITSELF = true> struct WaveGather {
     using MF = Mfma16x16x4<T>;
-    static constexpr int nh = NH<NF>, NT = WX * WY * WZ, KK = (NT + 3) / 4, MG = (nh + 3) / 4;
+    static constexpr int nh = NH<NF>, NT = WX * WY * WZ, KK = (NT + 3) / 4;
+    static constexpr bool TAIL = BYITSELF && nh % 4 == 1;
+    static constexpr int MG = TAIL ? nh / 4 : (nh + 3) / 4;
     // this lane's entry of A at step k, row i = l%16, neighbour t = 4k + l/16 (past
     // the last one: any in-range entry, its weight is zero; rows past NH feed
     // results that are dropped)
     // (LIN: step 0 only; PACK: two 16-bit offsets each, taken apart once per chunk)
     unsigned goff[LIN ? 1 : (PACK ? (KK + 1) / 2 : KK)];
+    int tail; // from there to the lane's entry of the last component
 
     // row(t): offset of neighbour t's row of fields
     __device__ __forceinline__ void init(int lane)
     {
         static_assert(LIN > 0, "rows at a constant distance");
         goff[0] = (lane >> 4) * LIN + MF::group(lane & 15) * nh + MF::comp(lane & 15);
+        set_tail(lane);
+    }
+    __device__ __forceinline__ void set_tail(int lane)
+    {
+        tail = ((lane & 3) - MF::group(lane & 15)) * nh + nh - 1 - MF::comp(lane & 15);
     }
     template <typename F> __device__ __forceinline__ void init(int lane, F&& row)
     {
         static_assert(LIN == 0, "rows anywhere");
+        set_tail(lane);
 #pragma unroll
         for (int k = 0; k < KK; k++) {
             const int t = 4 * k + (lane >> 4);
@@ -179,9 +222,11 @@ template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false, int LIN
 #pragma unroll
         for (int k = 0; k < KK; k++) transpose_rows(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
         // w[4 k + m] now holds tile m's operand of step k
-        T res[MG][4];
+        const int lane = threadIdx.x & 63;
+        T res[MG][4], last[4];
 #pragma unroll
         for (int m = 0; m < 4; m++) {
+            last[m] = T(0);
 #pragma unroll
             for (int c = 0; c < MG; c++) res[c][m] = T(0);
             if (m < ntile) {
@@ -191,10 +236,14 @@ template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false, int LIN
                 typename MF::acc_t acc[MG];
 #pragma unroll
                 for (int c = 0; c < MG; c++) acc[c] = typename MF::acc_t{T(0), T(0), T(0), T(0)};
+                typename MF::tail_t rest = MF::tail_zero();
 #pragma unroll
-                for (int k = 0; k < KK; k++)
+                for (int k = 0; k < KK; k++) {
 #pragma unroll
                     for (int c = 0; c < MG; c++) acc[c] = MF::step(G[off[k] + 4 * c], w[4 * k + m], acc[c]);
+                    if (TAIL) rest = MF::tail_step(G[off[k] + tail], w[4 * k + m], rest);
+                }
+                if (TAIL) last[m] = SIGN < 0 ? MF::tail_term(rest, lane, -v0, -v1, -v2) : MF::tail_term(rest, lane, v0, v1, v2);
 #pragma unroll
                 for (int c = 0; c < MG; c++)
                     res[c][m] = SIGN < 0 ? acc[c][0] - v0 * acc[c][1] - v1 * acc[c][2] - v2 * acc[c][3]
@@ -207,6 +256,10 @@ template <int NF, typename T, int WX, int WY, int WZ, bool PACK = false, int LIN
 #pragma unroll
             for (int j = 0; j < 4; j++)
                 if (4 * c + j < nh) out[4 * c + j] = res[c][j];
+        }
+        if (TAIL) { // the rows hold terms of one sum
+            transpose_rows(last[0], last[1], last[2], last[3]);
+            out[nh - 1] = (last[0] + last[1]) + (last[2] + last[3]);
         }
     }
 };
@@ -745,7 +798,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
             ptdx |= (unsigned)f[d] << (4 * (3 * m + d));
         }
     }
-    WaveGather<NF, T, WX, WY, WZ, PACK> gather;
+    WaveGather<NF, T, WX, WY, WZ, PACK, 0, sizeof(T) == 8 || s == 2 || s == 3> gather;
     if constexpr (s != 0) gather.init(lane, [&](int t) __attribute__((always_inline)) { return box_of(t) * QG; });
     // The last columns, when at most 8 remain past the 16-column tiles (NF = 3:
     // 36 = 2 x 16 + 4 without the auxiliaries, 39 = 2 x 16 + 7 with the
