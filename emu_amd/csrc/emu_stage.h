@@ -470,9 +470,9 @@ __device__ __forceinline__ int move1(int from, double x, double plo, double dxi,
 }
 
 // Ways to map waves to cells (MODE).
-//  0: every wave is its own patch of one cell (box = its 27 neighbours; two
-//     cells in FP32-bulk, below), stages its own box and flushes its deposit
-//     directly: no workgroup barrier.
+//  0: every wave is its own patch of two cells (below), stages its own box and
+//     flushes its deposit directly: no workgroup barrier.
+//  1: as 0 with one cell (box = its 27 neighbours).
 //  2: the WPB waves of a workgroup take a patch of WPB cells (2 along x, then
 //     2 along y, when the stencil is 3 wide there, else along z); the patch's
 //     neighbourhood box (PX + WX - 1) x (PY + WY - 1) x (PZ + WZ - 1) is staged
@@ -482,7 +482,7 @@ __device__ __forceinline__ int move1(int from, double x, double plo, double dxi,
 //  3: the WPB waves of a workgroup share one cell, 64 particles each in turn,
 //     with the box staged once and the deposits summed in LDS as in 2: for grids
 //     with too few cells to fill the chip and several chunks per cell.
-// PM (a shared patch) is MODE >= 2.  In MODE 0 a wave may also take CPW = 2
+// PM (a shared patch) is MODE >= 2.  In MODE 0 a wave takes CPW = 2
 // cells, x-adjacent, as one patch: their particles form one list of 16-particle
 // tiles (the first cell's, then the second's), so that a cell of 92 particles no
 // longer leaves 36 of a chunk's 64 lanes idle, and the wave stages the two
@@ -528,16 +528,16 @@ template <int NF, typename T, int AUX> constexpr int stage_lds_doubles_per_wave(
     return 64 * 9 + 64 * stage_source_row<NF>(AUX) * (int)sizeof(T) / 8;
 }
 
-// cells per wave: two in FP32-bulk's independent-wave launches of the 3-D
-// stencil (its 4 x 3 x 3 box still fits three waves per SIMD in LDS; FP64's
-// would not fit two)
-template <typename T, int WX, int MODE> constexpr int stage_cells_per_wave()
-{
-    return MODE == 0 && sizeof(T) == 4 && WX == 3 ? 2 : 1;
-}
+// cells per wave: MODE 0 takes two, side by side along x (emu_state::pairs says when)
+template <int MODE> constexpr int stage_cells_per_wave() { return MODE == 0 ? 2 : 1; }
+
+// whether MODE 0 is there at all: for the 3-D stencil, where the 4 x 3 x 3 box still
+// fits the waves per SIMD that the registers allow (three in FP32-bulk and for NF = 2;
+// FP64's NF = 3 would not fit two)
+template <int NF, typename T, int WX> constexpr bool stage_has_pairs() { return WX == 3 && (sizeof(T) == 4 || NF == 2); }
 
 template <typename T, int WX, int WY, int WZ, int WPB, int MODE>
-using StagePatch = Patch<WX, WY, WZ, (MODE == 2 ? WPB : stage_cells_per_wave<T, WX, MODE>())>;
+using StagePatch = Patch<WX, WY, WZ, (MODE == 2 ? WPB : stage_cells_per_wave<MODE>())>;
 
 // LDS of a workgroup, in doubles.  The tables of the box's cell indices (NB ints)
 // come first.  PM: then the staged neighbourhood box (gather stages, NB x 4 NH
@@ -563,9 +563,9 @@ constexpr int stage_lds_doubles_per_block()
 // NF = 3): the deposit-only launch in both precisions and FP32-bulk stage 4
 // merge their deposits (MODE 2); the other RK stages run faster with
 // independent waves
-template <typename T, int S, int AUX> constexpr int stage_mode()
+template <typename T, int S, int AUX> constexpr bool stage_merges()
 {
-    return S == 0 || (S == 4 && sizeof(T) == 4) ? 2 : 0;
+    return S == 0 || (S == 4 && sizeof(T) == 4);
 }
 // waves per workgroup: 4 (MODE 2 and 3); otherwise 2, or 1 for the launches
 // with the compute_dt auxiliaries, whose larger LDS rows would otherwise leave
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     const Geom& g = a.g;
     constexpr int s = S;
     constexpr bool aux = AUX != 0;
-    constexpr int CPW = stage_cells_per_wave<T, WX, MODE>();
+    constexpr int CPW = stage_cells_per_wave<MODE>();
     using PT = StagePatch<T, WX, WY, WZ, WPB, MODE>;
     constexpr int NB = PT::NB;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -689,16 +689,21 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     }
     if constexpr (s == 4) {
         // compute_dt's conservative bound (Evolve.cpp:40-56) of this wave's cell:
-        // N_ii and Nbar_ii from the auxiliaries S_ii and M_ii
+        // N_ii and Nbar_ii from the auxiliaries S_ii and M_ii (CPW = 2: the second
+        // cell's in the upper lanes)
         if (a.want_dt && owner) {
+            const int i = CPW == 2 ? lane & 31 : lane;
+            const bool second = CPW == 2 && lane >= 32;
             double v = 0.0;
-            if (lane < NF) {
-                const double M = a.gin[(int64_t)cell * QG + herm_re_rt<NF>(lane)] - (lane == 0 ? a.m00 : 0.0);
-                const double sum = a.aux[(int64_t)cell * NAUX + lane];
+            if (i < NF && (!second || inside1)) {
+                const int64_t c = cell + (second ? 1 : 0);
+                const double M = a.gin[c * QG + herm_re_rt<NF>(i)] - (i == 0 ? a.m00 : 0.0);
+                const double sum = a.aux[c * NAUX + i];
                 v = fmax(fmax(0.5 * (sum + M), 0.5 * (sum - M)), a.m00);
             }
             v = fmax(v, __shfl_xor(v, 1));
             if (NF == 3) v = fmax(v, __shfl_xor(v, 2));
+            if (CPW == 2) v = fmax(v, __shfl_xor(v, 32));
             if (lane == 0 && v > 0.0)
                 atomicMax(&a.red[DtRed::slot(blockIdx.x)],
                           (unsigned long long)__double_as_longlong(v * a.dtp.vst_scale));

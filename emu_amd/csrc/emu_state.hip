@@ -518,6 +518,7 @@ struct emu_state {
     int align = 1;
     int64_t cap = 1;
     bool split = false; // several waves per cell (k_stage's MODE 3)
+    bool pairs = false; // two cells per wave (MODE 0)
     // persistent arrays, two copies for the sort
     void* block[2] = {nullptr, nullptr};
     // scratch
@@ -588,6 +589,24 @@ bool split_cells(int64_t np, int64_t ncell, int precision)
     return (ncell <= at_once && np > 64 * ncell) || (ncell <= 2 * at_once && np > 160 * ncell);
 }
 
+// Whether a wave takes two cells (k_stage's MODE 0, where it is there): fewer
+// chunks are partly filled and neighbours' boxes overlap, but half as many waves run
+// at once.  From 3072 cells on, one per wave fills the chip (three waves per SIMD),
+// and in FP32-bulk the pairs win; FP64's NF = 2 has registers for fewer waves of
+// pairs, so there they pay only where two cells fill one chunk.  us per step, one
+// cell / two cells per wave, at 12, 26, 64 and 92 particles a cell:
+//   FP32-bulk NF = 2   8^3  55/57 57/62 63/78 -       12^3  71/72 78/78 87/100 103/124
+//                     16^3  96/95 101/105 114/125 145/155   24^3 245/235 265/253 317/304 419/409
+//             NF = 3   8^3  70/74 76/82 87/112 -      12^3 112/113 120/125 137/157 165/197
+//                     16^3 192/182 207/195 237/228 293/275  24^3 524/511 557/546 657/632 803/785
+//   FP64      NF = 2  12^3  77/79 85/89 98/122 122/159  16^3 120/106 130/115 155/155 207/194
+//                     24^3 291/277 314/311 405/448 569/647
+constexpr int64_t kPairCells = 3072;
+bool pair_cells(int64_t np, int64_t ncell, int precision)
+{
+    return ncell > kPairCells && (precision == EMU_FP32_BULK || np <= 32 * ncell);
+}
+
 template <typename T> Arrays<T> arrays_of(emu_state* st, int copy)
 {
     Arrays<T> A;
@@ -656,8 +675,19 @@ void launch_stage_mode(emu_state* st, StageArgs<T>& a)
 template <int NF, typename T, int WX, int WY, int WZ, int S, int AUX>
 void launch_stage_k(emu_state* st, StageArgs<T>& a)
 {
-    if (st->split) launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, 3>(st, a);
-    else launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, stage_mode<T, S, AUX>()>(st, a);
+    if (st->split) {
+        launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, 3>(st, a);
+    } else if constexpr (stage_merges<T, S, AUX>()) {
+        launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, 2>(st, a);
+    } else {
+        if constexpr (stage_has_pairs<NF, T, WX>()) {
+            if (st->pairs) {
+                launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, 0>(st, a);
+                return;
+            }
+        }
+        launch_stage_mode<NF, T, WX, WY, WZ, S, AUX, 1>(st, a);
+    }
 }
 
 template <int NF, typename T, int WX, int WY, int WZ>
@@ -851,6 +881,7 @@ extern "C" int emu_state_create(emu_ctx* ctx, int64_t np, int precision, emu_sta
     st->align = aligned ? a128 : 1;
     st->cap = std::max<int64_t>(np + st->ncell * (st->align - 1), 1);
     st->split = split_cells(np, st->ncell, precision);
+    st->pairs = pair_cells(np, st->ncell, precision);
     const int64_t npa = st->cap;
     const size_t pb = persistent_bytes(npa, st->nh, st->tsize);
     bool ok = hipMalloc(&st->block[0], pb) == hipSuccess && hipMalloc(&st->block[1], pb) == hipSuccess &&
