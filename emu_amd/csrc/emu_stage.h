@@ -327,6 +327,100 @@ __device__ __forceinline__ double advance_time(double t, double h)
     return t;
 }
 
+// ---------------------------------------------------------------------------
+// Stable counting sort by cell after each step.  A particle moves at most one
+// cell per dimension per step (c dt < dx, checked on the host), so its move
+// is one of 27 offsets e.  Particles arriving in cell t are ordered by the
+// canonical index of e, then by their position in their old cell: every
+// particle's destination is base[old cell][e] + (its rank among the particles
+// of its old cell with the same e), which makes the order deterministic.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ int wrap_cell(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
+
+// f(e, source) for every move e that exists on the grid (a 1-cell dimension
+// has only move 0, a 2-cell one 0 and +1), with the cell that particles come
+// from into cell t by it; canonical order of e.
+template <typename F> __device__ __forceinline__ void for_moves(int t, const Geom& g, F&& f)
+{
+    const int tx = t % g.n[0], ty = (t / g.n[0]) % g.n[1], tz = t / (g.n[0] * g.n[1]);
+#pragma unroll
+    for (int ez = -1; ez <= 1; ez++)
+#pragma unroll
+        for (int ey = -1; ey <= 1; ey++)
+#pragma unroll
+            for (int ex = -1; ex <= 1; ex++) {
+                const int ed[3] = {ex, ey, ez};
+                bool ok = true;
+#pragma unroll
+                for (int d = 0; d < 3; d++) ok = ok && !(g.n[d] == 1 && ed[d] != 0) && !(g.n[d] == 2 && ed[d] == -1);
+                if (!ok) continue;
+                const int sx = wrap_cell(tx - ex, g.n[0]), sy = wrap_cell(ty - ey, g.n[1]), sz = wrap_cell(tz - ez, g.n[2]);
+                f((ez + 1) * 9 + (ey + 1) * 3 + (ex + 1), ((int64_t)sz * g.n[1] + sy) * g.n[0] + sx);
+            }
+}
+
+// base[source][e] for every source of target t, in canonical move order, from
+// the target's first slot.
+__device__ __forceinline__ void write_bases(int t, int first, const int* __restrict__ m, const Geom& g, int* __restrict__ base)
+{
+    int run = first;
+    for_moves(t, g, [&](int e, int64_t src) {
+        base[src * 27 + e] = run;
+        run += m[src * 27 + e];
+    });
+}
+
+// The sort plan, between stage 1 (which counts the moves) and stage 4 (which needs the
+// bases), a lane per target cell: either by waves of its own at the front of the
+// stage 2 and stage 3 launches, or by two launches on a second stream (k_plan).
+struct SortPlan {
+    const int* m;  // mcount
+    int* start;    // first slot of each cell's run, a multiple of align
+    int* cnt;      // particles arriving in each cell; cnt[ncell] = 0 for the store's scan
+    int* sums;     // slots of each wave's cells
+    int* base;     // [ncell][27]
+    int align;
+    int per;       // 64-cell rows a wave takes
+    int waves;     // planning waves (per rows of 64 cells each cover 0 .. ncell)
+
+    // stage 2: the counts, and the starts counted from the wave's first slot
+    __device__ __forceinline__ void counts(int wave, int lane, const Geom& g, int ncell) const
+    {
+        int total = 0;
+        for (int j = 0; j < per; j++) {
+            const int t = (wave * per + j) * 64 + lane;
+            int n = 0;
+            if (t < ncell) for_moves(t, g, [&](int e, int64_t src) { n += m[src * 27 + e]; });
+            const int slots = (n + align - 1) / align * align;
+            int upto = slots; // inclusive scan over the lanes
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int o = __shfl_up(upto, off);
+                if (lane >= off) upto += o;
+            }
+            if (t <= ncell) cnt[t] = n;
+            if (t < ncell) start[t] = total + upto - slots;
+            total += __shfl(upto, 63);
+        }
+        if (lane == 0) sums[wave] = total;
+    }
+    // stage 3: the slots of the waves before complete the starts; the bases
+    __device__ __forceinline__ void bases(int wave, int lane, const Geom& g, int ncell) const
+    {
+        int before = 0;
+        for (int w = lane; w < wave; w += 64) before += sums[w];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off);
+        for (int j = 0; j < per; j++) {
+            const int t = (wave * per + j) * 64 + lane;
+            if (t >= ncell) return;
+            const int first = start[t] + before;
+            start[t] = first;
+            write_bases(t, first, m, g, base);
+        }
+    }
+};
+
 template <typename T> struct StageArgs {
     PArrays<T> cur; // current copy, sorted by cell_start
     PArrays<T> dst; // stage 4 writes the step's result here, sorted by the new cells
@@ -360,6 +454,8 @@ template <typename T> struct StageArgs {
     int stage; // 0 = deposit only, 1..4
     int want_aux;
     int blocks_per_xcd;
+    SortPlan plan;   // stages 2 and 3: planned by the first workgroups (none: no waves)
+    int plan_blocks; // a multiple of 8, so that the stage's own workgroups keep their XCDs
     Geom g;
     double vac[9]; // M2 c^4 / (2 hbar)
     double coef;   // sqrt2 GF / dV / hbar
@@ -613,10 +709,19 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(sizeof
     constexpr int NB = PT::NB;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
+    if constexpr (s == 2 || s == 3) {
+        if ((int)blockIdx.x < a.plan_blocks) { // the sort plan's waves
+            const int w = blockIdx.x * WPB + wave;
+            if (w >= a.plan.waves) return;
+            if (s == 2) a.plan.counts(w, lane, g, (int)a.ncell);
+            else a.plan.bases(w, lane, g, (int)a.ncell);
+            return;
+        }
+    }
     // blocks go round-robin over the 8 XCDs; give each XCD a contiguous run of patches
     const int npx = (g.n[0] + PT::PX - 1) / PT::PX, npy = (g.n[1] + PT::PY - 1) / PT::PY;
     const int npz = (g.n[2] + PT::PZ - 1) / PT::PZ;
-    const int b = blockIdx.x;
+    const int b = blockIdx.x - (s == 2 || s == 3 ? a.plan_blocks : 0);
     const int bgroup = (b & 7) * a.blocks_per_xcd + (b >> 3);
     // PM: the block's patch; otherwise this wave's patch of CPW cells, WPB consecutive per block
     const int patch = __builtin_amdgcn_readfirstlane(PM ? bgroup : bgroup * WPB + wave);

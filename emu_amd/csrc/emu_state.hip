@@ -50,96 +50,13 @@ __global__ void k_fill_grid(double* g, int64_t ncell, int Q, double m00, double*
     }
 }
 
-// ---------------------------------------------------------------------------
-// Stable counting sort by cell after each step.  A particle moves at most one
-// cell per dimension per step (c dt < dx, checked on the host), so its move
-// is one of 27 offsets e.  Particles arriving in cell t are ordered by the
-// canonical index of e, then by their position in their old cell: every
-// particle's destination is base[old cell][e] + (its rank among the particles
-// of its old cell with the same e), which makes the order deterministic.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int wrap_cell(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
-
-// f(e, source) for every move e that exists on the grid (a 1-cell dimension
-// has only move 0, a 2-cell one 0 and +1), with the cell that particles come
-// from into cell t by it; canonical order of e.
-template <typename F> __device__ __forceinline__ void for_moves(int t, const Geom& g, F&& f)
+// The sort plan by itself: its part of stage 2 or of stage 3.
+template <int S> __global__ __launch_bounds__(256) void k_plan(SortPlan plan, Geom g, int ncell)
 {
-    const int tx = t % g.n[0], ty = (t / g.n[0]) % g.n[1], tz = t / (g.n[0] * g.n[1]);
-#pragma unroll
-    for (int ez = -1; ez <= 1; ez++)
-#pragma unroll
-        for (int ey = -1; ey <= 1; ey++)
-#pragma unroll
-            for (int ex = -1; ex <= 1; ex++) {
-                const int ed[3] = {ex, ey, ez};
-                bool ok = true;
-#pragma unroll
-                for (int d = 0; d < 3; d++) ok = ok && !(g.n[d] == 1 && ed[d] != 0) && !(g.n[d] == 2 && ed[d] == -1);
-                if (!ok) continue;
-                const int sx = wrap_cell(tx - ex, g.n[0]), sy = wrap_cell(ty - ey, g.n[1]), sz = wrap_cell(tz - ez, g.n[2]);
-                f((ez + 1) * 9 + (ey + 1) * 3 + (ex + 1), ((int64_t)sz * g.n[1] + sy) * g.n[0] + sx);
-            }
-}
-
-constexpr int kPlanBlock = 256;
-
-// base[source][e] for every source of target t, in canonical move order, from
-// the target's first slot.
-__device__ __forceinline__ void write_bases(int t, int first, const int* __restrict__ m, const Geom& g, int* __restrict__ base)
-{
-    int run = first;
-    for_moves(t, g, [&](int e, int64_t src) {
-        base[src * 27 + e] = run;
-        run += m[src * 27 + e];
-    });
-}
-
-// The sort plan, first part, one thread per target cell: cnt[t] = particles
-// arriving in t; start[t] = the first slot of its run (a multiple of align),
-// counted from the block's first; bsum[b] = the block's slots.  cnt[ncell] = 0
-// for the store's scan.  A grid of one block is planned here in full.
-__global__ __launch_bounds__(kPlanBlock) void k_plan_counts(const int* __restrict__ m, Geom g, int ncell, int align,
-                                                            int* __restrict__ start, int* __restrict__ cnt,
-                                                            int* __restrict__ bsum, int* __restrict__ base)
-{
-    using Scan = hipcub::BlockScan<int, kPlanBlock>;
-    __shared__ typename Scan::TempStorage tmp;
-    const int t = blockIdx.x * kPlanBlock + threadIdx.x;
-    int n = 0;
-    if (t < ncell) for_moves(t, g, [&](int e, int64_t src) { n += m[src * 27 + e]; });
-    int first, total;
-    Scan(tmp).ExclusiveSum((n + align - 1) / align * align, first, total);
-    if (t <= ncell) cnt[t] = n;
-    if (t < ncell) start[t] = first;
-    if (gridDim.x > 1) {
-        if (threadIdx.x == 0) bsum[blockIdx.x] = total;
-    } else if (t < ncell) {
-        write_bases(t, first, m, g, base);
-    }
-}
-
-// The second part: every block sums the slots of the blocks before it (a few
-// thousand values at most), completes its cells' starts and writes the bases.
-// A scan kernel between the parts would be one more pass over the cells and two
-// more launches.
-__global__ __launch_bounds__(kPlanBlock) void k_plan_bases(const int* __restrict__ m, Geom g, int ncell,
-                                                           const int* __restrict__ bsum, int* __restrict__ start,
-                                                           int* __restrict__ base)
-{
-    using Reduce = hipcub::BlockReduce<int, kPlanBlock>;
-    __shared__ typename Reduce::TempStorage tmp;
-    __shared__ int before;
-    int s = 0;
-    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kPlanBlock) s += bsum[b];
-    s = Reduce(tmp).Sum(s);
-    if (threadIdx.x == 0) before = s;
-    __syncthreads();
-    const int t = blockIdx.x * kPlanBlock + threadIdx.x;
-    if (t >= ncell) return;
-    const int first = start[t] + before;
-    start[t] = first;
-    write_bases(t, first, m, g, base);
+    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (wave >= plan.waves) return;
+    if (S == 2) plan.counts(wave, lane, g, ncell);
+    else plan.bases(wave, lane, g, ncell);
 }
 
 template <typename T> using Arrays = PArrays<T>;
@@ -565,9 +482,18 @@ struct emu_state {
 
 namespace {
 
-// Up to here the plan's two small launches cost less in line than the event
-// pairs and the second stream that hide them.
+// Up to here the sort plan's waves ride on the launches of stages 2 and 3 (SortPlan).
+// Larger grids have the plan beside those stages on a second stream: there the two
+// launches and the event pair are small change, and planning waves at the front of
+// a stage keep its own from starting.  us per step, two launches (in line up to
+// 32^3, beside from 40^3 on) / riding:
+//   1 cell x 24 NF=2 FP64 30 / 28, 8^3 x 40 NF=2 FP32 60 / 46, 16^3 x 26 106 / 91,
+//   24^3 x 40 271 / 254, 32^3 x 92 892 / 880, NF=3 FP64 32^3 x 92 2467 / 2451;
+//   40^3 x 20 NF=2 FP32 958 / 966, 64^3 x 20 3608 / 3657, NF=3 FP32 8593 / 8737.
 constexpr int64_t kInlinePlanCells = 32768;
+// a planning wave takes a row of 64 cells, and more on grids of 2^17 cells and more,
+// so that the sums which each wave adds up stay about a thousand
+constexpr int64_t kPlanRowCells = 65536;
 
 // Whether four waves share a cell (k_stage's MODE 3): where the cells hold more
 // than one chunk of 64 particles each and are too few to fill the chip one (or,
@@ -657,6 +583,14 @@ int scan_counts(emu_state* st, const int* in, int* out, hipStream_t s = nullptr)
 }
 
 
+SortPlan sort_plan(const emu_state* st)
+{
+    SortPlan p{st->mcount, st->new_start, st->new_cnt, st->counts, st->mbase, st->align, 1, 0};
+    p.per = (int)std::max<int64_t>(1, st->ncell / kPlanRowCells);
+    p.waves = (int)(st->ncell / (64 * p.per) + 1); // cell ncell too
+    return p;
+}
+
 template <int NF, typename T, int WX, int WY, int WZ, int S, int AUX, int MODE>
 void launch_stage_mode(emu_state* st, StageArgs<T>& a)
 {
@@ -668,7 +602,8 @@ void launch_stage_mode(emu_state* st, StageArgs<T>& a)
     const int64_t nblk = MODE >= 2 ? npatch : (npatch + WPB - 1) / WPB;
     a.blocks_per_xcd = (int)((nblk + 7) / 8);
     const size_t lds = (size_t)stage_lds_doubles_per_block<NF, T, WX, WY, WZ, WPB, S, AUX, MODE>() * sizeof(double);
-    hipLaunchKernelGGL((k_stage<NF, T, WX, WY, WZ, WPB, S, AUX, MODE>), dim3((unsigned)(8 * a.blocks_per_xcd)),
+    a.plan_blocks = S == 2 || S == 3 ? ((a.plan.waves + WPB - 1) / WPB + 7) / 8 * 8 : 0;
+    hipLaunchKernelGGL((k_stage<NF, T, WX, WY, WZ, WPB, S, AUX, MODE>), dim3((unsigned)(a.plan_blocks + 8 * a.blocks_per_xcd)),
                        dim3(64 * WPB), lds, st->ctx->stream, a);
 }
 
@@ -789,6 +724,7 @@ StageArgs<T> stage_args(emu_state* st, int stage, const double* gin, double* gou
     // 2% slower with the diagonal sums alone (FP32-bulk's 1% faster).
     a.want_aux = x.want_aux ? (st->ctx->p.max_adaptive_speedup > 1 || sizeof(T) == 8 ? 2 : 1) : 0;
     a.blocks_per_xcd = 0;
+    a.plan = st->ncell <= kInlinePlanCells ? sort_plan(st) : SortPlan{};
     a.g = st->ctx->g;
     const emu_ctx* ctx = st->ctx;
     for (int c = 0; c < 9; c++) a.vac[c] = c < st->nh ? ctx->M2[c] * phys::c4 / 2.0 / phys::hbar : 0.0;
@@ -1107,7 +1043,6 @@ extern "C" int emu_state_evolve(emu_state* st, int nsteps, double fixed_dt)
     if (nsteps > 0) st->evolved = true;
     const bool flavor_dt = ctx->p.flavor_cfl_factor > 0.0 && fixed_dt <= 0;
     const bool adaptive = flavor_dt && ctx->p.max_adaptive_speedup > 1;
-    const int ncell = (int)st->ncell, plan_blocks = (ncell + kPlanBlock) / kPlanBlock; // a thread for cell ncell too
     const bool beside = st->ncell > kInlinePlanCells;
     for (int step = 0; step < nsteps; step++) {
         // the grids' turns: A holds the deposit of y_n, B is at its base, C free
@@ -1121,19 +1056,17 @@ extern "C" int emu_state_evolve(emu_state* st, int nsteps, double fixed_dt)
         x1.gclear = C;
         stage(1, A, B, x1); // also the moves over the step
         // the stable counting-sort plan by the new cell
-        hipStream_t ss = beside ? st->side : s;
         if (beside) {
+            const SortPlan plan = sort_plan(st);
+            const dim3 grid((unsigned)((plan.waves + 3) / 4)), block(256);
             EMU_HIP(ctx, hipEventRecord(st->ev_stage1, s));
-            EMU_HIP(ctx, hipStreamWaitEvent(ss, st->ev_stage1, 0));
+            EMU_HIP(ctx, hipStreamWaitEvent(st->side, st->ev_stage1, 0));
+            ev_record(st, 2, true, st->side);
+            hipLaunchKernelGGL(k_plan<2>, grid, block, 0, st->side, plan, g, (int)st->ncell);
+            hipLaunchKernelGGL(k_plan<3>, grid, block, 0, st->side, plan, g, (int)st->ncell);
+            ev_record(st, 2, false, st->side);
+            EMU_HIP(ctx, hipEventRecord(st->ev_plan, st->side));
         }
-        ev_record(st, 2, true, ss);
-        hipLaunchKernelGGL(k_plan_counts, dim3(plan_blocks), dim3(kPlanBlock), 0, ss, st->mcount, g, ncell, st->align,
-                           st->new_start, st->new_cnt, st->counts, st->mbase);
-        if (plan_blocks > 1)
-            hipLaunchKernelGGL(k_plan_bases, dim3(plan_blocks), dim3(kPlanBlock), 0, ss, st->mcount, g, ncell,
-                               st->counts, st->new_start, st->mbase);
-        ev_record(st, 2, false, ss);
-        if (beside) EMU_HIP(ctx, hipEventRecord(st->ev_plan, ss));
         x2.gclear = A;
         x2.clear_aux = flavor_dt;
         stage(2, B, C, x2);
