@@ -189,10 +189,11 @@ int emu_state_set_vvac_max(emu_state* st, double vvac_max);
 /* Write the state back (sorted order) with each particle's id.  Synchronous. */
 int emu_state_store(emu_state* st, emu_particles* parts, int64_t* ids);
 /* Advance nsteps RK4 steps (asynchronous; dt stays on the device between
- * steps).  A fixed_dt > 0 replaces compute_dt's value for every step.  Each
- * step's sort plan and compute_dt run on a second stream that the state owns,
- * forked from and joined back into the context's stream with events, so all of
- * a call's work is ordered before later work on the context's stream. */
+ * steps).  A fixed_dt > 0 replaces compute_dt's value for every step.  On grids
+ * of more than 32768 cells each step's sort plan runs on a second stream that
+ * the state owns, forked from and joined back into the context's stream with
+ * events, so all of a call's work is ordered before later work on the context's
+ * stream. */
 int emu_state_evolve(emu_state* st, int nsteps, double fixed_dt);
 /* Time, last dt, steps taken and the deferred status of the steps since load:
  * EMU_ERR_TRACE/NEGDIAG/LENGTH (Renormalize) or EMU_ERR_MOVE (a particle that
@@ -204,8 +205,10 @@ int emu_state_info(emu_state* st, double* time, double* dt, int64_t* steps, int6
  * clears earlier records). */
 int emu_state_profile(emu_state* st, int enable);
 /* Average milliseconds per launch of kernel class k (0 = stage kernels,
- * 1 = grid fills, 2 = cell sort, 3 = dt reduction) since profiling was
- * enabled.  Synchronous. */
+ * 1 = grid fills (none: the stages clear the grids), 2 = cell sort (on its own
+ * stream; none where it rides on the stages), 3 = dt reduction (with
+ * max_adaptive_speedup > 1; otherwise stage 4 does it)) since profiling was
+ * enabled; 0 without launches.  Synchronous. */
 int emu_state_kernel_ms(emu_state* st, int k, double* avg_ms, int64_t* launches);
 
 /* Diagnostic for growth rates: sums[0] = sum over cells of |N_01| and
