@@ -6,14 +6,16 @@
 //     update of the particle, then deposit of the next stage state into
 //     another grid; stage 1 also finds each particle's move over the step and
 //     its rank in it;
-//   a stable counting sort plan by the new cell (counts and bases);
+//   a stable counting sort plan by the new cell (counts beside stage 2, bases
+//     beside stage 3);
 //   stage 4 kernel: y_{n+1}, positions, periodic shift, Renormalize (FP64),
 //     each particle written straight to its slot in the new cell order; and
 //     compute_dt's maximum over the stage-4 deposit (main.cpp:193-197);
 //   the deposit of y_{n+1} that the next step's stage 1 reads; and the next dt.
-// Seven launches, or six where one workgroup plans the sort.  Three grids take
-// turns, so that each stage sets to its base the one that a later stage
-// deposits into, in the same launch.
+// Five launches, the plan riding on two of them, or seven on large grids, with
+// the plan's two on a second stream (kInlinePlanCells).  Three grids take turns,
+// so that each stage sets to its base the one that a later stage deposits into,
+// in the same launch.
 //
 // The mesh holds, per cell and flavour component c, the combined fields
 //   M_c  = N_c - conj(Nbar)_c  (+ rho Ye/Mp dV on 00, the matter term)
