@@ -22,7 +22,6 @@
 //   scatter (adjoint of the gather): LM_t += w_t(p) mu_p, LPhi_t -= w_t(p) v_p mu_p
 //   gather (adjoint of the deposit): Lq_p = sum_t w_t(p) (LM_t + v_p . LPhi_t)
 //   dL/df_p += N_p Lq_p;  dL/dfbar_p += sigma Nbar_p Lq_p;  dL/dNbar_p += sigma fbar_p . Lq_p
-#include "emu_cells.h"
 #include "emu_internal.h"
 #include "emu_stage.h"
 #include "../../include/emu_adjoint.h"
@@ -209,8 +208,7 @@ template <typename F> __device__ __forceinline__ void for_each_wave_key(bool act
     }
 }
 
-// np particles whose coordinates lie pitch doubles apart.
-__global__ void k_cell_keys(int64_t np, int64_t pitch, const double* pos, Geom g, int* key, int* counts)
+__global__ void k_cell_keys(int64_t np, const double* pos, Geom g, int* key, int* counts)
 {
     const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const bool act = p < np;
@@ -222,7 +220,7 @@ __global__ void k_cell_keys(int64_t np, int64_t pitch, const double* pos, Geom g
         for (int d = 0; d < 3; d++) {
             int idx;
             double w[3];
-            shape3((pos[d * pitch + p] - g.plo[d]) * g.dxi[d], g.order[d], idx, w);
+            shape3((pos[d * np + p] - g.plo[d]) * g.dxi[d], g.order[d], idx, w);
             c[d] = pmod(idx, g.n[d]);
         }
         k = (c[2] * g.n[1] + c[1]) * g.n[0] + c[0];
@@ -279,6 +277,72 @@ __global__ __launch_bounds__(256) void k_vjp_gather(AdjIn in, Geom g, const int*
             ln += sg * in.Y[(int64_t)(nh + c) * np + p] * lq[c];
         }
         if (lamNbar) lamNbar[p] += ln;
+    }
+}
+
+// Objective J = sum over cells of |N_01|^2 with N_01 = sum_p w N f01 (nu), without a
+// cell list (objective_deposit says when).  One thread per particle; the lanes of
+// a wave whose stencils share a centre cell (one or two such groups per wave in
+// cell order) sum each target's contribution across the wave before one atomic
+// per target and component: per-particle atomics would put every particle of a
+// cell on the same 27 targets.
+__device__ __forceinline__ double wave_sum(double v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    return v;
+}
+
+template <int NF, typename T>
+__global__ __launch_bounds__(256) void k_obj_deposit_unlisted(AdjInT<T> in, Geom g, double* g2)
+{
+    const int64_t np = in.np;
+    const int lane = threadIdx.x & 63;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    // p0 is the wave's first particle, so the loop bound is the same for all its lanes
+    for (int64_t p0 = blockIdx.x * (int64_t)blockDim.x + (threadIdx.x & ~63); p0 < np; p0 += stride) {
+        const int64_t p = p0 + lane;
+        const bool act = p < np;
+        int c[3] = {0, 0, 0};
+        double wd[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+        double re = 0.0, im = 0.0;
+        if (act) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                int idx;
+                shape3((in.pos[d * np + p] - g.plo[d]) * g.dxi[d], g.order[d], idx, wd[d]);
+                c[d] = pmod(idx, g.n[d]);
+            }
+            const double N = in.Nn[p];
+            re = N * double(in.Y[(int64_t)herm_re<NF>(0, 1) * np + p]);
+            im = N * double(in.Y[(int64_t)herm_im<NF>(0, 1) * np + p]);
+        }
+        const int key = (c[2] * g.n[1] + c[1]) * g.n[0] + c[0];
+        for_each_wave_key(act, key, [&](int k, unsigned long long m, int lead) {
+            const bool mine = (m >> lane) & 1ull;
+            const int kx = k % g.n[0], ky = (k / g.n[0]) % g.n[1], kz = k / (g.n[0] * g.n[1]);
+#pragma unroll
+            for (int kk = 0; kk < 3; kk++) {
+                if (g.order[2] == 0 && kk != 1) continue;
+                const int tz = pmod(kz + kk - 1, g.n[2]);
+#pragma unroll
+                for (int jj = 0; jj < 3; jj++) {
+                    if (g.order[1] == 0 && jj != 1) continue;
+                    const int ty = pmod(ky + jj - 1, g.n[1]);
+#pragma unroll
+                    for (int ii = 0; ii < 3; ii++) {
+                        if (g.order[0] == 0 && ii != 1) continue;
+                        const int64_t t = ((int64_t)tz * g.n[1] + ty) * g.n[0] + pmod(kx + ii - 1, g.n[0]);
+                        const double w = wd[0][ii] * wd[1][jj] * wd[2][kk];
+                        const double a = wave_sum(mine ? w * re : 0.0), b = wave_sum(mine ? w * im : 0.0);
+                        if (lane == lead) {
+                            unsafeAtomicAdd(&g2[2 * t], a);
+                            unsafeAtomicAdd(&g2[2 * t + 1], b);
+                        }
+                    }
+                }
+            }
+        });
     }
 }
 
@@ -575,8 +639,7 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_cell_deposit(AdjInT<T> in, 
 }
 
 
-// Objective J = sum over cells of |N_01|^2 with N_01 = sum_p w N f01 (nu), one cell
-// per wave: a lane sums its particles' contributions to the 27 targets in registers,
+// The objective's deposit through a cell list, one cell per wave: a lane sums its particles' contributions to the 27 targets in registers,
 // the wave adds the lanes up (transposing as it goes: 16 row transposes, then four
 // steps that halve the values a lane holds, so that lane l ends with value l), and
 // one atomic instruction adds the cell's 54 values to the grid.
@@ -1231,21 +1294,17 @@ static void cell_deposit(emu_ctx* ctx, const AdjInT<T>& in, const CellSort& cs, 
 
 // the particles listed by the centre cell of their stencil (positions are
 // frozen within a step, so every deposit of a call shares one list)
-static int cell_sort(emu_ctx* ctx, int64_t np, int64_t pitch, const double* pos, const CellSort& cs)
+template <typename T> static int cell_sort(emu_ctx* ctx, const AdjInT<T>& in, const CellSort& cs)
 {
-    const int64_t nc = ncell_of(ctx);
+    const int64_t np = in.np, nc = ncell_of(ctx);
     const int64_t zero_doubles = (2 * nc + 1 + 1) / 2; // start and cursor are adjacent ints
     hipLaunchKernelGGL(k_zero, dim3(nblk(zero_doubles)), dim3(kB), 0, ctx->stream, (double*)cs.start, zero_doubles);
     const unsigned nb = (unsigned)((np + kB - 1) / kB); // one thread per particle
-    hipLaunchKernelGGL(k_cell_keys, dim3(nb), dim3(kB), 0, ctx->stream, np, pitch, pos, ctx->g, cs.key, cs.start);
+    hipLaunchKernelGGL(k_cell_keys, dim3(nb), dim3(kB), 0, ctx->stream, np, in.pos, ctx->g, cs.key, cs.start);
     size_t bytes = cs.tmp_bytes;
     EMU_HIP(ctx, hipcub::DeviceScan::ExclusiveSum(cs.tmp, bytes, cs.start, cs.start, (int)(nc + 1), ctx->stream));
     hipLaunchKernelGGL(k_cell_perm, dim3(nb), dim3(kB), 0, ctx->stream, np, cs.key, cs.start, cs.cursor, cs.perm);
     return EMU_OK;
-}
-template <typename T> static int cell_sort(emu_ctx* ctx, const AdjInT<T>& in, const CellSort& cs)
-{
-    return cell_sort(ctx, in.np, in.np, in.pos, cs);
 }
 
 // the deposit of Y onto the base grid (matter in component 0, carrying the
@@ -1302,31 +1361,36 @@ extern "C" int emu_adj_rhs_vjp(emu_ctx* ctx, int64_t np, const double* pos, cons
     return EMU_OK;
 }
 
-// The cell list in the context's scratch, for a batch of particles at a time: 2^25,
-// or fewer where that does not fit beside what the caller holds.
-template <typename T> static int objective_deposit(emu_ctx* ctx, const AdjInT<T>& in, double* g2)
+// The objective's deposit, through a cell list where dJdY has the room for one (it is
+// written last, and each of its particles takes 4 to 18 times the list's 8 bytes):
+// the call works in the caller's memory alone, so that nothing of it is shared with
+// calls on other streams and it cannot run out of memory.  Without dJdY, with many
+// more cells than particles, or with dJdY over Y (which the deposit still reads) the
+// particles go one per thread.  3.0 M particles in 32^3 cells, NF = 2, FP64, four
+// steps after they were last in cell order: 0.20 ms with the list, 2.24 ms without.
+template <typename T> static int objective_deposit(emu_ctx* ctx, const AdjInT<T>& in, T* dJdY, double* g2)
 {
-    const int64_t nc = ncell_of(ctx);
-    const int bpx = cell_blocks_per_xcd(nc);
-    int64_t batch = std::min(in.np, int64_t(1) << 25);
-    void* scratch = nullptr;
-    while (batch > 0) {
-        const int e = box_scratch(ctx, sizeof(double) * (size_t)cell_sort_doubles(ctx, batch), &scratch);
-        if (e == EMU_OK) break;
-        if (batch < 1 << 16) return e;
-        batch /= 2;
-    }
-    for (int64_t at = 0; at < in.np; at += batch) {
-        const int64_t n = std::min(batch, in.np - at);
-        const AdjInT<T> part{in.np, in.pos + at, nullptr, in.Nn + at, in.Y + at};
-        const CellSort cs = cell_sort_at(ctx, n, (double*)scratch);
-        if (int e = cell_sort(ctx, n, in.np, part.pos, cs)) return e;
+    const int64_t np = in.np, nc = ncell_of(ctx);
+    if (np == 0) return EMU_OK;
+    const uintptr_t rows = (uintptr_t)(2 * ctx->p.nf * ctx->p.nf * np) * sizeof(T); // bytes of Y and of dJdY
+    const uintptr_t beg = (uintptr_t)dJdY, y = (uintptr_t)in.Y;
+    const bool apart = beg + rows <= y || y + rows <= beg;
+    const uintptr_t region = (beg + 255) & ~(uintptr_t)255;
+    if (dJdY && apart && np <= INT32_MAX &&
+        region + sizeof(double) * (uintptr_t)cell_sort_doubles(ctx, np) <= beg + rows) {
+        const int bpx = cell_blocks_per_xcd(nc);
+        const CellSort cs = cell_sort_at(ctx, np, (double*)region);
+        if (int e = cell_sort(ctx, in, cs)) return e;
         if (ctx->p.nf == 2)
-            hipLaunchKernelGGL((k_obj_deposit<2, T>), dim3(8 * bpx), dim3(64 * kCellWaves), 0, ctx->stream, part, ctx->g,
+            hipLaunchKernelGGL((k_obj_deposit<2, T>), dim3(8 * bpx), dim3(64 * kCellWaves), 0, ctx->stream, in, ctx->g,
                                cs.start, cs.perm, nc, bpx, g2);
         else
-            hipLaunchKernelGGL((k_obj_deposit<3, T>), dim3(8 * bpx), dim3(64 * kCellWaves), 0, ctx->stream, part, ctx->g,
+            hipLaunchKernelGGL((k_obj_deposit<3, T>), dim3(8 * bpx), dim3(64 * kCellWaves), 0, ctx->stream, in, ctx->g,
                                cs.start, cs.perm, nc, bpx, g2);
+    } else if (ctx->p.nf == 2) {
+        hipLaunchKernelGGL((k_obj_deposit_unlisted<2, T>), dim3(nblk(np)), dim3(kB), 0, ctx->stream, in, ctx->g, g2);
+    } else {
+        hipLaunchKernelGGL((k_obj_deposit_unlisted<3, T>), dim3(nblk(np)), dim3(kB), 0, ctx->stream, in, ctx->g, g2);
     }
     return EMU_OK;
 }
@@ -1341,7 +1405,7 @@ static int adj_objective(emu_ctx* ctx, int64_t np, const double* pos, const T* N
     double* g2 = work; // [ncell][2] N_01, then J
     double* dJ = g2 + 2 * nc;
     hipLaunchKernelGGL(k_zero, dim3(nblk(2 * nc + 1)), dim3(kB), 0, ctx->stream, g2, 2 * nc + 1);
-    if (int e = objective_deposit<T>(ctx, in, g2)) return e;
+    if (int e = objective_deposit<T>(ctx, in, dJdY, g2)) return e;
     hipLaunchKernelGGL(k_obj_sum, dim3(nblk(nc)), dim3(kB), 0, ctx->stream, g2, nc, dJ);
     if (dJdY && np > 0) {
         if (ctx->p.nf == 2)

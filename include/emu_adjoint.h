@@ -32,7 +32,9 @@ int emu_adj_rhs_vjp(emu_ctx* ctx, int64_t np, const double* pos, const double* p
 
 /* J = sum over cells of |N_01|^2, N_01 = sum_p w N f01 (the nu part of the
  * N01 grid components); dJdY (optional) receives dJ/dY.  'work': 2 ncell + 1
- * doubles at least (either work array of this header).  Synchronous. */
+ * doubles at least (either work array of this header).  Works in 'work' and
+ * dJdY alone; with dJdY (not in place of Y) the sum over the particles is
+ * several times faster.  Synchronous. */
 int emu_adj_objective(emu_ctx* ctx, int64_t np, const double* pos, const double* Nn, const double* Y, double* J,
                       double* dJdY, double* work);
 
