@@ -433,10 +433,17 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Whether neighbour t (of 27) is part of the stencil: in a dimension of shape order 0
+// only the centre is.  The others have weight 0, which a field that is not finite
+// would turn into NaN: they are left out of the products and of the deposits.
+__device__ __forceinline__ bool in_stencil(const Geom& g, int t)
+{
+    return (g.order[0] > 0 || t % 3 == 1) && (g.order[1] > 0 || (t / 3) % 3 == 1) && (g.order[2] > 0 || t / 9 == 1);
+}
+
 // A wave's copy of its cell's neighbourhood in LDS: 27 rows of 4 NH fields in T
-// (the FP32 form rounds the FP64 grid here), then a row of zeros that the gather's
-// last step reads with zero weights.  In a dimension of shape order 0 the weights
-// are (0, 1, 0), so the other rows do not count.
+// (the FP32 form rounds the FP64 grid here; zeros where the stencil has no cell),
+// then a row of zeros that the gather's last step reads with zero weights.
 // The gather read the grid through scalar loads before (one neighbour's fields at a
 // time, every lane the same ones), a chain of 27 loads per chunk with nothing else
 // for the wave to do: on 32^3 cells x 92 particles, 2 flavours in FP64, a stage took
@@ -445,7 +452,7 @@ template <int NF, typename T> struct CellBox {
     static constexpr int QG = 4 * NH<NF>, N = 28 * QG;
     using Gather = WaveGather<NF, T, 3, 3, 3, false, QG>;
 
-    // index of the neighbours' cells, for lanes 0..26 of the wave
+    // index of the neighbours' cells (-1: not in the stencil), for lanes 0..26 of the wave
     static __device__ __forceinline__ void table(const Geom& g, int cell, int lane, int* ctab)
     {
         if (lane < 27) {
@@ -453,7 +460,7 @@ template <int NF, typename T> struct CellBox {
             const int x = wrap(cell % g.n[0] + lane % 3 - 1, g.n[0]);
             const int y = wrap((cell / g.n[0]) % g.n[1] + (lane / 3) % 3 - 1, g.n[1]);
             const int z = wrap(cell / (g.n[0] * g.n[1]) + lane / 9 - 1, g.n[2]);
-            ctab[lane] = (z * g.n[1] + y) * g.n[0] + x;
+            ctab[lane] = in_stencil(g, lane) ? (z * g.n[1] + y) * g.n[0] + x : -1;
         }
     }
     // (after table and a wave_sync; followed by a wave_sync)
@@ -462,8 +469,13 @@ template <int NF, typename T> struct CellBox {
 #pragma unroll
         for (int e0 = 0; e0 < N; e0 += 64) {
             const int e = e0 + lane;
-            if (e < 27 * QG) box[e] = T(grid[(int64_t)ctab[e / QG] * QG + e % QG]);
-            else if (e < N) box[e] = T(0);
+            if (e < 27 * QG) {
+                const int c = ctab[e / QG];
+                const double v = grid[(int64_t)max(c, 0) * QG + e % QG];
+                box[e] = c < 0 ? T(0) : T(v);
+            } else if (e < N) {
+                box[e] = T(0);
+            }
         }
     }
 };
@@ -693,10 +705,8 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_obj_deposit(AdjInT<T> in, G
             v[e] = keep + __shfl_xor(send, h);
         }
     wave_sync();
-    const int t = lane >> 1; // targets off the centre in a dimension of order 0 take no part
-    const bool in_shape = (g.order[0] > 0 || t % 3 == 1) && (g.order[1] > 0 || (t / 3) % 3 == 1) &&
-                          (g.order[2] > 0 || t / 9 == 1);
-    if (t < 27 && in_shape) unsafeAtomicAdd(&g2[2 * (int64_t)ctab[t] + (lane & 1)], v[0]);
+    const int t = lane >> 1;
+    if (t < 27 && ctab[t] >= 0) unsafeAtomicAdd(&g2[2 * (int64_t)ctab[t] + (lane & 1)], v[0]);
 }
 
 // A wave's deposit of its cell's particles on the f64 matrix cores, a chunk
@@ -812,7 +822,7 @@ template <int NF> struct WaveDeposit {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int t = 16 * m + 4 * r + (lane >> 4);
-                if (t >= NT) continue;
+                if (t >= NT || !in_stencil(g, t)) continue;
                 double* Gd = target(t);
 #pragma unroll
                 for (int n = 0; n < NTF; n++) unsafeAtomicAdd(&Gd[16 * n + (lane & 15)], acc[m][n][r]);
@@ -823,7 +833,7 @@ template <int NF> struct WaveDeposit {
 #pragma unroll
             for (int k = 0; k < NSM; k++) {
                 const int t = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4), q = 16 * NTF + 4 * k + (lane & 3);
-                if (t >= NT || q >= QG) continue;
+                if (t >= NT || q >= QG || !in_stencil(g, t)) continue;
                 unsafeAtomicAdd(&target(t)[q], accs[m][k]);
             }
     }
@@ -1000,8 +1010,8 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
 // moves at 3.0 M particles, 2 flavours, FP64: 235 us of the 501 us it takes; two
 // gathers' and a deposit's matrix instructions do not overlap with the rest at the
 // two waves per SIMD that its registers allow.  Every
-// stencil width runs the 3 x 3 x 3 target set (the weights of an order-0
-// dimension are (0, 1, 0), so its other targets receive zeros).
+// stencil width runs the 3 x 3 x 3 target set (in_stencil: an order-0 dimension's
+// other targets take no part).
 template <int NF, typename T, bool G, bool C>
 __global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void k_vjp_fused(
     AdjInT<T> in, Geom g, const int* start, const int* perm, int64_t ncell, int bpx, const T* Ynext, const T* Ycur,
