@@ -875,22 +875,33 @@ int box_list_and_run(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& 
 }
 
 // Runs the call in batches of particles (the deposit adds up, the gather is
-// per particle), so that the scratch stays bounded: kBoxBatch particles, or
-// fewer where that does not fit beside what the caller holds.
+// per particle), so that the scratch stays bounded: kBoxBatch particles (6.7 GB in
+// the deposit at NF = 3), or fewer where that is more than a quarter of the device
+// memory that is free (the scratch stays with the context, and the caller's next
+// allocation needs room too) or cannot be had.  Each batch walks all boxes: at 64^3 x
+// 92, NF = 3, in batches of 2^25, 2^23, 2^22 and 2^21 the deposit takes 4.5 5.4 6.7 9.5
+// ms in box order and 7.1 7.7 9.2 11.5 three cells on, the gather 4.2 4.7 5.0 6.9 and 6.7
+// 6.9 8.3 9.6.  So a call that holds too little for its particles asks for more again.
 constexpr int64_t kBoxBatch = int64_t(1) << 25, kBoxBatchMin = int64_t(1) << 16;
+constexpr size_t kScratchShare = 4;
 
 int box_run_batched(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& fab, BoxCall call)
 {
-    if (ctx->box_batch == 0) ctx->box_batch = kBoxBatch;
+    auto size = [&](int64_t n) { return box_scratch_size(n, fab.cstride, ctx->p.nf, call).total; };
+    int64_t batch = std::min(P.np, kBoxBatch);
+    size_t need = size(batch);
+    if (need > ctx->box_scratch_bytes) {
+        size_t free = 0, total = 0;
+        const bool known = hipMemGetInfo(&free, &total) == hipSuccess;
+        const size_t most = std::max((free + ctx->box_scratch_bytes) / kScratchShare, ctx->box_scratch_bytes);
+        while (known && batch / 2 >= kBoxBatchMin && need > most) need = size(batch /= 2);
+    }
     void* scratch = nullptr;
-    size_t need = 0;
     for (;;) {
-        need = box_scratch_size(std::min(P.np, ctx->box_batch), fab.cstride, ctx->p.nf, call).total;
         const int e = box_scratch(ctx, need, &scratch);
         if (e == EMU_OK) break;
-        const int64_t half = std::min(P.np, ctx->box_batch) / 2;
-        if (half < kBoxBatchMin) return e;
-        ctx->box_batch = half;
+        if (batch / 2 < kBoxBatchMin) return e;
+        need = size(batch /= 2);
     }
     auto part = [](const PView& V, int64_t at, int64_t n) {
         PView p = V;
@@ -903,7 +914,7 @@ int box_run_batched(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& f
     };
     int64_t at = 0;
     do {
-        const int64_t n = std::min(P.np - at, ctx->box_batch);
+        const int64_t n = std::min(P.np - at, batch);
         const PView Pp = part(P, at, n), Dp = dst ? part(*dst, at, n) : PView{};
         const int e = box_list_and_run(ctx, Pp, dst ? &Dp : nullptr, fab, call, scratch, need);
         if (e != EMU_OK) return e;

@@ -75,7 +75,6 @@ struct emu_ctx {
     unsigned long long* d_red = nullptr; // reduction scratch (8 slots)
     void* box_scratch = nullptr;         // per-function deposit/gather: box list, records, combined fields
     size_t box_scratch_bytes = 0;
-    int64_t box_batch = 0;               // particles per batch of those calls (0: not set yet)
     bool adj_status_armed = false;       // d_red[5] holds the adjoint steps' deferred status
     std::string err;
 };

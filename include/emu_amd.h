@@ -103,7 +103,11 @@ int emu_grid_ngrow(const emu_ctx* ctx, int ngrow[3]);
 /* deposit_to_mesh (Evolve.cpp:91-126 via amrex::ParticleToMesh): zero the
  * deposit components over valid+ghost cells, deposit N f and N f p/pt with the
  * shape factors, fold ghost deposits onto their periodic images (SumBoundary;
- * ghosts keep their partial sums). */
+ * ghosts keep their partial sums).
+ * This call and the two gathers below keep device scratch in the context until
+ * emu_destroy, for 2^25 particles at most (56 + 16 NF^2 bytes each) and
+ * the grid's combined fields, and not more than a quarter of the memory that was
+ * free when it was taken: with less, they go through the particles in batches. */
 int emu_deposit_to_mesh(emu_ctx* ctx, const emu_particles* parts, emu_grid* state);
 
 /* emu_deposit_to_mesh without any allocation.  No counterpart in the
