@@ -887,6 +887,7 @@ constexpr size_t kScratchShare = 4;
 
 int box_run_batched(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& fab, BoxCall call)
 {
+    if (P.np > (int64_t)INT32_MAX) return set_error(ctx, EMU_ERR_UNSUPPORTED, "more than 2^31 particles or fab cells");
     auto size = [&](int64_t n) { return box_scratch_size(n, fab.cstride, ctx->p.nf, call).total; };
     int64_t batch = std::min(P.np, kBoxBatch);
     size_t need = size(batch);
