@@ -511,6 +511,15 @@ constexpr int64_t kPlanRowCells = 65536;
 //   FP64       8^3        x 92: 132 / 113   x 378: 329 / 211
 //              1024 (1-D) x 92:  97 / 110   x 200: 164 / 140
 //              12^3       x 92: 204 / 309   x 378: 563 / 634
+// and NF = 2, on the same side at each of these, which differ by less where they cross:
+//   FP32-bulk  4^3        x 66:  56 / 44    x 378: 131 / 62
+//              8^3        x 66:  59 / 50    x 378: 144 / 86
+//              10^3       x 66:  70 / 60    x 378: 182 / 117
+//              12^3       x 92:  82 / 108   x 200: 136 / 124
+//   FP64       8^3        x 66:  61 / 55    x 378: 162 / 105
+//              1024 (1-D) x 92:  59 / 55    x 200: 104 / 76
+//              10^3       x 92:  84 / 87    x 200: 140 / 108
+//              12^3       x 92:  96 / 133   x 378: 264 / 262
 bool split_cells(int64_t np, int64_t ncell, int precision)
 {
     const int64_t at_once = precision == EMU_FP32_BULK ? 1024 : 768;
@@ -529,10 +538,19 @@ bool split_cells(int64_t np, int64_t ncell, int precision)
 //                     16^3 192/182 207/195 237/228 293/275  24^3 524/511 557/546 657/632 803/785
 //   FP64      NF = 2  12^3  77/79 85/89 98/122 122/159  16^3 120/106 130/115 155/155 207/194
 //                     24^3 291/277 314/311 405/448 569/647
+// A domain of one column has no pairs to take: a wave's second cell would be empty and
+// its box 36 rows instead of 27.  Narrow odd domains, whose last column goes by itself,
+// gain less, but lose only where the waves of pairs just miss the last full round:
+//   FP64      NF = 2   at 12, 26, 31   1x64x64 152/166 165/176 164/182    3x33x33 93/90 103/103 104/105
+//                     3x64x64 242/239 267/262 266/264    5x32x32 123/120 133/140 135/143
+//   FP32-bulk NF = 2   at 26, 92   1x64x64 141/142 195/194    3x33x33 88/87 129/148    3x64x64 227/216 363/362
+//                     5x32x32 109/109 171/167
+//             NF = 3   1x64x64 213/222 310/322    1x160x160 1115/1148 1596/1652    3x33x33 164/166 252/261
+//                     3x64x64 476/470 711/701    5x32x32 216/217 319/316
 constexpr int64_t kPairCells = 3072;
-bool pair_cells(int64_t np, int64_t ncell, int precision)
+bool pair_cells(const Geom& g, int64_t np, int64_t ncell, int precision)
 {
-    return ncell > kPairCells && (precision == EMU_FP32_BULK || np <= 32 * ncell);
+    return g.n[0] > 1 && ncell > kPairCells && (precision == EMU_FP32_BULK || np <= 32 * ncell);
 }
 
 template <typename T> Arrays<T> arrays_of(emu_state* st, int copy)
@@ -819,7 +837,7 @@ extern "C" int emu_state_create(emu_ctx* ctx, int64_t np, int precision, emu_sta
     st->align = aligned ? a128 : 1;
     st->cap = std::max<int64_t>(np + st->ncell * (st->align - 1), 1);
     st->split = split_cells(np, st->ncell, precision);
-    st->pairs = pair_cells(np, st->ncell, precision);
+    st->pairs = pair_cells(ctx->g, np, st->ncell, precision);
     const int64_t npa = st->cap;
     const size_t pb = persistent_bytes(npa, st->nh, st->tsize);
     bool ok = hipMalloc(&st->block[0], pb) == hipSuccess && hipMalloc(&st->block[1], pb) == hipSuccess &&
