@@ -74,9 +74,11 @@ __device__ __forceinline__ bool particle_box(const PView& P, int64_t ip, const F
 // trip.  Grouping every box with an atomic inside the loop, and again in a
 // second pass for the permutation, took up to 64 round trips per wave on
 // scattered particles (0.17 + 0.36 ms per list of 3.0 M; this pass 0.11 ms, bound
-// by the atomics themselves).  Sampled blocks add their waves' boxes (the groups
-// and the single lanes) to counts[nk + 2], the measure of how scattered the
-// arrays are.
+// by the atomics themselves).  One wave of each sampled block (in turn, so that no
+// period of the arrays decides) adds its boxes (the groups and the single lanes) to
+// counts[nk + 2], the measure of how scattered the arrays are: 256 atomics on that
+// word at most, as they queue for it (with all four waves' the pass took 14.4 us for
+// 387k particles in order, 6.0 now).
 constexpr int kGroups = 8;
 
 __global__ __launch_bounds__(kB) void k_box_rank(PView P, Fab fab, Geom g, int nk, int sample_every, int* __restrict__ rank,
@@ -109,7 +111,8 @@ __global__ __launch_bounds__(kB) void k_box_rank(PView P, Fab fab, Geom g, int n
     if (act && lead == lane) base = atomicAdd(&counts[k], size);
     base = __shfl(base, lead);
     if (act) rank[ip] = base + below;
-    if (blockIdx.x % sample_every == 0 && lane == 0) atomicAdd(&counts[nk + 2], groups + (int)__popcll(left));
+    if (blockIdx.x % sample_every == 0 && threadIdx.x == 64 * (blockIdx.x / sample_every % (kB / 64)))
+        atomicAdd(&counts[nk + 2], groups + (int)__popcll(left));
 }
 
 __global__ void k_fill_i32(int* p, int64_t n, int v)
@@ -797,6 +800,14 @@ size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 //   gather by records          5.2    5.3    5.7    5.8    5.9    6.4
 //   deposit through perm       4.5    5.1    6.3    7.3    7.7    14.2
 //   deposit by records         -      6.1    6.5    6.6    6.6    7.1
+// Smaller arrays lie in the caches, and there the deposit's line comes some percent early
+// (perm / records, ms, at d = 0.6, 1.0, 1.5, 3.0 and in random order):
+//   deposit 32^3 x 92, NF = 3   .72/.87 .84/.91 .87/.91 1.27/.95 1.99/1.04
+//           32^3 x 92, NF = 2   .36/.46 .48/.53 .49/.53 .72/.59 1.35/.67
+//           40^3 x 24, NF = 2   .47/.52 .49/.55 .48/.55 .54/.58 .74/.59
+//   gather  32^3 x 92, NF = 3   .98/.74 1.59/.80 1.78/.80 2.85/.88 5.47/.96
+//           32^3 x 92, NF = 2   .62/.47 1.02/.54 1.15/.54 1.90/.60 3.22/.68
+//           40^3 x 24, NF = 2   .41/.31 .60/.34 .54/.33 1.03/.37 1.19/.39
 constexpr int kScatteredDeposit = 24, kScatteredGather = 7;
 
 } // namespace
@@ -844,7 +855,7 @@ int box_list_and_run(emu_ctx* ctx, const PView& P, const PView* dst, const Fab& 
     // blocks sampled for the order of the arrays: at most 256 of them
     const unsigned nb = nblk(P.np);
     const int every = (int)((nb + 255) / 256);
-    const int waves = (int)((nb + every - 1) / every) * (kB / 64);
+    const int waves = (int)((nb + every - 1) / every);
     const int rec_min = call == BoxCall::deposit_static ? -1 : (deposit ? kScatteredDeposit : kScatteredGather) * waves;
     hipLaunchKernelGGL(k_fill_i32, dim3(nblk(nk + 3)), dim3(kB), 0, s, b.counts, (int64_t)nk + 3, 0);
     hipLaunchKernelGGL(k_box_rank, dim3(nb), dim3(kB), 0, s, P, fab, ctx->g, nk, every, b.rank, b.counts);
