@@ -229,11 +229,14 @@ class AdjointProblem:
 
     def objective(self, pos, Nn, Y, grad=True):
         J = ctypes.c_double()
-        dJ = torch.empty_like(Y) if grad else None
+        # without the gradient the call still gets room for one, where its cell
+        # list lies while it sums: the step work past the objective's own part
+        # (0.51 ms at 32^3 x 92, 0.8 cells from cell order, the dropped gradient
+        # included; 8.1 ms with no room)
+        dJ = torch.empty_like(Y) if grad else self.step_work[2 * math.prod(self.emu.parms.ncell) + 1:]
         check(self._fn("emu_adj_objective")(self.emu.ctx, self.np, _p(pos), _p(Nn), _p(Y), ctypes.byref(J),
-                                            _p(dJ) if grad else None, _p(self.step_work)), "emu_adj_objective",
-              self.emu.ctx)
-        return J.value, dJ
+                                            _p(dJ), _p(self.step_work)), "emu_adj_objective", self.emu.ctx)
+        return J.value, dJ if grad else None
 
     def advance_positions(self, pos):
         self._fp64_only("advance_positions")
