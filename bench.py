@@ -89,7 +89,6 @@ def run_precision(core, parms, parts, precision, steps, warmup):
     t_wall = time.perf_counter() - t_wall0
     ms = ev0.elapsed_time(ev1)
     stage_ms, n_stage = st.kernel_ms(0)
-    fill_ms, _ = st.kernel_ms(1)
     sort_ms, _ = st.kernel_ms(2)
     dt_ms, _ = st.kernel_ms(3)
     st.profile(False)
@@ -99,7 +98,7 @@ def run_precision(core, parms, parts, precision, steps, warmup):
     st.close()
     return {"ms_total": ms, "wall_s": t_wall, "ms_per_step": ms / steps, "updates_per_s": parts.np * steps / (ms * 1e-3),
             "growth_rate": rate, "time_window": [info0["time"], info1["time"]], "amp": [a0[0], a1[0]],
-            "stage_ms": stage_ms, "stage_launches_per_step": n_stage / steps, "fill_ms": fill_ms, "sort_ms": sort_ms,
+            "stage_ms": stage_ms, "stage_launches_per_step": n_stage / steps, "sort_ms": sort_ms,
             "dt_ms": dt_ms}
 
 
@@ -323,8 +322,7 @@ def time_per_function(core, emu, parts, steps, warmup):
 
 def run_plain(args):
     """The per-function drop-in path (core.Integrator: deposit_to_mesh,
-    FillBoundary, copyParticles, interpolate_rhs_from_mesh and the RK4
-    Copy/Saxpy calls, then SyncLocation / RedistributeLocal / Renormalize /
+    FillBoundary, rhs_from_mesh and the RK4 Copy/Saxpy calls, then SyncLocation / RedistributeLocal / Renormalize /
     compute_dt) at the workload, FP64: particle-updates/s over the timed
     steps and the fraction of HBM peak the algorithmic bytes give."""
     import torch
@@ -480,9 +478,9 @@ def main():
         out["fp32_vs_per_function_fp64"] = {
             "ms_per_step_per_function": ms_pf, "steps": pf_steps,
             "speedup": ms_pf / res["fp32"]["ms_per_step"],
-            "path": "core.Integrator: deposit_to_mesh, FillBoundary, copyParticles, interpolate_rhs_from_mesh and "
-                    "the RK4 Copy/Saxpy calls of main.cpp, FP64"}
-    out["kernels_ms"] = {p: {k: res[p][k] for k in ("stage_ms", "fill_ms", "sort_ms", "dt_ms")} for p in res}
+            "path": "core.Integrator: deposit_to_mesh, FillBoundary, rhs_from_mesh (copyParticles and "
+                    "interpolate_rhs_from_mesh in one) and the RK4 Copy/Saxpy calls of main.cpp, FP64"}
+    out["kernels_ms"] = {p: {k: res[p][k] for k in ("stage_ms", "sort_ms", "dt_ms")} for p in res}
     # the same algorithmic bytes over the whole step's wall time (every launch)
     out["roofline"]["wall_frac"] = parts.np * bpu / (r["ms_per_step"] * 1e-3) / 1e9 / HBM_PEAK_GBS
     if "fp32" in res and "fp64" in res and not args.no_precision_check:

@@ -856,7 +856,7 @@ template <int NF, typename T> constexpr int step_waves(int boxes, bool dep)
 //  deferred into err) and advances the particle's position.  The accumulators
 //  after stages 1 and 2 are not stored: with Y2 = y + dt/2 k1 and Y3 = y + dt/2 k2
 //  the second is Y3 + (Y2 - Y3)/3, which stage 3 forms from y2 = Y2 and in.Y = Y3
-//  (24 NF^2 fewer values moved per particle and step; the change is at
+//  (6 NF^2 fewer values moved per particle and step; the change is at
 //  rounding level, as in the fused step).
 //  STORE 1 (the VJP's recompute): S = 1..3 write Y_{S+1} into ynext only.
 //  S = 1..3 also deposit Y_{S+1} onto gnext (its base already there), the wave's

@@ -2,8 +2,9 @@
 // RK update of every particle of a cell, and the deposit of the next stage
 // state as one small matrix product per cell on the FP64 matrix cores.
 //
-// One wave owns one cell (FP32-bulk's RK stages: two x-adjacent cells) and
-// takes its particles 64 at a time (lane = particle).
+// A wave owns one cell, or two x-adjacent ones on larger grids, or a quarter of the
+// chunks of a cell where cells are few and full (MODE), and takes its particles 64
+// at a time (lane = particle).
 //
 // Gather (MFMA): with s(p) = (1, -vx, -vy, -vz) and G_g(t, c) the four field
 // groups (M, Phix, Phiy, Phiz) of neighbour t,
@@ -443,7 +444,7 @@ template <typename T> struct StageArgs {
     double m00;         // the base: the matter term on component 0, zero elsewhere
     int want_dt;        // stage 4: the conservative flavour bound of the grid it gathers, into red
     unsigned long long* red; // compute_dt's maxima (DtRed)
-    int step_end;       // stage 0: also finish the step (StepEnd)
+    int step_end;       // stage 0: also finish the step (time, steps and the next dt)
     DtParams dtp;
     double* scal;       // [0] time [1] dt
     int64_t* steps;

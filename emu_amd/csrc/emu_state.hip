@@ -590,11 +590,10 @@ int ensure_cub(emu_state* st, size_t need)
     return EMU_OK;
 }
 
-// out = exclusive scan of in (ncell + 1 entries, in[ncell] = 0), on stream s
-// (the context's when null)
-int scan_counts(emu_state* st, const int* in, int* out, hipStream_t s = nullptr)
+// out = exclusive scan of in (ncell + 1 entries, in[ncell] = 0)
+int scan_counts(emu_state* st, const int* in, int* out)
 {
-    if (!s) s = st->ctx->stream;
+    hipStream_t s = st->ctx->stream;
     size_t need = 0;
     (void)hipcub::DeviceScan::ExclusiveSum(nullptr, need, in, out, (int)(st->ncell + 1), s);
     if (ensure_cub(st, need)) return set_error(st->ctx, EMU_ERR_NOMEM, "scan scratch");
