@@ -433,12 +433,15 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Whether neighbour t (of 27) is part of the stencil: in a dimension of shape order 0
-// only the centre is.  The others have weight 0, which a field that is not finite
-// would turn into NaN: they are left out of the products and of the deposits.
-__device__ __forceinline__ bool in_stencil(const Geom& g, int t)
+// Bit t: neighbour t (of 27) is part of the stencil.  In a dimension of shape order 0
+// only the centre is: the others have weight 0, which a field that is not finite
+// would turn into NaN, so they are left out of the products and of the deposits.
+constexpr unsigned kFullStencil = 0x7ffffffu;
+__device__ __forceinline__ unsigned stencil_mask(const Geom& g)
 {
-    return (g.order[0] > 0 || t % 3 == 1) && (g.order[1] > 0 || (t / 3) % 3 == 1) && (g.order[2] > 0 || t / 9 == 1);
+    const unsigned x = g.order[0] > 0 ? 7u : 2u;
+    const unsigned xy = g.order[1] > 0 ? x | x << 3 | x << 6 : x << 3;
+    return g.order[2] > 0 ? xy | xy << 9 | xy << 18 : xy << 9;
 }
 
 // A wave's copy of its cell's neighbourhood in LDS: 27 rows of 4 NH fields in T
@@ -452,7 +455,7 @@ template <int NF, typename T> struct CellBox {
     static constexpr int QG = 4 * NH<NF>, N = 28 * QG;
     using Gather = WaveGather<NF, T, 3, 3, 3, false, QG>;
 
-    // index of the neighbours' cells (-1: not in the stencil), for lanes 0..26 of the wave
+    // index of the neighbours' cells, for lanes 0..26 of the wave
     static __device__ __forceinline__ void table(const Geom& g, int cell, int lane, int* ctab)
     {
         if (lane < 27) {
@@ -460,23 +463,23 @@ template <int NF, typename T> struct CellBox {
             const int x = wrap(cell % g.n[0] + lane % 3 - 1, g.n[0]);
             const int y = wrap((cell / g.n[0]) % g.n[1] + (lane / 3) % 3 - 1, g.n[1]);
             const int z = wrap(cell / (g.n[0] * g.n[1]) + lane / 9 - 1, g.n[2]);
-            ctab[lane] = in_stencil(g, lane) ? (z * g.n[1] + y) * g.n[0] + x : -1;
+            ctab[lane] = (z * g.n[1] + y) * g.n[0] + x;
         }
     }
     // (after table and a wave_sync; followed by a wave_sync)
-    static __device__ __forceinline__ void stage(const double* grid, const int* ctab, int lane, T* box)
+    static __device__ __forceinline__ void stage(const double* grid, const Geom& g, const int* ctab, int lane, T* box)
     {
 #pragma unroll
         for (int e0 = 0; e0 < N; e0 += 64) {
             const int e = e0 + lane;
-            if (e < 27 * QG) {
-                const int c = ctab[e / QG];
-                const double v = grid[(int64_t)max(c, 0) * QG + e % QG];
-                box[e] = c < 0 ? T(0) : T(v);
-            } else if (e < N) {
-                box[e] = T(0);
-            }
+            if (e < 27 * QG) box[e] = T(grid[(int64_t)ctab[e / QG] * QG + e % QG]);
+            else if (e < N) box[e] = T(0);
         }
+        const unsigned mask = stencil_mask(g);
+        if (mask == kFullStencil) return;
+        wave_sync();
+        for (int e = lane; e < 27 * QG; e += 64)
+            if (!(mask >> (e / QG) & 1u)) box[e] = T(0);
     }
 };
 
@@ -706,7 +709,7 @@ __global__ __launch_bounds__(64 * kCellWaves) void k_obj_deposit(AdjInT<T> in, G
         }
     wave_sync();
     const int t = lane >> 1;
-    if (t < 27 && ctab[t] >= 0) unsafeAtomicAdd(&g2[2 * (int64_t)ctab[t] + (lane & 1)], v[0]);
+    if (stencil_mask(g) >> t & 1u) unsafeAtomicAdd(&g2[2 * (int64_t)ctab[t] + (lane & 1)], v[0]);
 }
 
 // A wave's deposit of its cell's particles on the f64 matrix cores, a chunk
@@ -816,13 +819,14 @@ template <int NF> struct WaveDeposit {
             const int tz = wrap(kz + t / 9 - 1, g.n[2]);
             return grid + (((int64_t)tz * g.n[1] + ty) * g.n[0] + tx) * QG;
         };
+        const unsigned mask = stencil_mask(g); // no bits from NT on
         // element r of lane l holds D[16m + 4r + l/16][16n + l%16]
 #pragma unroll
         for (int m = 0; m < MT; m++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int t = 16 * m + 4 * r + (lane >> 4);
-                if (t >= NT || !in_stencil(g, t)) continue;
+                if (!(mask >> t & 1u)) continue;
                 double* Gd = target(t);
 #pragma unroll
                 for (int n = 0; n < NTF; n++) unsafeAtomicAdd(&Gd[16 * n + (lane & 15)], acc[m][n][r]);
@@ -833,7 +837,7 @@ template <int NF> struct WaveDeposit {
 #pragma unroll
             for (int k = 0; k < NSM; k++) {
                 const int t = 16 * m + 4 * ((lane >> 2) & 3) + (lane >> 4), q = 16 * NTF + 4 * k + (lane & 3);
-                if (t >= NT || q >= QG || !in_stencil(g, t)) continue;
+                if (!(mask >> t & 1u) || q >= QG) continue;
                 unsafeAtomicAdd(&target(t)[q], accs[m][k]);
             }
     }
@@ -894,7 +898,7 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
     const int lane = threadIdx.x & 63;
     Box::table(g, cell, lane, tables + 28 * wave);
     wave_sync();
-    Box::stage(grid, tables + 28 * wave, lane, box);
+    Box::stage(grid, g, tables + 28 * wave, lane, box);
     wave_sync();
     typename Box::Gather gather;
     gather.init(lane);
@@ -1010,7 +1014,7 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(1, S < 4))) void k_fwd_stag
 // moves at 3.0 M particles, 2 flavours, FP64: 235 us of the 501 us it takes; two
 // gathers' and a deposit's matrix instructions do not overlap with the rest at the
 // two waves per SIMD that its registers allow.  Every
-// stencil width runs the 3 x 3 x 3 target set (in_stencil: an order-0 dimension's
+// stencil width runs the 3 x 3 x 3 target set (stencil_mask: an order-0 dimension's
 // other targets take no part).
 template <int NF, typename T, bool G, bool C>
 __global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void k_vjp_fused(
@@ -1036,8 +1040,8 @@ __global__ __launch_bounds__((64 * step_waves<NF, T>(int(G) + int(C), C))) void 
     if (beg == end) return;
     Box::table(g, cell, lane, tables + 28 * wave);
     wave_sync();
-    if constexpr (C) Box::stage(grid, tables + 28 * wave, lane, boxC);
-    if constexpr (G) Box::stage(gadj_in, tables + 28 * wave, lane, boxG);
+    if constexpr (C) Box::stage(grid, g, tables + 28 * wave, lane, boxC);
+    if constexpr (G) Box::stage(gadj_in, g, tables + 28 * wave, lane, boxG);
     wave_sync();
     typename Box::Gather gather;
     gather.init(lane);
