@@ -91,7 +91,10 @@ typedef struct emu_state emu_state;
  * main.cpp:37-85 and Evolve.H_M2_fill, generate_code.py:176-227). */
 int emu_create(const emu_params* params, emu_ctx** out);
 int emu_destroy(emu_ctx* ctx);
-int emu_set_stream(emu_ctx* ctx, void* hip_stream); /* NULL = default stream */
+/* NULL = default stream.  The new stream is not ordered after the old one: where
+ * per-function deposits or gathers (whose scratch is the context's) may still run
+ * there, wait for them or order the streams first. */
+int emu_set_stream(emu_ctx* ctx, void* hip_stream);
 int emu_sync(emu_ctx* ctx);                         /* hipStreamSynchronize */
 const char* emu_last_error(const emu_ctx* ctx);
 /* Ghost width per dim of the reference's MultiFab: 1 + (1+order)/2, order 0
